@@ -515,6 +515,46 @@ def test_bsa_key_split_long_rows_match_oracle(d, split, logits):
     assert torch.count_nonzero(got[0, bs:2 * bs, 0]) == 0
 
 
+@pytest.mark.parametrize("case", ["ids", "duplicate", "clamped", "many_blocks", "dense"])
+@pytest.mark.parametrize("b,h,nq", [(1, 1, 3), (2, 3, 5)])
+def test_bsa_long_rows_rank_ranges_match_oracle(case, b, h, nq):
+    """Rows of more than 64 visits over 64-key blocks: each unit takes a rank range of the row's
+    blocks in block order (ids), or its list slice where an id occurs twice (also after clamping) or
+    there are more blocks than the bitmap holds; fewer rows than XCDs and rows that split a head
+    between XCDs; a unit table must give the same bits as the grid without one."""
+    from worldattention_amd.hsa.block_sparse import bsa_forward
+    torch.manual_seed(b * 10 + nq)
+    bs, d = 64, 64
+    nkv = 2050 if case == "many_blocks" else 133
+    lq, lkv = nq * bs - 9, nkv * bs - 31
+    q, k, v = (torch.randn(b, n, h, d).bfloat16() for n in (lq, lkv, lkv))
+    index = torch.stack([torch.randperm(nkv) for _ in range(b * h * nq)]).view(b, h, nq, nkv).int()
+    num = torch.randint(65, 134, (b, h, nq), dtype=torch.int32)
+    if case == "duplicate":
+        index[..., 5] = index[..., 60]
+    elif case == "clamped":
+        index[index == 7] = nkv + 40        # clamped onto the last block, which most rows list too
+    if case == "dense":
+        num[:] = nkv
+    qd, kd, vd = q.to(DEV), k.to(DEV), v.to(DEV)
+    args = dict(index=None if case == "dense" else index.to(DEV), num=None if case == "dense" else num.to(DEV),
+                block_size=bs, layout="blhd", lq=lq, lkv=lkv, out_dtype=torch.float32)
+    got, _ = bsa_forward(qd, kd, vd, split=48, **args)
+    qp = O.pad_to_len(q, nq * bs).transpose(1, 2)
+    kp, vp = (O.pad_to_len(t, nkv * bs).transpose(1, 2) for t in (k, v))
+    if case == "dense":
+        index = torch.arange(nkv, dtype=torch.int32).expand(b, h, nq, nkv)
+    sizes = O.variable_block_sizes(lkv, nkv * bs, bs)
+    want = O.block_sparse_attention(qp.float(), kp.float(), vp.float(), index, num, sizes, bs).transpose(1, 2)[:, :lq]
+    assert_close(got, want, what=f"long rows {case}")
+    if case == "ids":                       # one visit count per head: the same launch from a unit table
+        num = num.amin(dim=(0, 2), keepdim=True).expand(b, h, nq).contiguous()
+        args["num"] = num.to(DEV)
+        plain, _ = bsa_forward(qd, kd, vd, split=48, **args)
+        table, _ = bsa_forward(qd, kd, vd, split=48, visits=num[0, :, 0].tolist(), **args)
+        assert torch.equal(plain, table)
+
+
 def test_hsa_forward_graph_replays_equal_eager_calls():
     """The cfg 2 call captured in a HIP graph (as bench.py times it): every replay, with eager work
     and synchronizations between replays, equals the eager call bit for bit."""

@@ -56,7 +56,7 @@ struct FwdParams {
   const bf16_t* gate_w; const float* gate_b;
   int gate_pre_bf16, gate_out_bf16, attn_round_bf16;
   // split bookkeeping
-  const int32_t* units;  // [n_units][2] = (row, split) or NULL: unit u = (u / max_splits, u % max_splits)
+  const int32_t* units;  // [n_units][2] = (row, split) or NULL: every split of every row (unit_of)
   int n_units, max_splits, split;
   int64_t n_rows;
   int k_slab_bytes, v_slab_bytes;  // bytes of one (batch, head) K / V slab: rows 0 .. Lkv-1
@@ -71,6 +71,29 @@ __device__ __forceinline__ int row_visits(const FwdParams& p, int64_t irow) {
   if (!p.index) return p.Nkv;
   const int n = p.num[irow];
   return max(0, min(n, (int)p.index_width));
+}
+
+// Unit of workgroup `id` without a unit table. XCD id % 8 owns a contiguous eighth of the rows and
+// walks it head by head, split-major inside a head: all its rows' split 0, then split 1, ... A unit
+// of a long row holds one rank range of the row's listed blocks (see bsa_unit_kernel), so the ~64
+// units an XCD runs at a time read the same stretch of a head's keys and share it in the 4 MB L2.
+__device__ __forceinline__ bool unit_of(const FwdParams& p, int id, int64_t& row, int& split) {
+  const int ms = p.max_splits, nq = p.Nq, rows = (int)p.n_rows, xcd = id % 8;
+  int local = id / 8;
+  const int r0 = (int)((int64_t)rows * xcd / 8), r1 = (int)((int64_t)rows * (xcd + 1) / 8);
+  if (local / ms >= r1 - r0) return false;
+  const int first = min(r1, (r0 / nq + 1) * nq) - r0;  // rows of the XCD's first (perhaps partial) head
+  int base = r0, seg = first;
+  if (local / ms >= first) {
+    local -= first * ms;
+    const int k = local / ms / nq;
+    base = r0 + first + k * nq;
+    seg = min(nq, r1 - base);
+    local -= k * nq * ms;
+  }
+  split = local / seg;
+  row = base + local % seg;
+  return true;
 }
 
 // Ascending bitonic sort of one int per lane across the 64-lane wave.
@@ -424,23 +447,23 @@ bsa_unit_kernel(FwdParams p) {
   __shared__ __attribute__((aligned(1024))) bf16_t vs0[TILE];
   __shared__ __attribute__((aligned(1024))) bf16_t vs1[TILE];
   __shared__ int steptab[NWT][64][2];
+  __shared__ uint32_t s_bits[64];  // listed block ids of a long row
 
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, l32 = lane & 31;
   const int qw = w % NW, kh = w / NW;  // query wave; key half (KS = 2)
 
-  const int u = wa_xcd_remap(blockIdx.x, p.n_units);
   // The prologue's memory reads in two round trips: the unit entry with the head map beside it,
   // then (once the row is known) its visit count, its list window and Q together.
   const int hmap = p.heads && lane < min(p.n_heads, 64) ? p.heads[lane] : 0;
   int64_t row;
   int split;
   if (p.units) {
+    const int u = wa_xcd_remap(blockIdx.x, p.n_units);
     row = p.units[2 * u];
     split = p.units[2 * u + 1];
   } else {
-    row = u / p.max_splits;
-    split = u % p.max_splits;
+    if (!unit_of(p, (int)blockIdx.x, row, split)) return;
   }
   if (row < 0 || row >= p.n_rows || split < 0 || split >= p.max_splits) return;
   const int qb = (int)(row % p.Nq);
@@ -451,15 +474,19 @@ bsa_unit_kernel(FwdParams p) {
   if (h < 0 || h >= p.H) return;  // uniform per workgroup
   const int64_t irow = ((int64_t)b * p.H + h) * p.Nq + qb;
 
-  // The row's list entries at positions lane (j0) and split * p.split + lane (j1), read before its
-  // visit count is known (in bounds of the row's index_width entries); the count then picks one.
+  // The row's first list entries, read before its visit count is known (in bounds of the row's
+  // index_width entries): position lane (j0: a row of at most 64 visits) and positions tid and
+  // tid + NTH (e0, e1: a longer row's block-id bitmap).
+  constexpr int NTH = 64 * NWT;
   const int nraw = p.index ? p.num[irow] : p.Nkv;
-  int j0 = 0, j1 = 0;
+  const int32_t* lrow = p.index ? p.index + irow * p.index_width : nullptr;
+  int j0 = 0, e0 = 0, e1 = 0;
   if (p.index) {
-    const int32_t* lrow = p.index + irow * p.index_width;
     if (lane < min((int)p.index_width, 64)) j0 = lrow[lane];
-    const int lo1 = split * p.split;
-    if (split > 0 && lane < min((int)p.index_width - lo1, 64)) j1 = lrow[lo1 + lane];
+    if (p.index_width > 64) {
+      if (tid < p.index_width) e0 = lrow[tid];
+      if (tid + NTH < p.index_width) e1 = lrow[tid + NTH];
+    }
   }
   // Q^T fragments (B operand): lane holds Q[qi, 16c + 8g .. +8) of each of its tiles.
   int qi[QT];
@@ -488,18 +515,65 @@ bsa_unit_kernel(FwdParams p) {
   const bf16_t* kbase = p.k + (int64_t)b * p.k_sb + (int64_t)h * p.k_sh;
   const bf16_t* vbase = p.v + (int64_t)b * p.v_sb + (int64_t)h * p.v_sh;
 
-  // List entries one per lane, read once. A row of at most 64 visits is loaded whole and sorted by
-  // block id, and split s of the row's ns units takes the sorted positions s, s + ns, s + 2 ns, ...:
-  // every unit of a head (they run together on one XCD) then sweeps the whole key range in step
-  // with the others, so the units that list a block fetch it at about the same time and share it in
-  // L2. The visit order only changes the summation order. A longer row gives each unit one
-  // contiguous slice of its list, sorted by block id the same way (a dense row is in order).
+  // List entries one per lane. A row of at most 64 visits is sorted by block id, and split s of the
+  // row's ns units takes the sorted positions s, s + ns, s + 2 ns, ...: every unit of a head (they
+  // run together on one XCD) then sweeps the whole key range in step with the others, so the units
+  // that list a block fetch it at about the same time and share it in L2. The visit order only
+  // changes the summation order. In a longer row unit s takes the listed blocks of rank
+  // [n s / ns, n (s + 1) / ns) in block-id order, found through a bitmap of the listed ids: the
+  // split-s units of a head's rows (neighbours in launch order) then visit the same ~1 / ns of the
+  // key range. Before, each unit had a slice of the list in weight order, spread over all keys:
+  // at B 1, H 12, D 128,
+  // Lq 4680, Lkv 32760, ~180 of 512 blocks a row, the launch took 617 us with slices, 452 us with
+  // rank ranges of at most 48 blocks and 429 us with 64.
+  // Ids listed twice (or more blocks than 2,048, or a list cut off by max_visits) keep the slices.
   const bool whole = n <= 64;
-  const int lo = whole ? 0 : s_begin;
-  const int take = whole ? n : s_end - s_begin;
+  int lo = whole ? 0 : s_begin;
+  int take = whole ? n : s_end - s_begin;
   int my_j = 0;
-  if (lane < take) my_j = p.index ? min(max(lo == 0 ? j0 : j1, 0), p.Nkv - 1) : lo + lane;
-  if (whole || p.index) my_j = wave_sort_ascending(lane < take ? my_j : 0x7fffffff, lane);
+  bool ranked = !p.index && !whole && (int64_t)ns * p.split >= n;  // a dense row lists block i at position i
+  if (ranked) {
+    lo = (int)((int64_t)n * split / ns);
+    take = (int)((int64_t)n * (split + 1) / ns) - lo;
+  }
+  if (p.index && !whole && p.Nkv <= 2048 && (int64_t)ns * p.split >= n) {  // uniform over the workgroup
+    if (tid < 64) s_bits[tid] = 0;
+    __syncthreads();
+    for (int i = tid; i < n; i += NTH) {
+      const int e = i < NTH ? e0 : i < 2 * NTH ? e1 : lrow[i];
+      const int id = min(max(e, 0), p.Nkv - 1);
+      atomicOr(&s_bits[id >> 5], 1u << (id & 31));
+    }
+    __syncthreads();
+    uint32_t word = s_bits[lane];
+    const int cnt = __popc(word);
+    int incl = cnt;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int up = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += up;
+    }
+    if (__builtin_amdgcn_readlane(incl, 63) == n) {
+      ranked = true;
+      lo = (int)((int64_t)n * split / ns);
+      take = (int)((int64_t)n * (split + 1) / ns) - lo;
+      int r = incl - cnt - lo;  // this lane's first block's position in the unit
+      if (r < take && r + cnt > 0) {
+        while (word) {
+          if (r >= 0 && r < take) steptab[w][r][0] = lane * 32 + __ffs(word) - 1;
+          word &= word - 1;
+          ++r;
+        }
+      }
+      if (lane < take) my_j = steptab[w][lane][0];
+    }
+  }
+  if (!ranked) {
+    if (lane < take) my_j = p.index ? min(max(lo == 0 ? j0 : lrow[lo + lane], 0), p.Nkv - 1) : lo + lane;
+    if (whole || p.index) my_j = wave_sort_ascending(lane < take ? my_j : 0x7fffffff, lane);
+  } else if (!p.index && lane < take) {
+    my_j = lo + lane;
+  }
   const bool mine = whole ? lane < n && lane % ns == split : lane < take;
   const int my_real = mine ? block_real(p, my_j, BS) : 0;
 
@@ -1043,8 +1117,7 @@ int64_t partial_bytes(int64_t rows, int64_t max_splits, int64_t block_size, int6
 }
 
 // Default visits per unit: 16 for 128-key blocks (cfg 2: 8-32 listed blocks per row); 48 for
-// 64-key blocks, whose Gini rows list ~180 blocks at the Wan shape (four units per row: the whole
-// call 0.735 ms in graph replay against 0.755 at 64 visits, 0.755 at 40 and 0.85 at 32).
+// 64-key blocks (callers with many rows pass 64: see bsa_forward in block_sparse.py).
 int64_t default_split(int64_t block_size) {
   return block_size == 64 ? WA_BSA_DEFAULT_SPLIT_64 : WA_BSA_DEFAULT_SPLIT;
 }
@@ -1170,7 +1243,7 @@ int bsa_fwd_impl(const wa_bsa_fwd_args* a, void* workspace, void* stream) {
   const int64_t max_visits = a->max_visits > 0 ? (a->max_visits < width ? a->max_visits : width) : width;
   const int64_t max_splits = max_visits > 0 ? (max_visits + split - 1) / split : 1;
   const int64_t n_units = a->units ? a->n_units : rows * max_splits;
-  WA_CHECK_ARG(rows < (int64_t)1 << 31 && n_units < (int64_t)1 << 31 && rows * max_splits < (int64_t)1 << 40 &&
+  WA_CHECK_ARG(rows < (int64_t)1 << 31 && n_units + (a->units ? 0 : 8 * max_splits) < (int64_t)1 << 31 && rows * max_splits < (int64_t)1 << 40 &&
                    a->Lq < (int64_t)1 << 30 && a->Lkv < (int64_t)1 << 30,
                "wa_bsa_fwd: problem too large");
   WA_CHECK_ARG(a->units == nullptr || a->n_units >= 0, "wa_bsa_fwd: bad unit count");
@@ -1219,6 +1292,7 @@ int bsa_fwd_impl(const wa_bsa_fwd_args* a, void* workspace, void* stream) {
                        dim3((unsigned)rows), dim3(2 * a->block_size), 0, s, fp);
     return wa_launch_status("bsa_fwd_empty_rows");
   }
+  if (!fp.units) fp.n_units = (int)((rows + 7) / 8 * 8 * max_splits);  // unit_of's grid: an eighth of the rows per XCD
   // steps per unit: one per visit of a 64-key block
   const bool key_split = a->block_size == 64 && (split < max_visits ? split : max_visits) >= 32;
   if (a->D == 64 && a->block_size == 64) return launch<64, 64>(fp, rows, cleared, key_split, s);
