@@ -418,6 +418,10 @@ typedef struct wa_compress_args {
 } wa_compress_args;
 int wa_compress_kv(const wa_compress_args* args, void* stream);
 
+/* n (1..64) compressions in order; neighbouring jobs of one shape (the keys and values of a call)
+ * share a launch. Every job is checked before the first launch. */
+int wa_compress_kv_n(const wa_compress_args* args, int32_t n, void* stream);
+
 /* Backward of wa_compress_kv. dout: gradient of the compressed rows (fp32, BLHD strides, the Lc
  * rows wa_compress_kv wrote); x, proj and the sizes as in the forward, with E = proj's stored
  * values (fp32, or bf16 widened). Per segment (rows row0 .. row0 + r of dout, tokens start ..):

@@ -191,6 +191,45 @@ def test_compress_kv_matches_oracle(dtype):
     assert_close(gv, wv, max_abs=1e-2, mean_abs=1e-3, what="compress v")
 
 
+@pytest.mark.parametrize("d,length,seg,bs,rank,plen,xdt,pdt,shift", [
+    (128, 1111, 500, 64, 8, 500, torch.float32, torch.bfloat16, 0),     # three segments, the last short
+    (128, 700, 700, 8, 88, 701, torch.float32, torch.float32, 1),        # rank over 32, odd E rows, misaligned x
+    (64, 97, 64, 64, 5, 64, torch.bfloat16, torch.float32, 0),           # bf16 x beside an fp32 projection
+    (64, 130, 130, 4, 33, 136, torch.bfloat16, torch.bfloat16, 4),       # one rank row in a second tile
+    (32, 31, 31, 1, 31, 40, torch.float32, torch.bfloat16, 0),           # less than one 32-token chunk
+    (128, 3000, 1560, 64, 25, 1560, torch.bfloat16, torch.bfloat16, 0),  # the streaming kernel
+])
+def test_compress_kernels_match_fp64_of_their_operands(d, length, seg, bs, rank, plen, xdt, pdt, shift):
+    """compress_kv rounds both operands to bf16 and sums in fp32: against the fp64 product of the
+    rounded operands, an output may differ by n 2^-24 sum |E||x| (any fp32 summation order over n
+    tokens), and by half an ulp (2^-9 relative) where it is stored in bf16. Keys and values in one
+    launch equal single launches bit for bit."""
+    torch.manual_seed(length)
+    b, h = 2, 3
+    store = torch.randn(2, b, length, h, d + shift).to(xdt)
+    pk, pv = (torch.rand(rank, plen).sub(0.3).div(16).to(pdt) for _ in range(2))
+    k, v = (t[..., shift:] for t in store.to(DEV))
+    jobs = [(k, pk.to(DEV), None), (v, pv.to(DEV), None)]
+    kw = dict(segment_len=seg, block_size=bs, layout="blhd")
+    pair = WA._compress_many(jobs, **kw)
+    for got, (x, p, _) in zip(pair, jobs):
+        assert torch.equal(got, WA._compress(x, p, **kw))
+    for got, x, p in zip(pair, store[..., shift:], (pk, pv)):
+        xe, pe = x.bfloat16().double().permute(0, 2, 1, 3), p.bfloat16().double()
+        want, bound = [], []
+        for s in range(0, length, seg):
+            xs = xe[:, :, s:s + seg]
+            n = xs.shape[2]
+            r = min(rank, -(-n // bs))
+            want.append(pe[:r, :n] @ xs)
+            bound.append(n * 2.0 ** -24 * (pe[:r, :n].abs() @ xs.abs()))
+        want, bound = (torch.cat(t, dim=2).permute(0, 2, 1, 3) for t in (want, bound))
+        if xdt == torch.bfloat16:
+            bound = bound + 2.0 ** -8 * want.abs()
+        assert got.shape == want.shape
+        assert ((got.cpu().double() - want).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("d", [64, 128])
 def test_dense_distillation_teacher_matches_oracle(d):
     """The distillation teacher (the dense flash kernel) against fp32 softmax attention (the

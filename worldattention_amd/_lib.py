@@ -324,6 +324,7 @@ SIGNATURES = {
     "wa_bsa_fwd": (c_int, [POINTER(BsaFwdArgs), c_void_p]),
     "wa_bsa_fwd_noalloc": (c_int, [POINTER(BsaFwdArgs), c_void_p]),
     "wa_compress_kv": (c_int, [POINTER(CompressArgs), c_void_p]),
+    "wa_compress_kv_n": (c_int, [POINTER(CompressArgs), c_int32, c_void_p]),
     "wa_compress_kv_bwd_workspace_bytes": (c_int64, [c_int64] * 4),
     "wa_compress_kv_bwd": (c_int, [POINTER(CompressBwdArgs), c_void_p]),
     "wa_elu1_state_workspace_bytes": (c_int64, [c_int64, c_int64, c_int64, c_int64]),

@@ -13,104 +13,123 @@
 
 namespace {
 
-template <typename T>
-__device__ __forceinline__ void load8(const T* src, float (&f)[8], bool ok) {
-#pragma unroll
-  for (int e = 0; e < 8; ++e) f[e] = ok ? (float)src[e] : 0.f;
-}
-
-// =============================================================================================
-// compress_kv: out[row0 + r, d] = sum_t E[r, t] x[start + t, d], one workgroup per
-// (segment, head, batch). Tokens are processed 64 at a time: x^T chunk in LDS, E fragments read
-// from global (tiny, cache resident). Wave w owns output column tiles w, w+4, ...
-// =============================================================================================
 struct CompressParams {
   const void* x; int64_t x_sb, x_st, x_sh; int x_dtype;
   const void* proj; int proj_dtype; int proj_rank, proj_len;
   int L, H, D, seg, block;
   void* out; int64_t o_sb, o_st, o_sh; int o_dtype;
   int64_t x_slab;   // bytes of one (batch, head) x slab: first row to the last row's end
+  int proj_vec;     // rows of E 16-byte aligned, a multiple of 8 elements long
 };
 
-template <int D>
-__global__ void __launch_bounds__(256) compress_kernel(CompressParams p) {
-  constexpr int TC = 64;              // tokens per LDS chunk
-  constexpr int XLD = TC + 8;
+// One launch takes up to two jobs of one grid (a call's keys and values): grid.z = jobs x batch.
+struct CompressJobs {
+  CompressParams j[2];
+  int batch;
+};
+
+// =============================================================================================
+// compress_kv: out[row0 + r, d] = sum_t E[r, t] x[start + t, d], one workgroup per
+// (segment, head, batch, job), as out^T = x^T E^T on the matrix cores (operands rounded to bf16,
+// fp32 sums). General kernel (any x type and alignment, D 32 / 64 / 128, rank up to 128); bf16 x
+// with 16-byte aligned rows takes compress_stream_kernel instead.
+//
+// Bound by reading x once. 4 token groups x D / 32 channel tiles of waves: a wave loads its operand
+// straight from global memory (lane = channel, 8 consecutive tokens: every load instruction covers
+// two 32-channel rows) for 32 tokens at a time, chunks dealt to the groups in turn, and the groups'
+// sums meet in LDS in group order. 16 waves x 16 loads in flight cover a memory round trip; the
+// kernel before it staged x through LDS with 4 waves and one barrier pair per 64 tokens, one
+// element per load: keys and values of H 12, L 32,760, D 128 fp32 at segment 1,560,
+// rank 25 took 379 us (two launches) against 84 us here, and B 2, H 6, L 5,003 336 us against ~20.
+// =============================================================================================
+constexpr int kTokenGroups = 4;
+
+__device__ __forceinline__ bf16x8 compress_e8(const CompressParams& p, int r, int t, int seg_len) {
+  bf16x8 f;
+  const int64_t off = (int64_t)r * p.proj_len + t;
+  if (p.proj_vec && t + 8 <= seg_len) {
+    if (p.proj_dtype == WA_BF16) return *(const bf16x8*)((const bf16_t*)p.proj + off);
+    const f32x4 a = *(const f32x4*)((const float*)p.proj + off), c = *(const f32x4*)((const float*)p.proj + off + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      f[e] = (bf16_t)a[e];
+      f[e + 4] = (bf16_t)c[e];
+    }
+    return f;
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) f[e] = t + e < seg_len ? (bf16_t)wa_load_f(p.proj, off + e, p.proj_dtype) : (bf16_t)0.f;
+  return f;
+}
+
+template <typename T, int D, int MT>
+__global__ void __launch_bounds__(kTokenGroups * 2 * D) compress_direct_kernel(CompressJobs jobs) {
   constexpr int DT = D / 32;
-  __shared__ __attribute__((aligned(16))) bf16_t xt[D * XLD];
-  const int sidx = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 5, l32 = lane & 31;
+  __shared__ float red[kTokenGroups - 1][DT][16][64];
+  const CompressParams p = jobs.j[blockIdx.z / jobs.batch];
+  const int sidx = blockIdx.x, h = blockIdx.y, b = blockIdx.z % jobs.batch;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ct = w % DT, tg = w / DT, g = lane >> 5, l32 = lane & 31;
   const int start = sidx * p.seg;
   const int seg_len = min(p.seg, p.L - start);
   const int rank = min(p.proj_rank, (seg_len + p.block - 1) / p.block);
   const int row0 = sidx * min(p.proj_rank, (p.seg + p.block - 1) / p.block);
-  const int mtiles = (rank + 31) / 32;
-
-  // wave w owns output column tile w (D <= 128, so at most one tile per wave)
-  const bool wave_active = w < DT;
-  f32x16 acc[4];  // [m tile]
+  const T* xcol = (const T*)p.x + (int64_t)b * p.x_sb + (int64_t)h * p.x_sh + (int64_t)start * p.x_st + 32 * ct + l32;
+  f32x16 acc[MT];
 #pragma unroll
-  for (int m = 0; m < 4; ++m) acc[m] = f32x16{};
-
-  for (int t0 = 0; t0 < seg_len; t0 += TC) {
-    __syncthreads();
-    // stage x[start+t0 .. +TC, :] transposed: unit = 4 tokens x 8 channels
-    for (int u = tid; u < (TC / 4) * (D / 8); u += 256) {
-      const int tq = u / (D / 8), c8 = (u % (D / 8)) * 8;
-      float f[4][8];
+  for (int m = 0; m < MT; ++m) acc[m] = f32x16{};
+#pragma unroll MT == 1 ? 2 : 1
+  for (int t0 = 32 * tg; t0 < seg_len; t0 += 32 * kTokenGroups) {
+    T xv[2][8];  // tokens t0 + 16 ks + 8 g + e
+    if (t0 + 32 <= seg_len) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = t0 + tq * 4 + r;
-        const bool ok = t < seg_len;
-        const int64_t off = (int64_t)b * p.x_sb + (int64_t)(start + (ok ? t : 0)) * p.x_st + (int64_t)h * p.x_sh + c8;
-        if (p.x_dtype == WA_BF16) load8((const bf16_t*)p.x + off, f[r], ok);
-        else load8((const float*)p.x + off, f[r], ok);
+      for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) xv[ks][e] = xcol[(int64_t)(t0 + 16 * ks + 8 * g + e) * p.x_st];
       }
+    } else {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        bf16x4 v4 = {(bf16_t)f[0][e], (bf16_t)f[1][e], (bf16_t)f[2][e], (bf16_t)f[3][e]};
-        *(bf16x4*)(xt + (c8 + e) * XLD + tq * 4) = v4;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kc = 0; kc < TC / 16; ++kc) {
-      const int tb = t0 + kc * 16 + g * 8;  // tokens of this lane group's fragment
-#pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        if (m >= mtiles) break;
-        const int r = m * 32 + l32;
-        bf16x8 af;
+      for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const int t = tb + e;
-          float v = 0.f;
-          if (r < rank && t < seg_len) {
-            const int64_t off = (int64_t)r * p.proj_len + t;
-            v = p.proj_dtype == WA_BF16 ? (float)((const bf16_t*)p.proj)[off] : ((const float*)p.proj)[off];
-          }
-          af[e] = (bf16_t)v;
+          const int t = t0 + 16 * ks + 8 * g + e;
+          xv[ks][e] = xcol[(int64_t)min(t, seg_len - 1) * p.x_st];
+          if (t >= seg_len) xv[ks][e] = (T)0.f;
         }
-        if (wave_active) {
-          const bf16x8 bfr = *(const bf16x8*)(xt + (w * 32 + l32) * XLD + kc * 16 + g * 8);
-          acc[m] = wa_mfma32(af, bfr, acc[m]);
-        }
+      }
+    }
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      bf16x8 xf;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xf[e] = (bf16_t)xv[ks][e];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        if (32 * m >= rank) break;  // uniform
+        // rows of E past the rank repeat its last one (their results are not stored)
+        acc[m] = wa_mfma32(xf, compress_e8(p, min(32 * m + l32, rank - 1), t0 + 16 * ks + 8 * g, seg_len), acc[m]);
       }
     }
   }
-  // accumulator: lane holds column d = 32t + l32, rows r = 32m + 8*(i/4) + 4g + i%4
+  // lane l32 holds rank row r = 32 m + l32, channels 32 ct + 8 (i / 4) + 4 g + i % 4
 #pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    if (m >= mtiles) break;
-    if (wave_active) {
-      const int d = w * 32 + l32;
+  for (int m = 0; m < MT; ++m) {
+    if (32 * m >= rank) break;  // uniform over the workgroup
+    if (m) __syncthreads();
+    if (tg > 0) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) red[tg - 1][ct][i][lane] = acc[m][i];
+    }
+    __syncthreads();
+    const int r = 32 * m + l32;
+    if (tg == 0 && r < rank) {
+      const int64_t o0 = (int64_t)b * p.o_sb + (int64_t)(row0 + r) * p.o_st + (int64_t)h * p.o_sh + 32 * ct + 4 * g;
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        const int r = m * 32 + 8 * (i >> 2) + 4 * g + (i & 3);
-        if (r < rank) {
-          const int64_t off = (int64_t)b * p.o_sb + (int64_t)(row0 + r) * p.o_st + (int64_t)h * p.o_sh + d;
-          wa_store_f(p.out, off, acc[m][i], p.o_dtype);
-        }
+        float v = acc[m][i];
+#pragma unroll
+        for (int q = 0; q < kTokenGroups - 1; ++q) v += red[q][ct][i][lane];
+        wa_store_f(p.out, o0 + 8 * (i >> 2) + (i & 3), v, p.o_dtype);
       }
     }
   }
@@ -124,11 +143,13 @@ __global__ void __launch_bounds__(256) compress_kernel(CompressParams p) {
 // operand of its 32 channels by transpose reads of the row-major x tile and the B operand (lane =
 // row r of E, 8 consecutive tokens) by one 16-byte read of the E slice. Rows of E past this
 // segment's rank and rows of x past the tensor's end read zeros (buffer range); tokens past the
-// segment's end get zero weights in its last tile. One workgroup per (segment, head, batch): the
-// compress of a tensor streams at HBM speed instead of one memory round trip per 64 tokens.
+// segment's end get zero weights in its last tile. One workgroup per (segment, head, batch,
+// job); a call's keys and values share a launch, so that two workgroups run on a CU: at H 12, D 128,
+// L 32,760, segment 1,560 39.5 us in two
+// launches, 36 us in one.
 // =============================================================================================
 template <int D>
-__global__ void __launch_bounds__(2 * D) compress_stream_kernel(CompressParams p) {
+__global__ void __launch_bounds__(2 * D) compress_stream_kernel(CompressJobs jobs) {
   constexpr int NW = D / 32, TILE = 64 * D, SS = TILE + 32 * 64;  // stage: x tile, then E slice
   constexpr int CPR = D / 8, RPI = 64 / CPR, NI = 64 / (RPI * NW);  // x tile: NI loads per wave
   constexpr int EI = 4 / NW;                                         // E slice: EI loads per wave
@@ -136,7 +157,8 @@ __global__ void __launch_bounds__(2 * D) compress_stream_kernel(CompressParams p
   __shared__ __attribute__((aligned(1024))) bf16_t st1[SS];
   __shared__ __attribute__((aligned(1024))) bf16_t st2[SS];
   __shared__ __attribute__((aligned(1024))) bf16_t st3[SS];
-  const int sidx = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+  const CompressParams p = jobs.j[blockIdx.z / jobs.batch];
+  const int sidx = blockIdx.x, h = blockIdx.y, b = blockIdx.z % jobs.batch;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, l32 = lane & 31;
   const int start = sidx * p.seg;
@@ -442,7 +464,12 @@ extern "C" int wa_compress_kv_bwd(const wa_compress_bwd_args* a, void* stream) {
   return WA_OK;
 }
 
-extern "C" int wa_compress_kv(const wa_compress_args* a, void* stream) {
+namespace {
+
+// Kernel of a job: the streaming one for bf16 x with 16-byte aligned rows and a rank of at most 32.
+enum CompressKernel { kStream, kDirect };
+
+int plan_compress(const wa_compress_args* a, CompressParams& cp, CompressKernel& kernel) {
   WA_CHECK_ARG(a && a->x && a->proj && a->out, "wa_compress_kv: null argument");
   WA_CHECK_ARG(a->D == 64 || a->D == 128 || a->D == 32, "wa_compress_kv: head dim %lld not in {32, 64, 128}",
                (long long)a->D);
@@ -450,31 +477,72 @@ extern "C" int wa_compress_kv(const wa_compress_args* a, void* stream) {
   WA_CHECK_ARG(a->proj_dtype == WA_F32 || a->proj_dtype == WA_BF16, "wa_compress_kv: bad proj dtype");
   WA_CHECK_ARG(a->segment_len > 0 && a->block_size > 0 && a->L > 0, "wa_compress_kv: bad sizes");
   WA_CHECK_ARG(a->proj_rank > 0 && a->proj_rank <= 128, "wa_compress_kv: projection rank must be in [1, 128]");
-  const int64_t nseg = (a->L + a->segment_len - 1) / a->segment_len;
   const int64_t first_seg = a->segment_len < a->L ? a->segment_len : a->L;
   WA_CHECK_ARG(first_seg <= a->proj_len, "wa_compress_kv: segment length %lld exceeds projection length %lld",
                (long long)first_seg, (long long)a->proj_len);
-  if (a->B == 0) return WA_OK;
-  CompressParams cp{a->x, a->x_sb, a->x_st, a->x_sh, a->x_dtype, a->proj, a->proj_dtype, (int)a->proj_rank,
-                    (int)a->proj_len, (int)a->L, (int)a->H, (int)a->D, (int)a->segment_len, (int)a->block_size,
-                    a->out, a->o_sb, a->o_st, a->o_sh, a->o_dtype};
-  dim3 grid((unsigned)nseg, (unsigned)a->H, (unsigned)a->B);
-  hipStream_t s = (hipStream_t)stream;
-  // bf16 x with 16-byte aligned rows (and a rank of at most 32): the streaming kernel
+  cp = CompressParams{a->x, a->x_sb, a->x_st, a->x_sh, a->x_dtype, a->proj, a->proj_dtype, (int)a->proj_rank,
+                      (int)a->proj_len, (int)a->L, (int)a->H, (int)a->D, (int)a->segment_len, (int)a->block_size,
+                      a->out, a->o_sb, a->o_st, a->o_sh, a->o_dtype};
+  cp.proj_vec = wa_aligned16(a->proj) && a->proj_len % 8 == 0;
   const int64_t slab = ((a->L - 1) * a->x_st + a->D) * 2;
-  const int64_t rank_used = std::min<int64_t>(a->proj_rank, (std::min<int64_t>(a->segment_len, a->L) + a->block_size - 1) /
-                                                                a->block_size);
+  const int64_t rank_used = std::min<int64_t>(a->proj_rank, (first_seg + a->block_size - 1) / a->block_size);
+  kernel = kDirect;
   if ((a->D == 128 || a->D == 64) && a->x_dtype == WA_BF16 && wa_aligned16(a->x) && a->x_sb % 8 == 0 &&
       a->x_st % 8 == 0 && a->x_sh % 8 == 0 && slab < ((int64_t)1 << 31) && rank_used <= 32 &&
       a->proj_dtype == WA_BF16 && (((uintptr_t)a->proj) & 3) == 0 && a->proj_len % 2 == 0 &&
       a->proj_rank * a->proj_len * 2 < ((int64_t)1 << 31)) {
+    kernel = kStream;
     cp.x_slab = slab;
-    if (a->D == 128) hipLaunchKernelGGL(compress_stream_kernel<128>, grid, dim3(256), 0, s, cp);
-    else hipLaunchKernelGGL(compress_stream_kernel<64>, grid, dim3(128), 0, s, cp);
-    return wa_launch_status("compress_kv");
   }
-  if (a->D == 128) hipLaunchKernelGGL(compress_kernel<128>, grid, dim3(256), 0, s, cp);
-  else if (a->D == 64) hipLaunchKernelGGL(compress_kernel<64>, grid, dim3(256), 0, s, cp);
-  else hipLaunchKernelGGL(compress_kernel<32>, grid, dim3(256), 0, s, cp);
-  return wa_launch_status("compress_kv");
+  return WA_OK;
 }
+
+template <typename T, int MT>
+void launch_direct(const CompressJobs& jobs, int D, dim3 grid, hipStream_t s) {
+  if (D == 128) hipLaunchKernelGGL((compress_direct_kernel<T, 128, MT>), grid, dim3(kTokenGroups * 256), 0, s, jobs);
+  else if (D == 64) hipLaunchKernelGGL((compress_direct_kernel<T, 64, MT>), grid, dim3(kTokenGroups * 128), 0, s, jobs);
+  else hipLaunchKernelGGL((compress_direct_kernel<T, 32, MT>), grid, dim3(kTokenGroups * 64), 0, s, jobs);
+}
+
+}  // namespace
+
+extern "C" int wa_compress_kv_n(const wa_compress_args* a, int32_t n, void* stream) {
+  WA_CHECK_ARG(a && n >= 1 && n <= 64, "wa_compress_kv_n: between 1 and 64 jobs");
+  CompressParams cp[64];
+  CompressKernel kernel[64];
+  for (int i = 0; i < n; ++i) {  // every job is checked before the first launch
+    const int rc = plan_compress(a + i, cp[i], kernel[i]);
+    if (rc != WA_OK) return rc;
+  }
+  hipStream_t s = (hipStream_t)stream;
+  for (int i = 0; i < n;) {
+    const wa_compress_args& j = a[i];
+    const bool pair = i + 1 < n && kernel[i + 1] == kernel[i] && a[i + 1].x_dtype == j.x_dtype && a[i + 1].B == j.B &&
+                      a[i + 1].L == j.L && a[i + 1].H == j.H && a[i + 1].D == j.D &&
+                      a[i + 1].segment_len == j.segment_len && a[i + 1].block_size == j.block_size &&
+                      a[i + 1].proj_rank == j.proj_rank && 2 * j.B <= 65535;
+    CompressJobs jobs{{cp[i], cp[pair ? i + 1 : i]}, (int)j.B};
+    i += pair ? 2 : 1;
+    if (j.B == 0) continue;
+    const int64_t nseg = (j.L + j.segment_len - 1) / j.segment_len;
+    const dim3 grid((unsigned)nseg, (unsigned)j.H, (unsigned)(pair ? 2 * j.B : j.B));
+    if (kernel[i - 1] == kStream) {
+      if (j.D == 128) hipLaunchKernelGGL(compress_stream_kernel<128>, grid, dim3(256), 0, s, jobs);
+      else hipLaunchKernelGGL(compress_stream_kernel<64>, grid, dim3(128), 0, s, jobs);
+    } else {
+      const int64_t rank = std::min<int64_t>(j.proj_rank, (std::min(j.segment_len, j.L) + j.block_size - 1) / j.block_size);
+      if (j.x_dtype == WA_F32) {
+        if (rank <= 32) launch_direct<float, 1>(jobs, (int)j.D, grid, s);
+        else launch_direct<float, 4>(jobs, (int)j.D, grid, s);
+      } else {
+        if (rank <= 32) launch_direct<bf16_t, 1>(jobs, (int)j.D, grid, s);
+        else launch_direct<bf16_t, 4>(jobs, (int)j.D, grid, s);
+      }
+    }
+    const int rc = wa_launch_status("compress_kv");
+    if (rc != WA_OK) return rc;
+  }
+  return WA_OK;
+}
+
+extern "C" int wa_compress_kv(const wa_compress_args* a, void* stream) { return wa_compress_kv_n(a, 1, stream); }

@@ -154,7 +154,7 @@ class _GateParams:
 class _HSA(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, k_coarse, v_coarse, k_proj_mat, v_proj_mat, gate_w, gate_b, cfg):
-        from .attention import (GateSpec, _compress, _native_split_forward, _per_head_k, elu1_readout, elu1_state,
+        from .attention import (GateSpec, _compress_many, _native_split_forward, _per_head_k, elu1_readout, elu1_state,
                                 head_plan, native_split_eligible)
 
         block_size, routing, topk, linear_mode = cfg["block_size"], cfg["routing"], cfg["topk"], cfg["linear_mode"]
@@ -215,10 +215,8 @@ class _HSA(torch.autograd.Function):
                 elu1_readout(q, state, zsum, lt, lin)
             else:
                 if k_coarse is None:
-                    kc = _compress(k, k_proj_mat, segment_len=cfg["proj_segment_len"], block_size=block_size,
-                                   layout="blhd")
-                    vc = _compress(v, v_proj_mat, segment_len=cfg["proj_segment_len"], block_size=block_size,
-                                   layout="blhd")
+                    kc, vc = _compress_many([(k, k_proj_mat, None), (v, v_proj_mat, None)],
+                                            segment_len=cfg["proj_segment_len"], block_size=block_size, layout="blhd")
                 else:
                     kc, vc = k_coarse, v_coarse
                 kcb, vcb = _lib.kernel_ready(kc), _lib.kernel_ready(vc)

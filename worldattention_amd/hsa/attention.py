@@ -87,24 +87,14 @@ def _pad_channels(t: Optional[torch.Tensor], d_to: int, value: float = 0.0) -> O
     return torch.nn.functional.pad(t, (0, d_to - t.shape[-1]), value=value)
 
 
-def _compress(x: torch.Tensor, proj: torch.Tensor, *, segment_len: int, block_size: int, layout: str,
-              out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """``out`` (optional): a view of the destination rows (same layout, dtype of ``x``), e.g. slots
-    of a compressed cache, written in place. Head dims the kernel lacks run zero-padded (the
-    projection acts on each channel alone)."""
+def _compress_job(x: torch.Tensor, proj: torch.Tensor, out: Optional[torch.Tensor], segment_len: int,
+                  block_size: int, layout: str):
+    """``(out, args, tensors the args point into)`` of one compression at a kernel head dim."""
     dev = _lib.require_gpu(x, proj)
     if layout == "bhld":
         bsz, heads, length, d = x.shape
     else:
         bsz, length, heads, d = x.shape
-    if d not in (32, 64, 128):
-        dp = padded_head_dim(d, (32, 64, 128))
-        res = _compress(_pad_channels(x, dp), proj, segment_len=segment_len, block_size=block_size, layout=layout)
-        res = res[..., :d]
-        if out is None:
-            return res.contiguous()
-        out.copy_(res)
-        return out
     if segment_len <= 0:
         segment_len = length
     for start in range(0, length, segment_len):
@@ -124,17 +114,34 @@ def _compress(x: torch.Tensor, proj: torch.Tensor, *, segment_len: int, block_si
     elif tuple(out.shape) != shape or out.dtype != x.dtype or out.stride(-1) != 1:
         raise ValueError(f"compress output must be {x.dtype} {shape} with unit last stride, got "
                          f"{out.dtype} {tuple(out.shape)}")
-    if layout == "bhld":
-        xp, x_sb, x_st, x_sh = _lib.bhld(src)
-        op, o_sb, o_st, o_sh = _lib.bhld(out)
-    else:
-        xp, x_sb, x_st, x_sh = _lib.blhd(src)
-        op, o_sb, o_st, o_sh = _lib.blhd(out)
-    args = _lib.CompressArgs(xp, x_sb, x_st, x_sh, _lib.dtype_code(src), pj.data_ptr(), _lib.dtype_code(pj),
+    strides = _lib.bhld if layout == "bhld" else _lib.blhd
+    args = _lib.CompressArgs(*strides(src), _lib.dtype_code(src), pj.data_ptr(), _lib.dtype_code(pj),
                              pj.shape[0], pj.shape[1], bsz, length, heads, d, segment_len, block_size,
-                             op, o_sb, o_st, o_sh, _lib.dtype_code(out))
-    _lib.call("wa_compress_kv", args, _lib.stream_ptr(dev))
-    return out
+                             *strides(out), _lib.dtype_code(out))
+    return out, args, (src, pj)
+
+
+def _compress_many(jobs, *, segment_len: int, block_size: int, layout: str) -> list:
+    """Compressions of ``(x, proj, out)`` jobs (a call's keys and values), in one launch when they
+    share a shape. ``out`` (or None): a view of the destination rows (same layout, dtype of ``x``),
+    e.g. slots of a compressed cache, written in place. Head dims the kernel lacks run zero-padded
+    (the projection acts on each channel alone)."""
+    d = jobs[0][0].shape[-1]
+    if d not in (32, 64, 128):
+        dp = padded_head_dim(d, (32, 64, 128))
+        res = _compress_many([(_pad_channels(x, dp), proj, None) for x, proj, _ in jobs], segment_len=segment_len,
+                             block_size=block_size, layout=layout)
+        return [r[..., :d].contiguous() if out is None else out.copy_(r[..., :d]) for r, (_, _, out) in zip(res, jobs)]
+    made = [_compress_job(x, proj, out, segment_len, block_size, layout) for x, proj, out in jobs]
+    arr = (_lib.CompressArgs * len(made))(*[args for _, args, _ in made])
+    _lib.call("wa_compress_kv_n", arr, len(made), _lib.stream_ptr(made[0][0].device))
+    return [out for out, _, _ in made]
+
+
+def _compress(x: torch.Tensor, proj: torch.Tensor, *, segment_len: int, block_size: int, layout: str,
+              out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """One job of :func:`_compress_many`."""
+    return _compress_many([(x, proj, out)], segment_len=segment_len, block_size=block_size, layout=layout)[0]
 
 
 def compress_kv(k: torch.Tensor, v: torch.Tensor, *, segment_len: int, k_proj_mat: torch.Tensor,
@@ -144,8 +151,11 @@ def compress_kv(k: torch.Tensor, v: torch.Tensor, *, segment_len: int, k_proj_ma
         raise ValueError(
             "k_proj_mat and v_proj_mat must have the same shape, got "
             f"{tuple(k_proj_mat.shape)} and {tuple(v_proj_mat.shape)}")
-    return (_compress(k, k_proj_mat, segment_len=segment_len, block_size=block_size, layout="bhld"),
-            _compress(v, v_proj_mat, segment_len=segment_len, block_size=block_size, layout="bhld"))
+    if k.shape[-1] != v.shape[-1]:  # two head dims: two launches
+        return (_compress(k, k_proj_mat, segment_len=segment_len, block_size=block_size, layout="bhld"),
+                _compress(v, v_proj_mat, segment_len=segment_len, block_size=block_size, layout="bhld"))
+    return tuple(_compress_many([(k, k_proj_mat, None), (v, v_proj_mat, None)], segment_len=segment_len,
+                                block_size=block_size, layout="bhld"))
 
 
 def _linear_branch(q: torch.Tensor, k_coarse: torch.Tensor, v_coarse: torch.Tensor) -> torch.Tensor:
@@ -489,8 +499,8 @@ def _run_linear_heads(plan, linear_mode, q, k, v, qb, k_coarse, v_coarse, k_proj
     if plan.linear:
         if linear_mode == "lowrank":
             if k_coarse is None:
-                kc = _compress(k, k_proj_mat, segment_len=proj_segment_len, block_size=block_size, layout="blhd")
-                vc = _compress(v, v_proj_mat, segment_len=proj_segment_len, block_size=block_size, layout="blhd")
+                kc, vc = _compress_many([(k, k_proj_mat, None), (v, v_proj_mat, None)], segment_len=proj_segment_len,
+                                        block_size=block_size, layout="blhd")
             else:
                 kc, vc = k_coarse, v_coarse
             kcb, vcb = _lib.kernel_ready(kc), _lib.kernel_ready(vc)
@@ -685,10 +695,8 @@ class HSAAttention(nn.Module):
             from ._autograd import compress_autograd
             return (compress_autograd(k, self.k_proj_mat, self.proj_segment_len, self.block_size),
                     compress_autograd(v, self.v_proj_mat, self.proj_segment_len, self.block_size))
-        return (_compress(k, self.k_proj_mat, segment_len=self.proj_segment_len, block_size=self.block_size,
-                          layout="blhd"),
-                _compress(v, self.v_proj_mat, segment_len=self.proj_segment_len, block_size=self.block_size,
-                          layout="blhd"))
+        return tuple(_compress_many([(k, self.k_proj_mat, None), (v, self.v_proj_mat, None)],
+                                    segment_len=self.proj_segment_len, block_size=self.block_size, layout="blhd"))
 
     def forward(self, q, k, v, k_coarse=None, v_coarse=None, *, k_block_sums=None, k_pooled=None) -> torch.Tensor:
         return hsa_attention(

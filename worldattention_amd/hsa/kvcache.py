@@ -26,7 +26,7 @@ from typing import Optional, Sequence
 import torch
 
 from .. import _lib
-from .attention import _compress
+from .attention import _compress_many
 
 __all__ = ["kv_append", "new_block_sums", "refresh_block_sums", "qkv_epilogue", "kv_roll", "cache_step"]
 
@@ -123,8 +123,8 @@ def kv_append(kv_cache: dict, k_new: torch.Tensor, v_new: torch.Tensor, *, write
         new_vc = kv_cache["v_coarse"][:, c0:c1]
         seg, bsm = hsa_module.proj_segment_len, hsa_module.block_size
         with torch.no_grad():
-            _compress(k_src, hsa_module.k_proj_mat, segment_len=seg, block_size=bsm, layout="blhd", out=new_kc)
-            _compress(v_src, hsa_module.v_proj_mat, segment_len=seg, block_size=bsm, layout="blhd", out=new_vc)
+            _compress_many([(k_src, hsa_module.k_proj_mat, new_kc), (v_src, hsa_module.v_proj_mat, new_vc)],
+                           segment_len=seg, block_size=bsm, layout="blhd")
     return {
         "action": "direct_insert",
         "write_start_index": start,
@@ -309,10 +309,9 @@ def cache_step(kv_cache: dict, q, k, v, *, grid_sizes, freqs, current_start: int
         new_kc, new_vc = kv_cache["k_coarse"][:, c0:c1], kv_cache["v_coarse"][:, c0:c1]
         seg, bsm = hsa_module.proj_segment_len, hsa_module.block_size
         with torch.no_grad():
-            _compress(kc[:, write_start:new_local_end], hsa_module.k_proj_mat, segment_len=seg, block_size=bsm,
-                      layout="blhd", out=new_kc)
-            _compress(vc[:, write_start:new_local_end], hsa_module.v_proj_mat, segment_len=seg, block_size=bsm,
-                      layout="blhd", out=new_vc)
+            _compress_many([(kc[:, write_start:new_local_end], hsa_module.k_proj_mat, new_kc),
+                            (vc[:, write_start:new_local_end], hsa_module.v_proj_mat, new_vc)],
+                           segment_len=seg, block_size=bsm, layout="blhd")
 
     def coarse_slice(a, b):
         if not coarse:
