@@ -428,7 +428,9 @@ int wa_compress_kv_n(const wa_compress_args* args, int32_t n, void* stream);
  *   dx[b, start + t, h, :] = sum_j E[j, t] dout[b, row0 + j, h, :]      (fp32; optional)
  *   dproj[j, t] = sum over segments, batches, heads and channels of dout[row0 + j] x[start + t]
  * dproj (optional) is [proj_rank, proj_len] fp32 row-major; entries no segment covers get zero.
- * With *_accumulate set the gradient is added to the existing contents. fp32 arithmetic; the
+ * With *_accumulate set the gradient is added to the existing contents. With dx_bf16 (optional) the
+ * x gradient, added to dx if dx_accumulate asks for it, is written there in bf16 and dx is only read
+ * (or NULL). fp32 arithmetic; the
  * dproj sum runs in a fixed order (per-segment partials in `workspace`, of
  * wa_compress_kv_bwd_workspace_bytes, added in segment order), so results repeat bit for bit.
  * dout and dx are read / written by float4 and x by 16 bytes: each must be 16-byte aligned with
@@ -442,6 +444,7 @@ typedef struct wa_compress_bwd_args {
   float* dx; int64_t dx_sb, dx_st, dx_sh; int32_t dx_accumulate;
   float* dproj; int32_t dproj_accumulate;
   void* workspace;
+  void* dx_bf16; int64_t dxo_sb, dxo_st, dxo_sh;
 } wa_compress_bwd_args;
 int64_t wa_compress_kv_bwd_workspace_bytes(int64_t L, int64_t proj_rank, int64_t segment_len, int64_t block_size);
 int wa_compress_kv_bwd(const wa_compress_bwd_args* args, void* stream);

@@ -192,6 +192,47 @@ def test_compress_backward_matches_oracle_autograd(b, length, h, d, seg, bs, ran
     assert_close(dx2, base + dx, 1e-6, 1e-7, what="accumulated dx")
 
 
+@pytest.mark.parametrize("b,length,h,d,seg,bs,rank,xdt,pdt", [
+    (1, 133, 5, 64, 100, 64, 2, torch.bfloat16, torch.bfloat16),    # a last segment of rank 1; 10 columns of 32
+    (2, 260, 1, 128, 130, 4, 33, torch.float32, torch.float32),     # one row in a second 32-row tile
+    (1, 640, 3, 32, 320, 4, 80, torch.float32, torch.float32),      # rank over 64
+    (1, 64, 2, 128, 64, 1, 64, torch.bfloat16, torch.float32),      # exactly one token tile and two row tiles
+    (3, 65, 2, 64, 65, 1, 65, torch.float32, torch.bfloat16),       # one token and one row past the tiles
+])
+def test_compress_backward_split_products_match_fp64(b, length, h, d, seg, bs, rank, xdt, pdt):
+    """dx and dE on the matrix cores from three-part splits of the fp32 operands, against fp64: a sum
+    of n fp32 products in any order is within n 2^-24 of the sum of their magnitudes; the bf16 form
+    of dx is the rounding of the fp32 one, and infinities and NaN in a gradient column stay in it."""
+    from worldattention_amd.hsa._autograd import _compress_backward
+    torch.manual_seed(length + rank)
+    x = torch.randn(b, length, h, d, device=DEV).to(xdt)
+    proj = (torch.randn(rank, seg, device=DEV) / 16).to(pdt)
+    spans = [(s, min(seg, length - s)) for s in range(0, length, seg)]
+    ranks = [min(rank, -(-n // bs)) for _, n in spans]
+    g = torch.randn(b, sum(ranks), h, d, device=DEV) * torch.randn(b, sum(ranks), h, d, device=DEV).exp()
+    base = torch.randn(b, length, h, d, device=DEV)
+    dx, dp = _compress_backward(g, x, proj, seg, bs)
+    added, _ = _compress_backward(g, x, proj, seg, bs, dx=base.clone())
+    rounded, _ = _compress_backward(g, x, proj, seg, bs, dx=base, out_dtype=torch.bfloat16)
+    assert torch.equal(added, base + dx) and torch.equal(rounded, added.bfloat16())
+    want_p, row = torch.zeros(2, rank, seg, dtype=torch.float64, device=DEV), 0
+    for (s, n), r in zip(spans, ranks):
+        e, xs, gs = proj[:r, :n].double(), x[:, s:s + n].double(), g[:, row:row + r].double()
+        want = torch.einsum("jt,bjhd->bthd", e, gs)
+        bound = (r + 2) * 2.0 ** -24 * torch.einsum("jt,bjhd->bthd", e.abs(), gs.abs())
+        assert ((dx[:, s:s + n].double() - want).abs() <= bound).all(), f"dx of segment {s}"
+        want_p[0, :r, :n] += torch.einsum("bjhd,bthd->jt", gs, xs)
+        want_p[1, :r, :n] += torch.einsum("bjhd,bthd->jt", gs.abs(), xs.abs())
+        row += r
+    assert ((dp.double() - want_p[0]).abs() <= (b * h * d + len(spans) + 8) * 2.0 ** -24 * want_p[1]).all()
+    g[0, 0, 0, 0], g[0, 0, 0, 1], g[0, 0, 0, 2] = float("inf"), float("nan"), 3.3e38
+    odd, _ = _compress_backward(g, x, proj, seg, bs)
+    t0 = spans[0][1] // 2
+    want = torch.einsum("jt,jd->td", proj[:ranks[0], t0:t0 + 1].double(), g[0, :ranks[0], 0, :4].double())
+    assert torch.equal(odd[0, t0, 0, 0].double(), want[0, 0]) and odd[0, t0, 0, 1].isnan()
+    assert (odd[0, t0, 0, 2].double() - want[0, 2]).abs() <= 1e-6 * want[0, 2].abs()
+
+
 def test_hsa_reference_mode_gradients_match_oracle():
     """Reference semantics: every head runs both branches, Gini routing, low-rank softmax branch."""
     torch.manual_seed(3)

@@ -145,6 +145,7 @@ CompressBwdArgs = _struct("wa_compress_bwd_args", [
     ("dx", c_void_p), ("dx_sb", c_int64), ("dx_st", c_int64), ("dx_sh", c_int64), ("dx_accumulate", c_int32),
     ("dproj", c_void_p), ("dproj_accumulate", c_int32),
     ("workspace", c_void_p),
+    ("dx_bf16", c_void_p), ("dxo_sb", c_int64), ("dxo_st", c_int64), ("dxo_sh", c_int64),
 ])
 
 Elu1StateArgs = _struct("wa_elu1_state_args", [

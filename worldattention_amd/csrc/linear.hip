@@ -251,129 +251,254 @@ struct CompressBwdParams {
   const void* proj; int proj_dtype; int R, P;
   int B, L, H, D, seg, block, n_first, r_full, n_seg;
   float* dx; int64_t dx_sb, dx_st, dx_sh; int dx_acc;
+  void* dx_out; int64_t dxo_sb, dxo_st, dxo_sh;  // bf16 result instead of writing dx back
   float* dproj; int dproj_acc;
   float* part;  // [n_seg][r_full][n_first]
 };
 
-__device__ __forceinline__ float proj_at(const CompressBwdParams& p, int j, int t) {
-  const int64_t off = (int64_t)j * p.P + t;
-  return p.proj_dtype == WA_BF16 ? (float)((const bf16_t*)p.proj)[off] : ((const float*)p.proj)[off];
+// fp32 products on the bf16 matrix cores: a float is the exact sum of three bf16 values of 8
+// significant bits each (cut off, not rounded, so hi never overflows; infinities keep zero lower
+// parts and NaN stays NaN). A bf16 operand times the three parts is exact before the fp32
+// accumulation; two split operands use every product but lo lo (2^-32 of the leading one). An
+// operand's infinities and NaN (its exponent field all ones) enter the leading product alone: the
+// others take `fin`, hi with those values 0, so that infinity never meets a zero lower part.
+struct Plain {
+  bf16x8 hi, fin;
+};
+struct Split3 {
+  bf16x8 hi, mid, lo, fin;
+};
+
+__device__ __forceinline__ bf16x8 finite8(const bf16x8& v) {
+  u32x4 u = __builtin_bit_cast(u32x4, v);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if ((u[q] & 0x7f80u) == 0x7f80u) u[q] &= 0xffff0000u;
+    if ((u[q] & 0x7f800000u) == 0x7f800000u) u[q] &= 0xffffu;
+  }
+  return __builtin_bit_cast(bf16x8, u);
 }
 
-// dx: one workgroup per (16-token tile of a segment, 128 float4 columns of (head, channel), batch);
-// a thread keeps its column of the segment's dout rows 16 at a time in registers and the matching
-// 16 x 16 block of E in LDS, and sums over j in increasing order.
-constexpr int kDxTokens = 16, kDxRows = 16, kDxThreads = 128;
-__global__ void __launch_bounds__(kDxThreads) compress_bwd_dx_kernel(CompressBwdParams p) {
-  __shared__ float es[kDxRows][kDxTokens];
+__device__ __forceinline__ Split3 split3(const float (&v)[8]) {
+  u32x4 h, m, l;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    uint32_t hb[2], mb[2], lb[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float x = v[2 * q + i];
+      hb[i] = __float_as_uint(x);
+      const float xh = __uint_as_float(hb[i] & 0xffff0000u);
+      const float r = x == xh ? 0.f : x - xh;
+      mb[i] = __float_as_uint(r);
+      const float rm = __uint_as_float(mb[i] & 0xffff0000u);
+      lb[i] = __float_as_uint(r == rm ? 0.f : r - rm);
+    }
+    // the high halves of two floats side by side
+    h[q] = __builtin_amdgcn_perm(hb[1], hb[0], 0x07060302);
+    m[q] = __builtin_amdgcn_perm(mb[1], mb[0], 0x07060302);
+    l[q] = __builtin_amdgcn_perm(lb[1], lb[0], 0x07060302);
+  }
+  const bf16x8 hi = __builtin_bit_cast(bf16x8, h);
+  return {hi, __builtin_bit_cast(bf16x8, m), __builtin_bit_cast(bf16x8, l), finite8(hi)};
+}
+
+// hi + lo += a b, smallest products first; of two split operands only the leading products go to hi,
+// so that it takes one rounding per 16 terms, as with a bf16 operand's three.
+__device__ __forceinline__ void mfma_split(const Split3& a, const Plain& b, f32x16& hi, f32x16&) {
+  hi = wa_mfma32(a.lo, b.fin, hi);
+  hi = wa_mfma32(a.mid, b.fin, hi);
+  hi = wa_mfma32(a.hi, b.hi, hi);
+}
+__device__ __forceinline__ void mfma_split(const Split3& a, const Split3& b, f32x16& hi, f32x16& lo) {
+  lo = wa_mfma32(a.lo, b.mid, lo);
+  lo = wa_mfma32(a.mid, b.lo, lo);
+  lo = wa_mfma32(a.lo, b.fin, lo);
+  lo = wa_mfma32(a.fin, b.lo, lo);
+  lo = wa_mfma32(a.mid, b.mid, lo);
+  lo = wa_mfma32(a.mid, b.fin, lo);
+  lo = wa_mfma32(a.fin, b.mid, lo);
+  hi = wa_mfma32(a.hi, b.hi, hi);
+}
+
+// dx: one workgroup per (64-token tile of a segment, four 32-channel columns of (head, channel),
+// batch); wave w owns column 4 blockIdx.x + w. dx^T = dout^T E with E from LDS by transpose reads
+// (32 rank rows x 64 tokens at a time) and dout split in registers; lane = token, registers = four
+// consecutive channels, so the fp32 gradient it adds to is read by 16 bytes per lane and the result
+// stored by 16 (bf16: 8). Bound by that traffic: the products are 6 (bf16 E) or 12 per 32 x 32 tile.
+// H 12, D 128, L 32,760, rank 25: adding to an fp32 gradient and writing it back took 142 us as fp32
+// VALU products, and a separate pass to bf16 51 us more; here adding and writing bf16 takes
+// 118 us (with lane = channel, 4-byte reads and 2-byte stores: 129 us).
+constexpr int kDxTokens = 64;
+
+template <typename PT>
+__global__ void __launch_bounds__(256) compress_bwd_dx_kernel(CompressBwdParams p) {
+  constexpr bool SPLIT_E = sizeof(PT) == 4;
+  constexpr int ET = 32 * kDxTokens;
+  __shared__ __attribute__((aligned(1024))) bf16_t es[(SPLIT_E ? 3 : 1) * ET];
   const int tps = (p.n_first + kDxTokens - 1) / kDxTokens;
-  const int s = blockIdx.x / tps, t0 = (blockIdx.x % tps) * kDxTokens, b = blockIdx.z;
+  const int s = blockIdx.y / tps, t0 = (blockIdx.y % tps) * kDxTokens, b = blockIdx.z;
   const int start = s * p.seg, n = min(p.seg, p.L - start);
   if (t0 >= n) return;  // uniform
   const int r = min(p.R, (n + p.block - 1) / p.block), row0 = s * p.r_full;
-  const int tid = threadIdx.x;
-  const int c = blockIdx.y * kDxThreads + tid;  // float4 column
-  const bool active = c < p.H * p.D / 4;
-  const int h = active ? c * 4 / p.D : 0, d = active ? c * 4 % p.D : 0;
-  const float* gcol = p.dout + (int64_t)b * p.d_sb + (int64_t)h * p.d_sh + d;
-  f32x4 acc[kDxTokens];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 5, l32 = lane & 31;
+  const int ct = blockIdx.x * 4 + w;
+  const bool active = ct < p.H * p.D / 32;  // uniform over the wave
+  const int h = active ? ct * 32 / p.D : 0, d = active ? ct * 32 % p.D : 0;
+  const float* gcol = p.dout + (int64_t)b * p.d_sb + (int64_t)row0 * p.d_st + (int64_t)h * p.d_sh + d + l32;
+  // this lane's tokens t0 + 32 tt + l32, channels d + 8 rq + 4 g + i
+  const int64_t dx0 = (int64_t)b * p.dx_sb + (int64_t)start * p.dx_st + (int64_t)h * p.dx_sh + d + 4 * g;
+  f32x4 prev[2][4];
 #pragma unroll
-  for (int i = 0; i < kDxTokens; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int j0 = 0; j0 < r; j0 += kDxRows) {
-    __syncthreads();  // the previous block of E has been read
-    for (int i = tid; i < kDxRows * kDxTokens; i += kDxThreads) {
-      const int jj = i / kDxTokens, tl = i % kDxTokens, j = j0 + jj, t = t0 + tl;
-      es[jj][tl] = j < r && t < n ? proj_at(p, j, t) : 0.f;
+  for (int tt = 0; tt < 2; ++tt) {
+#pragma unroll
+    for (int rq = 0; rq < 4; ++rq)
+      prev[tt][rq] = p.dx_acc && active
+                         ? *(const f32x4*)(p.dx + dx0 + (int64_t)min(t0 + 32 * tt + l32, n - 1) * p.dx_st + 8 * rq)
+                         : f32x4{};
+  }
+  f32x16 acc[2] = {f32x16{}, f32x16{}}, low[2] = {f32x16{}, f32x16{}};
+  for (int j0 = 0; j0 < r; j0 += 32) {
+    if (j0) __syncthreads();  // the previous rows have been read
+    {
+      const int jj = tid / 8, c = tid % 8, j = j0 + jj, t = t0 + 8 * c;  // 8 tokens of one row per thread
+      float e8[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) e8[e] = j < r && t + e < n ? (float)((const PT*)p.proj)[(int64_t)j * p.P + t + e] : 0.f;
+      const Split3 sp = split3(e8);  // a bf16 value is its own hi part
+      tile_put8<kDxTokens>(es, jj, c, sp.hi);
+      if constexpr (SPLIT_E) {
+        tile_put8<kDxTokens>(es + ET, jj, c, sp.mid);
+        tile_put8<kDxTokens>(es + 2 * ET, jj, c, sp.lo);
+      }
     }
-    f32x4 g[kDxRows];
+    Split3 gs[2];
 #pragma unroll
-    for (int jj = 0; jj < kDxRows; ++jj)
-      g[jj] = active && j0 + jj < r ? *(const f32x4*)(gcol + (int64_t)(row0 + j0 + jj) * p.d_st)
-                                    : f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int ks = 0; ks < 2; ++ks) {
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int j = j0 + 16 * ks + 8 * g + e;
+        v[e] = gcol[(int64_t)min(j, r - 1) * p.d_st];
+        if (j >= r) v[e] = 0.f;
+      }
+      gs[ks] = split3(v);
+    }
     __syncthreads();
 #pragma unroll
-    for (int tl = 0; tl < kDxTokens; ++tl) {
+    for (int tt = 0; tt < 2; ++tt) {
 #pragma unroll
-      for (int jj = 0; jj < kDxRows; ++jj) {
-        const float e = es[jj][tl];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) acc[tl][q] = fmaf(e, g[jj][q], acc[tl][q]);
+      for (int ks = 0; ks < 2; ++ks) {
+        const bf16x8 eh = tile_tr8n<kDxTokens>(es, ks, 32 * tt, lane);
+        if constexpr (SPLIT_E) {
+          const Split3 ea = {eh, tile_tr8n<kDxTokens>(es + ET, ks, 32 * tt, lane),
+                             tile_tr8n<kDxTokens>(es + 2 * ET, ks, 32 * tt, lane), finite8(eh)};
+          mfma_split(gs[ks], ea, acc[tt], low[tt]);
+        } else {
+          mfma_split(gs[ks], Plain{eh, finite8(eh)}, acc[tt], low[tt]);
+        }
       }
     }
   }
   if (!active) return;
 #pragma unroll
-  for (int tl = 0; tl < kDxTokens; ++tl) {
-    const int t = t0 + tl;
-    if (t >= n) break;
-    f32x4* dst = (f32x4*)(p.dx + (int64_t)b * p.dx_sb + (int64_t)(start + t) * p.dx_st + (int64_t)h * p.dx_sh + d);
-    *dst = p.dx_acc ? *dst + acc[tl] : acc[tl];
+  for (int tt = 0; tt < 2; ++tt) {
+    const int t = t0 + 32 * tt + l32;
+    if (t >= n) continue;
+    bf16_t* o16 = (bf16_t*)p.dx_out + ((int64_t)b * p.dxo_sb + (int64_t)(start + t) * p.dxo_st + (int64_t)h * p.dxo_sh + d + 4 * g);
+    float* o32 = p.dx + dx0 + (int64_t)t * p.dx_st;
+#pragma unroll
+    for (int rq = 0; rq < 4; ++rq) {
+      f32x4 v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float a = SPLIT_E ? acc[tt][4 * rq + i] + low[tt][4 * rq + i] : acc[tt][4 * rq + i];
+        v[i] = prev[tt][rq][i] + a;
+      }
+      if (p.dx_out) *(bf16x4*)(o16 + 8 * rq) = bf16x4{(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]};
+      else *(f32x4*)(o32 + 8 * rq) = v;
+    }
   }
 }
 
-// dE share of one segment: one workgroup of 4 waves per (64-token tile, segment); lane = token,
-// wave w sums heads w, w + 4, ... of every batch for all r rows, then the four waves' sums are added
-// in wave order through LDS into the segment's partial.
-template <int RMAX>
-__global__ void __launch_bounds__(256) compress_bwd_dproj_kernel(CompressBwdParams p) {
-  __shared__ float red[4][16][64];
+// dE share of one segment, as dout (rows) times x^T over (batch, head, channel): one workgroup of 8
+// waves per (64-token tile, segment); wave w sums the 32-channel runs w, w + 8, ... on the matrix
+// cores (A: dout rows split in three, B: x rows, lane = token), then the waves' sums are added in
+// wave order through LDS into the segment's partial. Bound by reading x once (each token tile
+// re-reads the segment's dout rows from L2). H 12, D 128, L 32,760, rank 25, bf16 x: 251 us as fp32
+// VALU products, 60 us with four waves a workgroup, 50 us here.
+constexpr int kDprojWaves = 8;
+
+template <typename T, int MT>
+__global__ void __launch_bounds__(64 * kDprojWaves) compress_bwd_dproj_kernel(CompressBwdParams p) {
+  __shared__ float red[kDprojWaves][16][64];
+  constexpr bool SPLIT_X = sizeof(T) == 4, LOW = SPLIT_X && MT < 4;  // (registers)
   const int s = blockIdx.y, t0 = blockIdx.x * 64;
   const int start = s * p.seg, n = min(p.seg, p.L - start);
   if (t0 >= n) return;  // uniform
   const int r = min(p.R, (n + p.block - 1) / p.block), row0 = s * p.r_full;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int t = t0 + lane;
-  const bool ok = t < n;
-  float acc[RMAX];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 5, l32 = lane & 31;
+  f32x16 acc[MT][2], low[MT][2];
 #pragma unroll
-  for (int j = 0; j < RMAX; ++j) acc[j] = 0.f;
-  for (int b = 0; b < p.B; ++b) {
-    for (int h = w; h < p.H; h += 4) {
-      const int64_t xo = (int64_t)b * p.x_sb + (int64_t)(start + (ok ? t : 0)) * p.x_st + (int64_t)h * p.x_sh;
-      const float* grow = p.dout + (int64_t)b * p.d_sb + (int64_t)row0 * p.d_st + (int64_t)h * p.d_sh;
-      for (int d0 = 0; d0 < p.D; d0 += 8) {
-        float xf[8];
-        if (p.x_dtype == WA_BF16) {
-          const bf16x8 v = *(const bf16x8*)((const bf16_t*)p.x + xo + d0);
+  for (int m = 0; m < MT; ++m) acc[m][0] = acc[m][1] = low[m][0] = low[m][1] = f32x16{};
+  // rows past the rank and tokens past the segment repeat the last one (their results are dropped)
+  int64_t xo[2], go[MT];
 #pragma unroll
-          for (int e = 0; e < 8; ++e) xf[e] = ok ? (float)v[e] : 0.f;
+  for (int tt = 0; tt < 2; ++tt) xo[tt] = (int64_t)(start + min(t0 + 32 * tt + l32, n - 1)) * p.x_st + 8 * g;
+#pragma unroll
+  for (int m = 0; m < MT; ++m) go[m] = (int64_t)(row0 + min(32 * m + l32, r - 1)) * p.d_st + 8 * g;
+  const int runs = p.D / 32, total = p.B * p.H * runs;
+#pragma unroll 2
+  for (int u = w; u < total; u += kDprojWaves) {
+    const int bh = u / runs, c0 = (u % runs) * 32, b = bh / p.H, h = bh % p.H;
+    const T* xb = (const T*)p.x + (int64_t)b * p.x_sb + (int64_t)h * p.x_sh + c0;
+    const float* gb = p.dout + (int64_t)b * p.d_sb + (int64_t)h * p.d_sh + c0;
+#pragma unroll
+    for (int d0 = 0; d0 < 32; d0 += 16) {
+      std::conditional_t<SPLIT_X, Split3, Plain> xf[2];
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt) {
+        if constexpr (SPLIT_X) {
+          const f32x4 v0 = *(const f32x4*)(xb + xo[tt] + d0), v1 = *(const f32x4*)(xb + xo[tt] + d0 + 4);
+          const float v[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+          xf[tt] = split3(v);
         } else {
-          const f32x4 v0 = *(const f32x4*)((const float*)p.x + xo + d0);
-          const f32x4 v1 = *(const f32x4*)((const float*)p.x + xo + d0 + 4);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            xf[e] = ok ? v0[e] : 0.f;
-            xf[4 + e] = ok ? v1[e] : 0.f;
-          }
+          const bf16x8 v = *(const bf16x8*)(xb + xo[tt] + d0);
+          xf[tt] = {v, finite8(v)};
         }
+      }
 #pragma unroll
-        for (int j = 0; j < RMAX; ++j) {
-          if (j >= r) break;
-          const f32x4 g0 = *(const f32x4*)(grow + (int64_t)j * p.d_st + d0);
-          const f32x4 g1 = *(const f32x4*)(grow + (int64_t)j * p.d_st + d0 + 4);
-          float a = acc[j];
+      for (int m = 0; m < MT; ++m) {
+        if (32 * m >= r) break;  // uniform
+        const f32x4 v0 = *(const f32x4*)(gb + go[m] + d0), v1 = *(const f32x4*)(gb + go[m] + d0 + 4);
+        const float v[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+        const Split3 gs = split3(v);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) a = fmaf(xf[e], g0[e], a);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) a = fmaf(xf[4 + e], g1[e], a);
-          acc[j] = a;
-        }
+        for (int tt = 0; tt < 2; ++tt) mfma_split(gs, xf[tt], acc[m][tt], LOW ? low[m][tt] : acc[m][tt]);
       }
     }
   }
   float* part = p.part + (int64_t)s * p.r_full * p.n_first;
 #pragma unroll
-  for (int j0 = 0; j0 < RMAX; j0 += 16) {
-    if (j0 >= r) break;
-    __syncthreads();
+  for (int m = 0; m < MT; ++m) {
+    if (32 * m >= r) break;
 #pragma unroll
-    for (int jj = 0; jj < 16; ++jj) red[w][jj][lane] = acc[j0 + jj < RMAX ? j0 + jj : 0];
-    __syncthreads();
-    // wave q writes rows j0 + q, j0 + q + 4, ...: the sum over waves 0..3 in order
-    for (int jj = w; jj < 16; jj += 4) {
-      const int j = j0 + jj;
-      if (j < r && ok)
-        part[(int64_t)j * p.n_first + t] = ((red[0][jj][lane] + red[1][jj][lane]) + red[2][jj][lane]) + red[3][jj][lane];
+    for (int tt = 0; tt < 2; ++tt) {
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < 16; ++i) red[w][i][lane] = LOW ? acc[m][tt][i] + low[m][tt][i] : acc[m][tt][i];
+      __syncthreads();
+      // wave q adds registers q, q + 8: lane (l32, g) of register i is row 32 m + 8 (i / 4) + 4 g + i % 4
+      const int t = t0 + 32 * tt + l32;
+      for (int i = w; i < 16; i += kDprojWaves) {
+        const int j = 32 * m + 8 * (i >> 2) + 4 * g + (i & 3);
+        float v = red[0][i][lane];
+#pragma unroll
+        for (int q = 1; q < kDprojWaves; ++q) v += red[q][i][lane];
+        if (j < r && t < n) part[(int64_t)j * p.n_first + t] = v;
+      }
     }
   }
 }
@@ -386,10 +511,21 @@ __global__ void __launch_bounds__(256) compress_bwd_reduce_kernel(CompressBwdPar
   const int j = (int)(i / p.P), t = (int)(i % p.P);
   float sum = 0.f;
   if (j < p.r_full && t < p.n_first) {
-    for (int s = 0; s < p.n_seg; ++s) {
+    // every segment but the last is full: it covers (j, t)
+    const float* pp = p.part + (int64_t)j * p.n_first + t;
+    const int64_t stride = (int64_t)p.r_full * p.n_first;
+    int s = 0;
+    for (; s + 8 < p.n_seg; s += 8) {  // eight loads in flight
+      float v[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v[q] = pp[(s + q) * stride];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) sum += v[q];
+    }
+    for (; s < p.n_seg; ++s) {
       const int n = min(p.seg, p.L - s * p.seg);
       const int r = min(p.R, (n + p.block - 1) / p.block);
-      if (j < r && t < n) sum += p.part[((int64_t)s * p.r_full + j) * p.n_first + t];
+      if (j < r && t < n) sum += pp[s * stride];
     }
   }
   p.dproj[i] = p.dproj_acc ? p.dproj[i] + sum : sum;
@@ -419,7 +555,7 @@ extern "C" int wa_compress_kv_bwd(const wa_compress_bwd_args* a, void* stream) {
   const int64_t n_first = a->segment_len < a->L ? a->segment_len : a->L;
   WA_CHECK_ARG(n_first <= a->proj_len, "wa_compress_kv_bwd: segment length %lld exceeds projection length %lld",
                (long long)n_first, (long long)a->proj_len);
-  // vector accesses: dout / dx by float4, x by 16 bytes (8 bf16 or 2 x 4 fp32)
+  // vector accesses: dout by float4, x by 16 bytes (8 bf16 or 2 x 4 fp32)
   const int64_t xv = a->x_dtype == WA_BF16 ? 8 : 4;
   WA_CHECK_ARG(wa_aligned16(a->dout) && a->d_sb % 4 == 0 && a->d_st % 4 == 0 && a->d_sh % 4 == 0,
                "wa_compress_kv_bwd: dout must be 16-byte aligned with strides that are multiples of 4");
@@ -427,6 +563,9 @@ extern "C" int wa_compress_kv_bwd(const wa_compress_bwd_args* a, void* stream) {
                "wa_compress_kv_bwd: x must be 16-byte aligned with strides that are multiples of 16 bytes");
   WA_CHECK_ARG(a->dx == nullptr || (wa_aligned16(a->dx) && a->dx_sb % 4 == 0 && a->dx_st % 4 == 0 && a->dx_sh % 4 == 0),
                "wa_compress_kv_bwd: dx must be 16-byte aligned with strides that are multiples of 4");
+  WA_CHECK_ARG(a->dx_bf16 == nullptr || (((uintptr_t)a->dx_bf16 & 7u) == 0 && a->dxo_sb % 4 == 0 && a->dxo_st % 4 == 0 &&
+                                         a->dxo_sh % 4 == 0),
+               "wa_compress_kv_bwd: dx_bf16 must be 8-byte aligned with strides that are multiples of 4");
   WA_CHECK_ARG(a->L <= INT32_MAX && a->proj_rank * a->proj_len <= INT32_MAX, "wa_compress_kv_bwd: sizes too large");
   const int64_t r_full = std::min(a->proj_rank, (n_first + a->block_size - 1) / a->block_size);
   const int64_t n_seg = (a->L + a->segment_len - 1) / a->segment_len;
@@ -434,24 +573,29 @@ extern "C" int wa_compress_kv_bwd(const wa_compress_bwd_args* a, void* stream) {
                        a->proj, a->proj_dtype, (int)a->proj_rank, (int)a->proj_len,
                        (int)a->B, (int)a->L, (int)a->H, (int)a->D, (int)a->segment_len, (int)a->block_size,
                        (int)n_first, (int)r_full, (int)n_seg,
-                       a->dx, a->dx_sb, a->dx_st, a->dx_sh, a->dx_accumulate,
+                       a->dx, a->dx_sb, a->dx_st, a->dx_sh, a->dx ? a->dx_accumulate : 0,
+                       a->dx_bf16, a->dxo_sb, a->dxo_st, a->dxo_sh,
                        a->dproj, a->dproj_accumulate, (float*)a->workspace};
   hipStream_t s = (hipStream_t)stream;
-  if (a->B > 0 && a->dx) {
+  if (a->B > 0 && (a->dx || a->dx_bf16)) {
     const int64_t tps = (n_first + kDxTokens - 1) / kDxTokens;
-    const int64_t cols = a->H * a->D / 4;
-    dim3 grid((unsigned)(n_seg * tps), (unsigned)((cols + kDxThreads - 1) / kDxThreads), (unsigned)a->B);
-    hipLaunchKernelGGL(compress_bwd_dx_kernel, grid, dim3(kDxThreads), 0, s, cp);
+    // the columns of a token tile are neighbours in launch order: whole rows of memory at a time
+    dim3 grid((unsigned)((a->H * a->D / 32 + 3) / 4), (unsigned)(n_seg * tps), (unsigned)a->B);
+    if (a->proj_dtype == WA_BF16) hipLaunchKernelGGL(compress_bwd_dx_kernel<bf16_t>, grid, dim3(256), 0, s, cp);
+    else hipLaunchKernelGGL(compress_bwd_dx_kernel<float>, grid, dim3(256), 0, s, cp);
     const int rc = wa_launch_status("compress_kv_bwd (dx)");
     if (rc != WA_OK) return rc;
   }
   if (a->dproj) {
     if (a->B > 0) {
       dim3 grid((unsigned)((n_first + 63) / 64), (unsigned)n_seg);
-      if (r_full <= 16) hipLaunchKernelGGL(compress_bwd_dproj_kernel<16>, grid, dim3(256), 0, s, cp);
-      else if (r_full <= 32) hipLaunchKernelGGL(compress_bwd_dproj_kernel<32>, grid, dim3(256), 0, s, cp);
-      else if (r_full <= 64) hipLaunchKernelGGL(compress_bwd_dproj_kernel<64>, grid, dim3(256), 0, s, cp);
-      else hipLaunchKernelGGL(compress_bwd_dproj_kernel<128>, grid, dim3(256), 0, s, cp);
+      auto go = [&](auto bf, auto fp) {
+        if (a->x_dtype == WA_BF16) hipLaunchKernelGGL(bf, grid, dim3(64 * kDprojWaves), 0, s, cp);
+        else hipLaunchKernelGGL(fp, grid, dim3(64 * kDprojWaves), 0, s, cp);
+      };
+      if (r_full <= 32) go(compress_bwd_dproj_kernel<bf16_t, 1>, compress_bwd_dproj_kernel<float, 1>);
+      else if (r_full <= 64) go(compress_bwd_dproj_kernel<bf16_t, 2>, compress_bwd_dproj_kernel<float, 2>);
+      else go(compress_bwd_dproj_kernel<bf16_t, 4>, compress_bwd_dproj_kernel<float, 4>);
       const int rc = wa_launch_status("compress_kv_bwd (dproj)");
       if (rc != WA_OK) return rc;
     } else {

@@ -91,12 +91,13 @@ def elu1_backward(q, k, v, dout, state, zsum, heads_t, dq, dk, dv, *, dq_accumul
 # ----------------------------------------------------------------------------------------------
 # low-rank compression (attention.py:64-110) under autograd
 # ----------------------------------------------------------------------------------------------
-def _compress_backward(grad, x, proj, segment_len, block_size, dx=None):
+def _compress_backward(grad, x, proj, segment_len, block_size, dx=None, out_dtype=torch.float32):
     """Gradients of ``out_seg = E[:r, :len] @ x_seg`` per segment (``wa_compress_kv_bwd``):
     ``dx_seg = E^T dout_seg`` and ``dE[:r, :len] = sum_{b, h} dout_seg x_seg^T``, fp32, for a
     ``[B, L, H, D]`` x and a ``[B, Lc, H, D]`` gradient. ``dx`` (optional): an fp32 ``[B, L, H, D]``
     tensor with unit last stride that the x gradient is added to; otherwise a new one is returned.
-    Returns ``(dx, dproj)``, dproj fp32 of the projection's shape."""
+    With ``out_dtype`` bf16 the (accumulated) x gradient comes back as a new bf16 tensor, rounded
+    once, and ``dx`` is only read. Returns ``(dx, dproj)``, dproj fp32 of the projection's shape."""
     dev = _lib.require_gpu(x, proj)
     bsz, length, heads, d = x.shape
     seg = segment_len if segment_len > 0 else length
@@ -106,8 +107,9 @@ def _compress_backward(grad, x, proj, segment_len, block_size, dx=None):
     pj = proj if proj.dtype in (torch.float32, torch.bfloat16) else proj.float()
     pj = pj.contiguous()
     accumulate = dx is not None
+    res = torch.empty((bsz, length, heads, d), dtype=torch.bfloat16, device=dev) if out_dtype == torch.bfloat16 else None
     if dx is None:
-        dx = torch.empty((bsz, length, heads, d), dtype=torch.float32, device=dev)
+        dx = torch.empty((bsz, length, heads, d), dtype=torch.float32, device=dev) if res is None else None
     elif dx.dtype != torch.float32 or tuple(dx.shape) != (bsz, length, heads, d) or dx.stride(-1) != 1:
         raise ValueError(f"dx must be float32 {(bsz, length, heads, d)} with unit last stride")
     dproj = torch.empty(pj.shape, dtype=torch.float32, device=dev)
@@ -115,9 +117,10 @@ def _compress_backward(grad, x, proj, segment_len, block_size, dx=None):
                      dtype=torch.uint8, device=dev)
     args = _lib.CompressBwdArgs(*_lib.blhd(g), *_lib.blhd(xs), _lib.dtype_code(xs), pj.data_ptr(),
                                 _lib.dtype_code(pj), pj.shape[0], pj.shape[1], bsz, length, heads, d, seg,
-                                block_size, *_lib.blhd(dx), int(accumulate), dproj.data_ptr(), 0, ws.data_ptr())
+                                block_size, *_blhd(dx), int(accumulate), dproj.data_ptr(), 0, ws.data_ptr(),
+                                *_blhd(res))
     _lib.call("wa_compress_kv_bwd", args, _lib.stream_ptr(dev))
-    return dx, dproj
+    return dx if res is None else res, dproj
 
 
 class _Compress(torch.autograd.Function):
@@ -131,7 +134,8 @@ class _Compress(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad):
         x, proj = ctx.saved_tensors
-        dx, dproj = _compress_backward(grad, x, proj, *ctx.cfg)
+        dx, dproj = _compress_backward(grad, x, proj, *ctx.cfg,
+                                       out_dtype=torch.bfloat16 if x.dtype == torch.bfloat16 else torch.float32)
         return dx.to(x.dtype), dproj.to(proj.dtype), None, None
 
 
@@ -274,40 +278,49 @@ class _HSA(torch.autograd.Function):
         # Split heads (each head in exactly one branch, elu1 linear heads): every gradient element
         # has one first writer (gate for dq of linear heads, the sparse backward for its heads,
         # elu1 for dk / dv of linear heads), which writes instead of adding, so the buffers need no
-        # zero fill. Otherwise they start at zero and every kernel accumulates.
-        fresh = (not plan.both and len(plan.sparse_only) + len(plan.linear_only) == heads
+        # zero fill. With the low-rank branch the gate is dq's first writer where every head is
+        # linear, and the sparse backward dk's and dv's where every head is sparse. Otherwise they
+        # start at zero and every kernel accumulates.
+        split = (not plan.both and len(plan.sparse_only) + len(plan.linear_only) == heads
                  and (not plan.linear or cfg["linear_mode"] == "elu1"))
-        alloc = torch.empty if fresh else torch.zeros
-        dq = alloc((bsz, q_len, heads, d), **f32)
-        # written once in their final type when that is bf16 (no fp32 buffer, no cast pass)
+        lowrank = bool(plan.linear) and cfg["linear_mode"] == "lowrank"
+        fresh_q = split or (lowrank and len(plan.linear) == heads)
+        fresh_kv = split or (lowrank and len(plan.sparse) == heads)
+        dq = (torch.empty if fresh_q else torch.zeros)((bsz, q_len, heads, d), **f32)
+        # dk / dv are written once in their final type when that is bf16 and no compression backward
+        # adds to them (no fp32 buffer, no cast pass)
         kd, vd = ctx.dtypes[1], ctx.dtypes[2]
-        kv_dt = torch.bfloat16 if fresh and kd == vd == torch.bfloat16 else torch.float32
+        inline = lowrank and not ctx.has_coarse
+        kv_dt = torch.bfloat16 if fresh_kv and not inline and kd == vd == torch.bfloat16 else torch.float32
+        alloc = torch.empty if fresh_kv else torch.zeros
         dk = alloc((bsz, kv_len, heads, d), dtype=kv_dt, device=dev)
         dv = alloc((bsz, kv_len, heads, d), dtype=kv_dt, device=dev)
         dgw = dgb = dkc = dvc = dEk = dEv = None
         if plan.linear:
             dlin = torch.empty((bsz, q_len, heads, d), **f32)
             dgw, dgb = fuse_backward(qb, lin, ex["modes_t"], gate, spec, dout, dlin, dq, lin_round=ex["lin_round"],
-                                     dq_accumulate=not fresh)
+                                     dq_accumulate=not fresh_q)
         if plan.sparse:
             bsa_backward(qb, kb, vb, sparse, lse_s, dout, index=index, num=num, block_size=block_size,
                          layout="blhd", heads=plan.t["sparse"], lq=q_len, lkv=kv_len, dq=dq, dk=dk, dv=dv,
-                         accumulate=not fresh, scale=cfg.get("scale", 0.0))
+                         accumulate=not split, kv_accumulate=not fresh_kv, scale=cfg.get("scale", 0.0))
         if plan.linear:
             lt = plan.t["linear"]
             if cfg["linear_mode"] == "elu1":
                 elu1_backward(q, k, v, dlin, state, zsum, lt, dq, dk, dv, dq_accumulate=True,
-                              kv_accumulate=not fresh)
+                              kv_accumulate=not fresh_kv)
             else:
                 lc = kcb.shape[1]
-                dkc = torch.zeros((bsz, lc, heads, d), **f32)
-                dvc = torch.zeros((bsz, lc, heads, d), **f32)
+                fresh_c = len(plan.linear) == heads
+                dkc = (torch.empty if fresh_c else torch.zeros)((bsz, lc, heads, d), **f32)
+                dvc = (torch.empty if fresh_c else torch.zeros)((bsz, lc, heads, d), **f32)
                 bsa_backward(qb, kcb, vcb, lin, lse_l, dlin, index=None, num=None, block_size=block_size,
                              layout="blhd", heads=lt, lq=q_len, lkv=lc, dq=dq, dk=dkc, dv=dvc, accumulate=True,
-                             scale=cfg.get("scale", 0.0))
-                if not ctx.has_coarse:
-                    _, dEk = _compress_backward(dkc, k, k_proj_mat, cfg["proj_segment_len"], block_size, dx=dk)
-                    _, dEv = _compress_backward(dvc, v, v_proj_mat, cfg["proj_segment_len"], block_size, dx=dv)
+                             kv_accumulate=not fresh_c, scale=cfg.get("scale", 0.0))
+                if inline:
+                    seg = cfg["proj_segment_len"]
+                    dk, dEk = _compress_backward(dkc, k, k_proj_mat, seg, block_size, dx=dk, out_dtype=kd)
+                    dv, dEv = _compress_backward(dvc, v, v_proj_mat, seg, block_size, dx=dv, out_dtype=vd)
         qd, kd, vd, kcd, vcd, ekd, evd, gwd, gbd = ctx.dtypes
 
         def cast(t, dt):

@@ -13,13 +13,15 @@ __all__ = ["bsa_backward"]
 
 
 def bsa_backward(q, k, v, out, lse, grad_out, *, index, num, block_size, block_sizes=None, layout="bhld",
-                 heads=None, lq=None, lkv=None, dq=None, dk=None, dv=None, accumulate=False, scale=0.0):
+                 heads=None, lq=None, lkv=None, dq=None, dk=None, dv=None, accumulate=False, scale=0.0,
+                 kv_accumulate=None):
     """``(dq, dk, dv)`` of :func:`bsa_forward` in ``layout`` (fp32; given ``dk`` / ``dv`` may be bf16).
 
     ``out`` is the forward's attention output (fp32 preferred, it sets ``delta``), ``lse`` its
     natural-log log-sum-exp ``[B, H, Lq]``; ``scale`` the forward's logit scale (0: ``D ** -0.5``).
     Given ``dq`` / ``dk`` / ``dv`` buffers are written, or
-    added to with ``accumulate`` (fp32 only); only the heads in ``heads`` (device int32) are touched.
+    added to with ``accumulate`` (fp32 only; ``kv_accumulate``: for ``dk`` / ``dv``, default as
+    ``accumulate``); only the heads in ``heads`` (device int32) are touched.
     """
     dev = _lib.require_gpu(q, k, v, out, grad_out)
     strides = _lib.bhld if layout == "bhld" else _lib.blhd
@@ -39,7 +41,8 @@ def bsa_backward(q, k, v, out, lse, grad_out, *, index, num, block_size, block_s
         dv = torch.zeros(v.shape, dtype=torch.float32, device=dev)
     if dk.dtype != dv.dtype or dk.dtype not in (torch.float32, torch.bfloat16) or dq.dtype != torch.float32:
         raise ValueError("dq must be fp32 and dk / dv both fp32 or both bf16")
-    if accumulate and dk.dtype != torch.float32:
+    kv_accumulate = accumulate if kv_accumulate is None else kv_accumulate
+    if kv_accumulate and dk.dtype != torch.float32:
         raise ValueError("bf16 dk / dv are written, not accumulated")
     grad_out = grad_out if grad_out.stride(-1) == 1 else grad_out.contiguous()
     n_slots = heads.numel() if heads is not None else nheads
@@ -55,7 +58,7 @@ def bsa_backward(q, k, v, out, lse, grad_out, *, index, num, block_size, block_s
         lse.data_ptr(), _lib.ptr(index), _lib.ptr(num), width, _lib.ptr(block_sizes),
         *_lib.heads_arg(heads),
         bsz, nheads, lq, lkv, d, block_size, float(scale),
-        *strides(dq), int(accumulate), *strides(dk), int(accumulate), *strides(dv), int(accumulate),
+        *strides(dq), int(accumulate), *strides(dk), int(kv_accumulate), *strides(dv), int(kv_accumulate),
         ws.data_ptr(), _lib.dtype_code(dk))
     _lib.call("wa_bsa_bwd", args, _lib.stream_ptr(dev))
     return dq, dk, dv
