@@ -55,6 +55,31 @@ def test_sparse_backward_matches_oracle_autograd(d, bs):
                      what=f"{name} d={d} bs={bs}")
 
 
+@pytest.mark.parametrize("d,bs,tail", [(64, 64, 1), (128, 64, 20), (128, 64, 45), (64, 128, 70), (128, 128, 127)])
+def test_sparse_backward_long_lists_in_block_order(d, bs, tail):
+    """Lists of more than 32 blocks are walked in block order unless a block occurs twice; the last
+    key block holds ``tail`` real keys (none of a wave's key half, or part of it)."""
+    torch.manual_seed(d + bs + tail)
+    b, h, nq, nkv = 1, 2, 3, 40
+    lkv = (nkv - 1) * bs + tail
+    q, k, v = (torch.randn(b, h, n * bs, d).bfloat16() for n in (nq, nkv, nkv))
+    k[:, :, lkv:] = 0
+    v[:, :, lkv:] = 0
+    index = torch.stack([torch.randperm(nkv) for _ in range(b * h * nq)]).view(b, h, nq, nkv).int()
+    num = torch.tensor([[33, 32, 40], [40, 37, 34]], dtype=torch.int32).view(b, h, nq)
+    index[0, 1, 0, 3] = index[0, 1, 0, 30]  # a duplicate keeps the list's order
+    index[0, 1, 1, 5] = nkv + 9             # clamped onto the last block
+    sizes = O.variable_block_sizes(lkv, nkv * bs, bs)
+    do = torch.randn(b, h, nq * bs, d)
+    qr, kr, vr = (t.double().requires_grad_() for t in (q, k, v))
+    O.block_sparse_attention(qr, kr, vr, index, num, sizes, bs).backward(do.double())
+    qg, kg, vg = (t.to(DEV).requires_grad_() for t in (q, k, v))
+    got = W.block_sparse_attention_reference(qg, kg, vg, index.to(DEV), num.to(DEV), sizes.to(DEV), bs)
+    got.float().backward(do.to(DEV))
+    for name, g, r in (("dq", qg.grad, qr.grad), ("dk", kg.grad, kr.grad), ("dv", vg.grad, vr.grad)):
+        assert_close(g[:, :, :lkv] if name != "dq" else g, r[:, :, :lkv] if name != "dq" else r, what=name)
+
+
 def test_sparse_backward_rectangular_lq_ne_lkv():
     """cfg-5-like rectangle (the Triton reference backward assumes Lq == Lkv)."""
     torch.manual_seed(5)

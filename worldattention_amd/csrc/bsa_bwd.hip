@@ -288,26 +288,38 @@ __device__ __forceinline__ void ring_wait(int ahead) {
   else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+// Lists of at most this many key blocks can be put in block order through a bitmap.
+constexpr int DQ_SORT_BLOCKS = 2048;
+
 // ---------------------------------------------------------------------------------------------
-// dq: one workgroup (BS / 32 waves, wave w = query rows 32w..) per (batch, head slot, query
-// block); 64-key steps over the row's list, K and V streamed through the ring.
+// dq: one workgroup per (batch, head slot, query block); 64-key steps over the row's list, K and V
+// streamed through the ring. KS = 1 (128-query blocks): four waves, wave w = query rows 32w... KS = 2
+// (64-query blocks): four waves as well, the two of a 32-query tile taking the 32-key halves of every
+// step and adding their dQ through LDS after the last one; the ring allows two workgroups per CU, so
+// with one wave per tile each SIMD had a single wave and nothing to run under its waits. A list
+// without duplicates is walked in block order (whatever the routing order): the rows an XCD runs at
+// a time then sweep a head's keys together and share them in L2. H 12, D 128, Lq 4680, Lkv 32,760,
+// ~180 blocks a row: 698 us with two waves in list order, 575 us here. A list of
+// at most 32 blocks keeps its order: the sort's two barriers cost more than it saves (8 heads of 16
+// 128-key blocks: 96 us unsorted, 104-113 us sorted).
 // ---------------------------------------------------------------------------------------------
 template <int D, int BS>
-__global__ void __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))) bwd_dq_kernel(BwdParams p) {
-  constexpr int NW = BS / 32, DC = D / 16, DT = D / 32;
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) bwd_dq_kernel(BwdParams p) {
+  constexpr int KS = BS == 64 ? 2 : 1, NQW = BS / 32, NW = NQW * KS, DC = D / 16, DT = D / 32;
+  constexpr int KT = 2 / KS;                       // 32-key tiles of a step per wave
   constexpr int TILE = 64 * D, ST = DQ_STAGES, LM = DQ_LIST_MAX;
   using TS = TileStream<D, NW>;
   constexpr int PER = 2 * TS::NI;                  // loads per wave per step: K and V
   constexpr int HPV = BS / 64;                     // 64-key steps per visited block
-  constexpr int XS = ST == 4 ? 2 * TILE : 8;      // stages 2 and 3 exist only in 4-stage rings
+  static_assert(ST == 2 && NW == 4, "two ring stages, four waves");
   // stage s: K tile at [0, TILE), V tile at [TILE, 2 TILE)
   __shared__ __attribute__((aligned(1024))) bf16_t kv0[2 * TILE];
   __shared__ __attribute__((aligned(1024))) bf16_t kv1[2 * TILE];
-  __shared__ __attribute__((aligned(1024))) bf16_t kv2[XS];
-  __shared__ __attribute__((aligned(1024))) bf16_t kv3[XS];
   __shared__ int32_t s_lst[LM];  // visited block | (its valid key count << 16)
+  __shared__ uint32_t s_bits[DQ_SORT_BLOCKS / 32];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, l32 = lane & 31;
+  const int qw = w % NQW, kh = w / NQW;  // 32-query tile; key half (KS = 2)
   // 1-D grid over (batch, head slot, query block), taken XCD by XCD (wa_xcd_remap): an XCD runs
   // a contiguous run of whole slabs, so the query blocks of a head share its K / V tiles in one L2
   const int pos = wa_xcd_remap((int)blockIdx.x, (int)gridDim.x);
@@ -316,16 +328,13 @@ __global__ void __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))
   if (h < 0 || h >= p.H) return;
   const int64_t irow = ((int64_t)b * p.H + h) * p.Nq + qb;
   const int n = row_visits(p, irow);
-  const int qi = qb * BS + w * 32 + l32;
+  const int qi = qb * BS + qw * 32 + l32;
   const bool q_ok = qi < p.Lq;
   const int64_t srow = ((int64_t)b * p.n_heads + hs) * p.Lq;
 
   const int32_t* lst = p.index ? p.index + irow * p.index_width : nullptr;
-  auto visit = [&](int s2) {
-    const int j = lst ? min(max(lst[s2], 0), p.Nkv - 1) : s2;
-    return j | (kv_real(p, j, BS) << 16);
-  };
-  for (int i = tid; i < min(n, LM); i += 2 * BS) s_lst[i] = visit(i);
+  auto block_at = [&](int s2) { return lst ? min(max(lst[s2], 0), p.Nkv - 1) : s2; };
+  auto packed = [&](int j) { return j | (kv_real(p, j, BS) << 16); };
   bf16x8 qf[DC], dof[DC];
   {
     const bf16_t* qr = p.q + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + (int64_t)(q_ok ? qi : 0) * p.q_st;
@@ -341,6 +350,31 @@ __global__ void __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))
   // a query past Lq or without a log-sum-exp gets lse2 = +inf: zero probabilities, zero gradient
   float lse2 = q_ok ? p.lse2[srow + qi] : INFINITY;
   float dl = q_ok ? p.delta[srow + qi] : 0.f;
+  bool in_order = false;
+  if (lst && n > 32 && n <= LM && p.Nkv <= DQ_SORT_BLOCKS) {  // uniform over the workgroup
+    if (tid < DQ_SORT_BLOCKS / 32) s_bits[tid] = 0;
+    __syncthreads();
+    for (int i = tid; i < n; i += 256) {
+      const int j = block_at(i);
+      atomicOr(&s_bits[j >> 5], 1u << (j & 31));
+    }
+    __syncthreads();
+    uint32_t word = s_bits[lane];
+    const int cnt = __popc(word);
+    int incl = cnt;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int up = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += up;
+    }
+    in_order = __builtin_amdgcn_readlane(incl, 63) == n;  // no block listed twice
+    if (in_order && w == 0) {
+      for (int r = incl - cnt; word; ++r, word &= word - 1) s_lst[r] = packed(lane * 32 + __ffs(word) - 1);
+    }
+  }
+  if (!in_order) {
+    for (int i = tid; i < min(n, LM); i += 256) s_lst[i] = packed(block_at(i));
+  }
   // materialize the fragments before the ring's loads are issued: a use after the prologue would
   // otherwise wait for every load in flight
 #pragma unroll
@@ -360,12 +394,12 @@ __global__ void __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))
   // (an empty half streams rows from key 0: never read, keeps the load count uniform)
   auto step_at = [&](int t, int& real) -> int {
     const int s2 = t / HPV, hf = t % HPV;
-    const int e = __builtin_amdgcn_readfirstlane(s2 < LM ? s_lst[s2] : visit(s2));
+    const int e = __builtin_amdgcn_readfirstlane(s2 < LM ? s_lst[s2] : packed(block_at(s2)));
     real = (e >> 16) - 64 * hf;
     return real > 0 ? (e & 0xFFFF) * BS + 64 * hf : 0;
   };
   auto issue = [&](auto S, int t) {
-    bf16_t* kv = stage_of<decltype(S)::value>(kv0, kv1, kv2, kv3);
+    bf16_t* kv = decltype(S)::value ? kv1 : kv0;
     int real;
     const int r0 = step_at(t, real);
     ks.issue(kv, r0, w);
@@ -379,35 +413,36 @@ __global__ void __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))
     int real;
     step_at(t, real);
     if (real <= 0) return;  // uniform: an empty half contributes nothing
-    const bf16_t* kc = stage_of<SV>(kv0, kv1, kv2, kv3);
+    const bf16_t* kc = SV ? kv1 : kv0;
     const bf16_t* vc = kc + TILE;
+    const int key0 = KS == 2 ? 32 * kh : 0;  // this wave's first key of the step
     // S^T = K Q^T and dP^T = V dO^T (A from LDS, B from registers)
-    f32x16 sacc[2], pacc[2];
+    f32x16 sacc[KT], pacc[KT];
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) sacc[kt] = pacc[kt] = f32x16{};
+    for (int kt = 0; kt < KT; ++kt) sacc[kt] = pacc[kt] = f32x16{};
 #pragma unroll
     for (int c = 0; c < DC; ++c) {
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-        sacc[kt] = wa_mfma32(tile_row8<D>(kc, kt * 32 + l32, 2 * c + g), qf[c], sacc[kt]);
-        pacc[kt] = wa_mfma32(tile_row8<D>(vc, kt * 32 + l32, 2 * c + g), dof[c], pacc[kt]);
+      for (int kt = 0; kt < KT; ++kt) {
+        sacc[kt] = wa_mfma32(tile_row8<D>(kc, key0 + kt * 32 + l32, 2 * c + g), qf[c], sacc[kt]);
+        pacc[kt] = wa_mfma32(tile_row8<D>(vc, key0 + kt * 32 + l32, 2 * c + g), dof[c], pacc[kt]);
       }
     }
     // keys past a partial block's end (their tile rows hold other keys) get zero probability
     if (real < 64) {
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
+      for (int kt = 0; kt < KT; ++kt) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const int key = kt * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
+          const int key = key0 + kt * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
           if (key >= real) sacc[kt][r] = -INFINITY;
         }
       }
     }
     // dS^T = P^T (dP^T - delta), packed in accumulator order for the next product
-    bf16x8 dsb[4];
+    bf16x8 dsb[2 * KT];
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
+    for (int kt = 0; kt < KT; ++kt) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const float pr = __builtin_amdgcn_exp2f(fmaf(sacc[kt][r], p.scale_log2, -lse2));
@@ -416,26 +451,38 @@ __global__ void __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))
     }
     // dQ[q, d] += dS[q, key] K[key, d]: A = dS (registers), B = K (transpose reads)
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
+    for (int c = 0; c < 2 * KT; ++c) {
 #pragma unroll
-      for (int tt = 0; tt < DT; ++tt) dqacc[tt] = wa_mfma32(dsb[c], tile_tr8<D>(kc, c, 32 * tt, lane), dqacc[tt]);
+      for (int tt = 0; tt < DT; ++tt)
+        dqacc[tt] = wa_mfma32(dsb[c], tile_tr8<D>(kc + key0 * D, c, 32 * tt, lane), dqacc[tt]);
     }
   };
-  // prologue: tiles 0 .. ST - 2
   if (total > 0) issue(IC<0>{}, 0);
-  if constexpr (ST == 4) {
-    if (total > 1) issue(IC<1>{}, 1);
-    if (total > 2) issue(IC<2>{}, 2);
-  }
   for (int t = 0; t < total; t += ST) {
     step(IC<0>{}, t);
     if (t + 1 < total) step(IC<1>{}, t + 1);
-    if constexpr (ST == 4) {
-      if (t + 2 < total) step(IC<2>{}, t + 2);
-      if (t + 3 < total) step(IC<3>{}, t + 3);
+  }
+  if constexpr (KS == 2) {
+    // the key halves' sums meet in the drained ring
+    static_assert(NQW * DT * 16 * 64 * 4 <= 2 * TILE * 2, "the exchange does not fit a stage");
+    float* xo = (float*)kv0 + qw * DT * 16 * 64 + lane;
+    __syncthreads();  // every wave is done with the last step's tiles
+    if (kh == 1) {
+#pragma unroll
+      for (int tt = 0; tt < DT; ++tt) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) xo[(tt * 16 + r) * 64] = dqacc[tt][r];
+      }
+    }
+    __syncthreads();
+    if (kh == 1) return;
+#pragma unroll
+    for (int tt = 0; tt < DT; ++tt) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) dqacc[tt][r] += xo[(tt * 16 + r) * 64];
     }
   }
-  // accumulator lane (d = 32t + l32, g) holds rows q = 32w + 8(r/4) + 4g + r%4. With accumulation
+  // accumulator lane (d = 32t + l32, g) holds rows q = 32qw + 8(r/4) + 4g + r%4. With accumulation
   // every previous value of a tile is read before any store, so the reads overlap (a store may
   // alias a later read, which would otherwise serialize each read-add-write round trip).
   const int64_t dq_off = (int64_t)b * p.dq_sb + (int64_t)h * p.dq_sh + l32;
@@ -445,7 +492,7 @@ __global__ void __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))
     for (int tt = 0; tt < DT; ++tt) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int q = qb * BS + w * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
+        const int q = qb * BS + qw * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
         if (q < p.Lq) dq_out[(int64_t)q * p.dq_st + 32 * tt] = (bf16_t)(dqacc[tt][r] * p.scale);
       }
     }
@@ -457,12 +504,12 @@ __global__ void __launch_bounds__(2 * BS) __attribute__((amdgpu_waves_per_eu(2))
     float prev[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int q = qb * BS + w * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
+      const int q = qb * BS + qw * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
       prev[r] = p.dq_acc && q < p.Lq ? dq_col[(int64_t)q * p.dq_st + 32 * tt] : 0.f;
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int q = qb * BS + w * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
+      const int q = qb * BS + qw * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
       if (q < p.Lq) dq_col[(int64_t)q * p.dq_st + 32 * tt] = prev[r] + dqacc[tt][r] * p.scale;
     }
   }
@@ -837,7 +884,7 @@ int launch_bwd(const BwdParams& bp, hipStream_t s, hipStream_t sq, hipEvent_t fo
     hipError_t e;
     if ((e = hipEventRecord(fork, s)) != hipSuccess || (e = hipStreamWaitEvent(sq, fork, 0)) != hipSuccess)
       return wa_fail((int)e, "wa_bsa_bwd: fork: %s", hipGetErrorString(e));
-    hipLaunchKernelGGL((bwd_dq_kernel<D, BS>), dim3((unsigned)(bp.Nq * nh * bp.B)), dim3(2 * BS), 0, sq, bp);
+    hipLaunchKernelGGL((bwd_dq_kernel<D, BS>), dim3((unsigned)(bp.Nq * nh * bp.B)), dim3(256), 0, sq, bp);
     rc = wa_launch_status("bsa_bwd_dq");
     if ((e = hipEventRecord(join, sq)) != hipSuccess) return rc ? rc : wa_fail((int)e, "wa_bsa_bwd: join: %s", hipGetErrorString(e));
     if (rc) {
@@ -857,7 +904,7 @@ int launch_bwd(const BwdParams& bp, hipStream_t s, hipStream_t sq, hipEvent_t fo
     hipLaunchKernelGGL(k2q_kernel, dim3((bp.Nkv + 255) / 256, nh, bp.B), dim3(256), 0, s, bp);
   if ((rc = wa_launch_status("bsa_bwd_k2q"))) return joined(rc);
   if (bp.dq && !split) {
-    hipLaunchKernelGGL((bwd_dq_kernel<D, BS>), dim3((unsigned)(bp.Nq * nh * bp.B)), dim3(2 * BS), 0, s, bp);
+    hipLaunchKernelGGL((bwd_dq_kernel<D, BS>), dim3((unsigned)(bp.Nq * nh * bp.B)), dim3(256), 0, s, bp);
     if ((rc = wa_launch_status("bsa_bwd_dq"))) return rc;
   }
   if (bp.dk && bp.dv) {
