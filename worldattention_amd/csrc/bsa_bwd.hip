@@ -159,14 +159,19 @@ __global__ void __launch_bounds__(256) bwd_pre_kernel(BwdParams p) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// k2q by counting: one workgroup per (64 key blocks, head slot, batch). Every list entry of the
-// head that falls in the workgroup's key range adds 1 to cnt[key block][query block] in LDS; then
-// thread j walks row j in query order and writes the non-zero counts. For Nq <= K2Q_COUNT_NQ.
+// k2q by counting: one workgroup of 16 waves per (32 key blocks, head slot, batch). Wave w reads the
+// lists of rows w, w + 16, ... (64 entries a load, four loads in flight); every entry in the
+// workgroup's key range adds 1 to cnt[key block][query block] in LDS; then each wave emits the
+// non-zero counts of two key blocks in query order, a 64-query ballot at a time. For
+// Nq <= K2Q_COUNT_NQ. Latency-bound: each workgroup reads its head's lists whole, so what counts is
+// loads in flight. 12 heads of 74 rows x ~180 of 512 blocks: 40 us with 4 waves per 64 key blocks and
+// one thread emitting a block, 11 us here.
 // ---------------------------------------------------------------------------------------------
-constexpr int K2Q_COUNT_KB = 64;
+constexpr int K2Q_COUNT_KB = 32;
 constexpr int K2Q_COUNT_NQ = 256;
+constexpr int K2Q_WAVES = 16;
 
-__global__ void __launch_bounds__(256) k2q_count_kernel(BwdParams p) {
+__global__ void __launch_bounds__(64 * K2Q_WAVES) k2q_count_kernel(BwdParams p) {
   __shared__ uint32_t cnt[K2Q_COUNT_KB * K2Q_COUNT_NQ];
   __shared__ int32_t s_num[K2Q_COUNT_NQ];
   const int hs = blockIdx.y, b = blockIdx.z, j0 = blockIdx.x * K2Q_COUNT_KB;
@@ -174,45 +179,42 @@ __global__ void __launch_bounds__(256) k2q_count_kernel(BwdParams p) {
   if (h < 0 || h >= p.H) return;
   const int64_t row0 = ((int64_t)b * p.H + h) * p.Nq;
   const int width = (int)p.index_width, nq = p.Nq;
-  __shared__ int s_maxn;
-  if (threadIdx.x == 0) s_maxn = 0;
-  for (int u = threadIdx.x; u < K2Q_COUNT_KB * nq; u += 256) cnt[u] = 0;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  for (int u = tid; u < K2Q_COUNT_KB * nq; u += 64 * K2Q_WAVES) cnt[u] = 0;
+  if (tid < nq) s_num[tid] = row_visits(p, row0 + tid);
   __syncthreads();
-  for (int i = threadIdx.x; i < nq; i += 256) {
-    const int n = row_visits(p, row0 + i);
-    s_num[i] = n;
-    atomicMax(&s_maxn, n);
-  }
-  __syncthreads();
-  // only the listed entries: (row, slot < the longest row's count), four loads in flight per thread
-  const int maxn = s_maxn, total = nq * maxn;
-  for (int u0 = threadIdx.x; u0 < total; u0 += 4 * 256) {
-    int jj[4], ii[4];
-    bool on[4];
+  for (int i = w; i < nq; i += K2Q_WAVES) {
+    const int n = __builtin_amdgcn_readfirstlane(s_num[i]);
+    const int32_t* lst = p.index + (row0 + i) * width;
+    for (int s0 = 0; s0 < n; s0 += 4 * 64) {
+      int jj[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int u = u0 + k * 256;
-      ii[k] = u / maxn;  // maxn > 0 whenever the loop runs
-      on[k] = u < total && u - ii[k] * maxn < s_num[min(ii[k], nq - 1)];
-      jj[k] = on[k] ? p.index[(row0 + ii[k]) * width + (u - ii[k] * maxn)] : 0;
-    }
+      for (int k = 0; k < 4; ++k) {
+        const int s = s0 + 64 * k + lane;
+        jj[k] = s < n ? min(max(lst[s], 0), p.Nkv - 1) : -1;
+      }
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int j = min(max(jj[k], 0), p.Nkv - 1) - j0;
-      if (on[k] && j >= 0 && j < K2Q_COUNT_KB) atomicAdd(&cnt[j * nq + ii[k]], 1u);
+      for (int k = 0; k < 4; ++k) {
+        const int j = jj[k] - j0;
+        if (jj[k] >= 0 && j >= 0 && j < K2Q_COUNT_KB) atomicAdd(&cnt[j * nq + i], 1u);
+      }
     }
   }
   __syncthreads();
-  const int j = j0 + (int)threadIdx.x;
-  if (threadIdx.x >= K2Q_COUNT_KB || j >= p.Nkv) return;
-  int32_t* out = p.k2q + (((int64_t)b * p.n_heads + hs) * p.Nkv + j) * p.Nq;
-  const uint32_t* c = cnt + threadIdx.x * nq;
-  int n = 0;
-  for (int i = 0; i < nq; ++i) {
-    const int m = (int)c[i];
-    if (m > 0) out[n++] = i | (min(m, 32767) << 16);
+  for (int jl = w; jl < K2Q_COUNT_KB; jl += K2Q_WAVES) {
+    const int j = j0 + jl;
+    if (j >= p.Nkv) break;
+    int32_t* out = p.k2q + (((int64_t)b * p.n_heads + hs) * p.Nkv + j) * p.Nq;
+    int n = 0;
+    for (int i0 = 0; i0 < nq; i0 += 64) {
+      const int i = i0 + lane;
+      const int m = i < nq ? (int)cnt[jl * nq + i] : 0;
+      const uint64_t some = __ballot(m > 0);
+      if (m > 0) out[n + __popcll(some & ((1ull << lane) - 1))] = i | (min(m, 32767) << 16);
+      n += __popcll(some);
+    }
+    if (lane == 0) p.k2q_num[((int64_t)b * p.n_heads + hs) * p.Nkv + j] = n;
   }
-  p.k2q_num[((int64_t)b * p.n_heads + hs) * p.Nkv + j] = n;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -898,8 +900,8 @@ int launch_bwd(const BwdParams& bp, hipStream_t s, hipStream_t sq, hipEvent_t fo
     return code != WA_OK ? code : e != hipSuccess ? wa_fail((int)e, "wa_bsa_bwd: join: %s", hipGetErrorString(e)) : WA_OK;
   };
   if (bp.index && bp.Nq <= K2Q_COUNT_NQ)
-    hipLaunchKernelGGL(k2q_count_kernel, dim3((bp.Nkv + K2Q_COUNT_KB - 1) / K2Q_COUNT_KB, nh, bp.B), dim3(256), 0, s,
-                       bp);
+    hipLaunchKernelGGL(k2q_count_kernel, dim3((bp.Nkv + K2Q_COUNT_KB - 1) / K2Q_COUNT_KB, nh, bp.B),
+                       dim3(64 * K2Q_WAVES), 0, s, bp);
   else
     hipLaunchKernelGGL(k2q_kernel, dim3((bp.Nkv + 255) / 256, nh, bp.B), dim3(256), 0, s, bp);
   if ((rc = wa_launch_status("bsa_bwd_k2q"))) return joined(rc);
