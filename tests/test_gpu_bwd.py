@@ -99,6 +99,32 @@ def test_sparse_backward_rectangular_lq_ne_lkv():
         assert_close(g, r, what=name)
 
 
+@pytest.mark.parametrize("nq,nkv", [(65, 31), (130, 33), (256, 32)])
+def test_sparse_backward_transposed_lists_by_counting(nq, nkv):
+    """Transposed lists from the counting kernel at the edges of its 64-query and 32-key-block runs,
+    with duplicates, empty rows and rows of up to all key blocks; gradients keep bf16 inputs' type."""
+    torch.manual_seed(nq)
+    b, h, d, bs = 1, 2, 64, 64
+    q, k, v = (torch.randn(b, h, n * bs, d).bfloat16() for n in (nq, nkv, nkv))
+    index = torch.stack([torch.randperm(nkv) for _ in range(b * h * nq)]).view(b, h, nq, nkv).int()
+    num = torch.randint(0, 4, (b, h, nq), dtype=torch.int32)
+    num[0, 0, nq - 1], num[0, 1, 0] = nkv, 0
+    index[0, 1, 1, :2] = nkv - 1
+    num[0, 1, 1] = 2
+    sizes = torch.full((nkv,), bs, dtype=torch.int32)
+    do = torch.randn(b, h, nq * bs, d)
+    qr, kr, vr = (t.float().requires_grad_() for t in (q, k, v))
+    O.block_sparse_attention_gather(qr, kr, vr, index, num, sizes, bs).backward(do)
+    qg, kg, vg = (t.to(DEV).requires_grad_() for t in (q, k, v))
+    got = W.block_sparse_attention_reference(qg, kg, vg, index.to(DEV), num.to(DEV), sizes.to(DEV), bs)
+    got.backward(do.to(DEV).bfloat16())
+    for name, g, r in (("dq", qg.grad, qr.grad), ("dk", kg.grad, kr.grad), ("dv", vg.grad, vr.grad)):
+        # dO is rounded to bf16 on the GPU side (2^-9), gradients of up to ~|r| are stored in bf16
+        assert g.dtype == torch.bfloat16
+        scale = max(1.0, r.abs().max().item())
+        assert_close(g, r, 2e-2 * scale, 2e-3 * scale, what=name)
+
+
 def test_sparse_backward_many_query_blocks():
     """More than 256 query blocks: the transposed lists come from the scanning kernel instead of the
     counting one."""

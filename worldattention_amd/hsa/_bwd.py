@@ -15,7 +15,7 @@ __all__ = ["bsa_backward"]
 def bsa_backward(q, k, v, out, lse, grad_out, *, index, num, block_size, block_sizes=None, layout="bhld",
                  heads=None, lq=None, lkv=None, dq=None, dk=None, dv=None, accumulate=False, scale=0.0,
                  kv_accumulate=None):
-    """``(dq, dk, dv)`` of :func:`bsa_forward` in ``layout`` (fp32; given ``dk`` / ``dv`` may be bf16).
+    """``(dq, dk, dv)`` of :func:`bsa_forward` in ``layout`` (fp32; given buffers may be bf16).
 
     ``out`` is the forward's attention output (fp32 preferred, it sets ``delta``), ``lse`` its
     natural-log log-sum-exp ``[B, H, Lq]``; ``scale`` the forward's logit scale (0: ``D ** -0.5``).
@@ -39,8 +39,10 @@ def bsa_backward(q, k, v, out, lse, grad_out, *, index, num, block_size, block_s
         dk = torch.zeros(k.shape, dtype=torch.float32, device=dev)
     if dv is None:
         dv = torch.zeros(v.shape, dtype=torch.float32, device=dev)
-    if dk.dtype != dv.dtype or dk.dtype not in (torch.float32, torch.bfloat16) or dq.dtype != torch.float32:
-        raise ValueError("dq must be fp32 and dk / dv both fp32 or both bf16")
+    if dk.dtype != dv.dtype or any(t.dtype not in (torch.float32, torch.bfloat16) for t in (dq, dk)):
+        raise ValueError("dq must be fp32 or bf16 and dk / dv both fp32 or both bf16")
+    if accumulate and dq.dtype != torch.float32:
+        raise ValueError("a bf16 dq is written, not accumulated")
     kv_accumulate = accumulate if kv_accumulate is None else kv_accumulate
     if kv_accumulate and dk.dtype != torch.float32:
         raise ValueError("bf16 dk / dv are written, not accumulated")
@@ -59,6 +61,6 @@ def bsa_backward(q, k, v, out, lse, grad_out, *, index, num, block_size, block_s
         *_lib.heads_arg(heads),
         bsz, nheads, lq, lkv, d, block_size, float(scale),
         *strides(dq), int(accumulate), *strides(dk), int(kv_accumulate), *strides(dv), int(kv_accumulate),
-        ws.data_ptr(), _lib.dtype_code(dk))
+        ws.data_ptr(), _lib.dtype_code(dk), _lib.dtype_code(dq))
     _lib.call("wa_bsa_bwd", args, _lib.stream_ptr(dev))
     return dq, dk, dv

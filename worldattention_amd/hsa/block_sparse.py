@@ -201,9 +201,14 @@ class _BlockSparseAttention(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_out):
         qb, kb, vb, out, lse, index, num, block_sizes = ctx.saved_tensors
-        dq, dk, dv = bsa_backward(qb, kb, vb, out, lse, grad_out, index=index, num=num,
-                                  block_size=ctx.block_size, block_sizes=block_sizes, scale=ctx.scale)
         qd, kd, vd = ctx.dtypes
+        # every element is written once by the kernels, in its final type when that is bf16 (rounded
+        # there instead of by a zero fill, an fp32 buffer and a cast pass each)
+        dq = torch.empty(qb.shape, dtype=torch.bfloat16 if qd == torch.bfloat16 else torch.float32, device=qb.device)
+        dk, dv = (torch.empty(kb.shape, dtype=torch.bfloat16 if kd == vd == torch.bfloat16 else torch.float32,
+                              device=qb.device) for _ in range(2))
+        bsa_backward(qb, kb, vb, out, lse, grad_out, index=index, num=num, block_size=ctx.block_size,
+                     block_sizes=block_sizes, scale=ctx.scale, dq=dq, dk=dk, dv=dv)
         return dq.to(qd), dk.to(kd), dv.to(vd), None, None, None, None, None
 
 
