@@ -546,7 +546,10 @@ int wa_hsa_fuse_bwd(const wa_hsa_fuse_args* args, void* stream);
  * With `factors` (device complex64 as float pairs, [n_rows][n_temporal]), y is x with complex pair
  * p < n_temporal of every head multiplied by factors[min(t / row_tokens, n_rows - 1)][p] in fp32
  * and rounded to x's dtype (the reference de-ropes into the cache dtype, then pools in fp32);
- * without `factors`, y = x. With `normalize`, each out row becomes row / max(|row|_2, 1e-12).
+ * without `factors`, y = x. Instead of `factors`, `freqs64` (device complex128 RoPE table as double
+ * pairs, 16-byte aligned, freqs_rows rows of freqs_stride pairs) gives row r of the table the factor
+ * freqs64[0] conj(freqs64[start_row + r]) (rows clamped to the table), formed in fp64 and narrowed to
+ * fp32: what the caller would otherwise compute as `factors`. With `normalize`, each out row becomes row / max(|row|_2, 1e-12).
  * Replaces page_key_index + derope_temporal (pipeline/hkv/retrieval.py:50-72, rope.py:70-82),
  * query_index (retrieval.py:41-47) and prompt_index (retrieval.py:32-38, normalize = 1).
  * Workspace: wa_hkv_summary_workspace_bytes(B, n_seg, C, max_seg_tokens). */
@@ -558,11 +561,12 @@ typedef struct wa_hkv_summary_args {
   int32_t normalize;
   float* out;
   void* workspace;
+  const double* freqs64; int64_t freqs_stride, freqs_rows, start_row;
 } wa_hkv_summary_args;
 int64_t wa_hkv_summary_workspace_bytes(int64_t B, int64_t n_seg, int64_t C, int64_t max_seg_tokens);
 int wa_hkv_page_summary(const wa_hkv_summary_args* args, void* stream);
 
-/* Page scoring and selection in one workgroup:
+/* Page scoring and selection (with `scores`, more than 32 pages are scored by a launch of their own):
  *   scores[p] = (index[p] . query) / scale   (no division when scale <= 0), p < n_pages <= 4096,
  * then the k highest in descending order, the lower page index first among equal scores (NaN
  * ranks highest), into sel (int32) and sel_scores. Pages with mask[p] != 0 (device uint8,

@@ -103,6 +103,48 @@ def test_query_and_prompt_index_match_oracle(dim):
 # ---------------------------------------------------------------------------------------------
 # scoring and selection
 # ---------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("b,frames,fsl,page,start,c0", [(1, 5, 33, 2, 0, 0), (2, 3, 100, 1, 7, 0), (1, 9, 16, 4, -3, 0),
+                                                        (1, 2, 40, 1, 60, 0), (1, 3, 20, 1, 2, 1)])
+def test_page_key_index_forms_its_factors_from_the_table(b, frames, fsl, page, start, c0):
+    """De-rope factors formed in the summary kernel from the fp64 table (whose row 0 need not be 1,
+    positions past either end clamped, leading or shifted columns of a wider table) against the torch
+    factor table: the same factors, so the same bits; few segments take the finer token splits."""
+    torch.manual_seed(fsl)
+    h, d = 3, 32
+    nt = 16 - 2 * (16 // 3)
+    ang = torch.rand(64, nt + 5, dtype=torch.float64) * 6
+    table = torch.polar(torch.rand(64, nt + 5, dtype=torch.float64) + 0.5, ang).to(DEV)[:, c0:c0 + nt]
+    keys = torch.randn(b, frames * fsl, h, d, device=DEV).bfloat16()
+    spans = [(t, min(t + page * fsl, frames * fsl)) for t in range(0, frames * fsl, page * fsl)]
+    kw = dict(frame_seq_length=fsl, start_frame=start)
+    assert _ops.derope_in_place(table, keys.device) and not _ops.derope_in_place(table.cpu(), keys.device)
+    got = W.page_key_index(keys, spans, temporal_freqs=table, **kw)
+    want = W.page_key_index(keys, spans, temporal_freqs=table.cpu(), **kw)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("tokens,dim", [(31, 64), (33, 2048), (4680, 1536), (9000, 4096)])
+def test_single_segment_means_over_fine_splits(tokens, dim):
+    """One mean over up to 128 token splits: fp32 sums of n values in any order (n 2^-24 sum |x| / n)."""
+    torch.manual_seed(tokens)
+    x = torch.randn(2, tokens, dim, device=DEV).bfloat16()
+    got = W.query_index(x)
+    want = x.double().mean(dim=(0, 1))
+    assert ((got.double() - want).abs() <= tokens * 2.0 ** -24 * x.double().abs().mean(dim=(0, 1))).all()
+
+
+@pytest.mark.parametrize("n_pages", [32, 33, 500])
+def test_scores_alone_and_with_the_selection_are_the_same_bits(n_pages):
+    """Up to 32 pages are scored by the selecting workgroup, more by a launch of their own."""
+    torch.manual_seed(n_pages)
+    index, query = torch.randn(n_pages, 1000, device=DEV), torch.randn(1000, device=DEV)
+    scores = W.score_pages(query, index)
+    alone = torch.cat([W.score_pages(query, index[i:i + 1]) for i in range(n_pages)])
+    assert torch.equal(scores, alone)
+    sel, top = W.select_pages(index, query, 5)
+    assert torch.equal(top, torch.topk(scores, 5).values) and torch.equal(scores[sel.long()], top)
+
+
 @pytest.mark.parametrize("pages,dim,k", [(120, 1536, 8), (1, 64, 1), (4096, 256, 33), (777, 100, 777)])
 def test_score_topk_matches_oracle(pages, dim, k):
     torch.manual_seed(pages)

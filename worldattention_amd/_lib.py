@@ -274,6 +274,7 @@ HkvSummaryArgs = _struct("wa_hkv_summary_args", [
     ("normalize", c_int32),
     ("out", c_void_p),
     ("workspace", c_void_p),
+    ("freqs64", c_void_p), ("freqs_stride", c_int64), ("freqs_rows", c_int64), ("start_row", c_int64),
 ])
 
 HKV_MAX_PAGES = 4096

@@ -81,13 +81,20 @@ __device__ __forceinline__ void rotate_band(float (&f)[VEC], int d0, const float
 // reduction per segment. One thread owns VEC consecutive channels of one head.
 // =============================================================================================
 // 256 tokens per split: one round of workgroups at the cfg 3 shape (120 pages x 7 splits); 64 made
-// 3,000 workgroups of which the last ~440 ran a second, nearly empty round (125 -> 116 us).
-constexpr int SUM_TOKENS_PER_SPLIT = 256;
-constexpr int SUM_MAX_SPLITS = 64;
+// 3,000 workgroups of which the last ~440 ran a second, nearly empty round (125 -> 116 us). Few
+// segments (a query or prompt mean, short histories) are cut finer, down to 32 tokens and up to 128
+// splits, until about two workgroups per CU run: one 4,680-token mean 32 us with 19 workgroups,
+// 8 us with 128.
+constexpr int SUM_TOKENS_PER_SPLIT = 256, SUM_FEWEST_TOKENS = 32;
+constexpr int SUM_MAX_SPLITS = 64, SUM_MAX_FINE_SPLITS = 128;
 
-int64_t summary_splits(int64_t max_seg_tokens) {
-  const int64_t s = (std::max<int64_t>(max_seg_tokens, 1) + SUM_TOKENS_PER_SPLIT - 1) / SUM_TOKENS_PER_SPLIT;
-  return std::min<int64_t>(s, SUM_MAX_SPLITS);
+int64_t summary_splits(int64_t B, int64_t n_seg, int64_t C, int64_t max_seg_tokens) {
+  const int64_t tokens = std::max<int64_t>(max_seg_tokens, 1);
+  const int64_t s = std::min<int64_t>((tokens + SUM_TOKENS_PER_SPLIT - 1) / SUM_TOKENS_PER_SPLIT, SUM_MAX_SPLITS);
+  const int64_t per_split = B * n_seg * ((C + 2047) / 2048);  // workgroups
+  const int64_t fine = std::min({(512 + per_split - 1) / per_split, (tokens + SUM_FEWEST_TOKENS - 1) / SUM_FEWEST_TOKENS,
+                                 (int64_t)SUM_MAX_FINE_SPLITS});
+  return std::max(s, fine);
 }
 
 struct SumParams {
@@ -95,8 +102,19 @@ struct SumParams {
   int B, T, D, C;
   int seg_tokens; const int32_t* spans; int n_seg; int splits;
   const float2* factors; int nt, row_tokens, n_rows;
+  // instead of factors: the fp64 RoPE table itself; row r's factor is table[0] conj(table[start + r])
+  // (positions clamped to the table), formed in fp64 and narrowed
+  const double2* table; int64_t table_stride; int table_rows; int64_t start_row;
   float* ws;
 };
+
+__device__ __forceinline__ float2 derope_factor(const SumParams& p, int row, int pr) {
+#pragma clang fp contract(off)
+  const int64_t at = min(max(p.start_row + row, (int64_t)0), (int64_t)p.table_rows - 1);
+  const double2 z = p.table[pr], f = p.table[at * p.table_stride + pr];
+  // z conj(f), every product and sum rounded, as torch's complex128 product
+  return float2{(float)(z.x * f.x + z.y * f.y), (float)(z.y * f.x - z.x * f.y)};
+}
 
 __device__ __forceinline__ void segment_bounds(const SumParams& p, int seg, int& s0, int& s1) {
   if (p.spans) {
@@ -122,7 +140,7 @@ __global__ void __launch_bounds__(256) summary_partial_kernel(SumParams p) {
   const int per = (s1 - s0 + p.splits - 1) / p.splits;
   const int ts = s0 + split * per, te = min(ts + per, s1);
   const int d0 = c0 % p.D;  // VEC divides D: the run stays inside one head
-  const bool band = p.factors != nullptr && d0 < 2 * p.nt;
+  const bool band = (p.factors != nullptr || p.table != nullptr) && d0 < 2 * p.nt;
   const T* base = (const T*)p.x + (int64_t)b * p.x_sb + c0;
 
   // The de-rope factor row of a token is its frame (t / row_tokens). The factors of this thread's
@@ -134,11 +152,11 @@ __global__ void __launch_bounds__(256) summary_partial_kernel(SumParams p) {
   auto set_row = [&](int t) {
     row = min(t / p.row_tokens, p.n_rows - 1);
     next = row == p.n_rows - 1 ? 0x7fffffff : (row + 1) * p.row_tokens;
-    const float2* frow = p.factors + (int64_t)row * p.nt;
 #pragma unroll
     for (int e = 0; e < NP; ++e) {
       const int pr = (d0 >> 1) + e;
-      w[e] = pr < p.nt ? frow[pr] : float2{1.f, 0.f};
+      w[e] = float2{1.f, 0.f};
+      if (pr < p.nt) w[e] = p.table ? derope_factor(p, row, pr) : p.factors[(int64_t)row * p.nt + pr];
     }
   };
   if (band && ts < te) set_row(ts);
@@ -146,6 +164,8 @@ __global__ void __launch_bounds__(256) summary_partial_kernel(SumParams p) {
   float acc[VEC];
 #pragma unroll
   for (int e = 0; e < VEC; ++e) acc[e] = 0.f;
+  // Bound by HBM: 120 pages x 1,560 tokens x 1,536 bf16 channels 111 us (5.2 TB/s); with the next U
+  // tokens in flight while these are added 115 us (the other waves of the SIMD cover the wait).
   constexpr int U = 8;  // tokens in flight per thread
   for (int t = ts; t < te; t += U) {
     float f[U][VEC];
@@ -197,9 +217,17 @@ __global__ void __launch_bounds__(256) summary_reduce_kernel(SumParams p, float*
     float tot = 0.f;
     for (int b = 0; b < p.B; ++b) {
       const float* w = p.ws + ((int64_t)seg * p.B + b) * p.splits * (int64_t)p.C + c;
-      // the split partials are loaded 16 at a time (all in flight together) and added in split order
+      // the split partials are loaded 32, then 16 at a time (all in flight together) and added in
+      // split order
       float s = 0.f;
       int sp = 0;
+      for (; sp + 32 <= p.splits; sp += 32) {
+        float v[32];
+#pragma unroll
+        for (int j = 0; j < 32; ++j) v[j] = w[(int64_t)(sp + j) * p.C];
+#pragma unroll
+        for (int j = 0; j < 32; ++j) s += v[j];
+      }
       for (; sp + 16 <= p.splits; sp += 16) {
         float v[16];
 #pragma unroll
@@ -231,7 +259,9 @@ __global__ void __launch_bounds__(256) summary_reduce_kernel(SumParams p, float*
 }
 
 // =============================================================================================
-// Score + top-k: one workgroup of 1024 threads. Keys are (order-preserving score bits, inverted
+// Score + top-k: one wave per page forms the scores (in a launch of their own for more than 32 pages,
+// if the caller takes them: one workgroup's 16 waves took 67 us for 120 pages x 1,536 channels,
+// 11 us in two launches), then one workgroup of 1024 threads selects. Keys are (order-preserving score bits, inverted
 // page index), sorted descending with a bitonic network in LDS; key 0 marks masked / padding.
 // =============================================================================================
 struct TopkParams {
@@ -244,22 +274,53 @@ struct TopkParams {
   float* scores; int32_t* sel; float* sel_scores;
 };
 
+// One page's score by one wave: lane i adds channels i, i + 64, ... in order (eight loads in flight).
+__device__ __forceinline__ float page_score(const TopkParams& p, int pg, int lane) {
+  const float* row = p.index + (int64_t)pg * p.index_stride;
+  float s = 0.f;
+  int i = lane;
+  for (; i + 7 * 64 < p.dim; i += 8 * 64) {
+    float a[8], q[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      a[u] = row[i + 64 * u];
+      q[u] = p.query[i + 64 * u];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s += a[u] * q[u];
+  }
+  for (; i < p.dim; i += 64) s += row[i] * p.query[i];
+  s = wa_wave_sum(s);
+  return p.scale > 0.f ? s / p.scale : s;
+}
+
+__global__ void __launch_bounds__(256) score_kernel(TopkParams p) {
+  const int lane = threadIdx.x & 63, pg = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (pg >= p.n_pages) return;
+  const float s = page_score(p, pg, lane);
+  if (lane == 0) p.scores[pg] = s;
+}
+
+template <bool SCORED>
 __global__ void __launch_bounds__(1024) score_topk_kernel(TopkParams p) {
   __shared__ uint64_t keys[WA_HKV_MAX_PAGES];
   __shared__ float sc[WA_HKV_MAX_PAGES];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  for (int pg = w; pg < p.n_pages; pg += 16) {
-    const float* row = p.index + (int64_t)pg * p.index_stride;
-    float s = 0.f;
-    for (int i = lane; i < p.dim; i += 64) s += row[i] * p.query[i];
-    s = wa_wave_sum(s);
-    if (p.scale > 0.f) s = s / p.scale;
-    if (lane == 0) {
-      sc[pg] = s;
-      if (p.scores) p.scores[pg] = s;
-      const uint32_t hi = isnan(s) ? 0xFFFFFFFFu : wa_float_key(s);
-      const bool masked = p.mask != nullptr && p.mask[pg] != 0;
-      keys[pg] = masked ? 0ull : (((uint64_t)hi << 32) | (uint64_t)(0xFFFFFFFFu - (uint32_t)pg));
+  auto put = [&](int pg, float s) {
+    sc[pg] = s;
+    const uint32_t hi = isnan(s) ? 0xFFFFFFFFu : wa_float_key(s);
+    const bool masked = p.mask != nullptr && p.mask[pg] != 0;
+    keys[pg] = masked ? 0ull : (((uint64_t)hi << 32) | (uint64_t)(0xFFFFFFFFu - (uint32_t)pg));
+  };
+  if constexpr (SCORED) {
+    for (int pg = tid; pg < p.n_pages; pg += 1024) put(pg, p.scores[pg]);
+  } else {
+    for (int pg = w; pg < p.n_pages; pg += 16) {
+      const float s = page_score(p, pg, lane);
+      if (lane == 0) {
+        put(pg, s);
+        if (p.scores) p.scores[pg] = s;
+      }
     }
   }
   int n2 = 1;
@@ -425,13 +486,13 @@ int hkv_copies(const wa_hkv_copy* c, int64_t n, hipMemcpyKind kind, void* stream
 // =============================================================================================
 extern "C" int64_t wa_hkv_summary_workspace_bytes(int64_t B, int64_t n_seg, int64_t C, int64_t max_seg_tokens) {
   if (B <= 0 || n_seg <= 0 || C <= 0) return 0;
-  return B * n_seg * C * summary_splits(max_seg_tokens) * (int64_t)sizeof(float);
+  return B * n_seg * C * summary_splits(B, n_seg, C, max_seg_tokens) * (int64_t)sizeof(float);
 }
 
 extern "C" int wa_hkv_page_summary(const wa_hkv_summary_args* a, void* stream) {
   WA_CHECK_ARG(a && a->x && a->out && a->workspace, "wa_hkv_page_summary: null argument");
   WA_CHECK_ARG(a->x_dtype == WA_BF16 || a->x_dtype == WA_F32, "wa_hkv_page_summary: x must be bf16 or fp32");
-  WA_CHECK_ARG(a->B >= 1 && a->T >= 0 && a->H >= 1 && a->D >= 1 && (a->factors == nullptr || a->D % 2 == 0),
+  WA_CHECK_ARG(a->B >= 1 && a->T >= 0 && a->H >= 1 && a->D >= 1 && ((a->factors == nullptr && a->freqs64 == nullptr) || a->D % 2 == 0),
                "wa_hkv_page_summary: bad shape B=%lld T=%lld H=%lld D=%lld", (long long)a->B, (long long)a->T,
                (long long)a->H, (long long)a->D);
   WA_CHECK_ARG(a->n_seg >= 1 && a->n_seg <= 65535 * 64, "wa_hkv_page_summary: n_seg out of range");
@@ -439,14 +500,18 @@ extern "C" int wa_hkv_page_summary(const wa_hkv_summary_args* a, void* stream) {
   WA_CHECK_ARG(a->max_seg_tokens >= 1, "wa_hkv_page_summary: max_seg_tokens must be >= 1");
   WA_CHECK_ARG(a->spans != nullptr || a->seg_tokens <= a->max_seg_tokens,
                "wa_hkv_page_summary: seg_tokens exceeds max_seg_tokens");
-  if (a->factors) {
+  WA_CHECK_ARG(a->factors == nullptr || a->freqs64 == nullptr, "wa_hkv_page_summary: factors or freqs64, not both");
+  WA_CHECK_ARG(a->freqs64 == nullptr || (a->freqs_rows >= 1 && fits_int(a->freqs_rows) && a->freqs_stride >= a->n_temporal &&
+                                         wa_aligned16(a->freqs64)),
+               "wa_hkv_page_summary: bad RoPE table");
+  if (a->factors || a->freqs64) {
     WA_CHECK_ARG(a->n_temporal >= 1 && 2 * a->n_temporal <= a->D && a->row_tokens >= 1 && a->n_rows >= 1,
                  "wa_hkv_page_summary: bad de-rope table (n_temporal=%lld row_tokens=%lld n_rows=%lld)",
                  (long long)a->n_temporal, (long long)a->row_tokens, (long long)a->n_rows);
   }
   const int64_t C = a->H * a->D;
   WA_CHECK_ARG(fits_int(C) && fits_int(a->T), "wa_hkv_page_summary: sizes exceed int32");
-  const int64_t splits = summary_splits(a->max_seg_tokens);
+  const int64_t splits = summary_splits(a->B, a->n_seg, C, a->max_seg_tokens);
   const bool vec8 = a->D % 8 == 0 && a->x_sb % 8 == 0 && a->x_st % 8 == 0 && wa_aligned16(a->x);
   const int vec = vec8 ? 8 : (a->D % 2 == 0 ? 2 : 1);
   const int64_t lanes = (C + vec - 1) / vec;
@@ -458,7 +523,8 @@ extern "C" int wa_hkv_page_summary(const wa_hkv_summary_args* a, void* stream) {
   SumParams p{a->x, a->x_sb, a->x_st, (int)a->B, (int)a->T, (int)a->D, (int)C,
               (int)std::min<int64_t>(a->seg_tokens, 0x7fffffff), a->spans, (int)a->n_seg, (int)splits,
               (const float2*)a->factors, (int)a->n_temporal, (int)std::max<int64_t>(a->row_tokens, 1),
-              (int)std::max<int64_t>(a->n_rows, 1), (float*)a->workspace};
+              (int)std::max<int64_t>(a->n_rows, 1), (const double2*)a->freqs64, a->freqs_stride, (int)a->freqs_rows,
+              a->start_row, (float*)a->workspace};
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid((unsigned)(a->n_seg * splits), (unsigned)col_groups, (unsigned)a->B);
   if (a->x_dtype == WA_BF16) {
@@ -485,7 +551,14 @@ extern "C" int wa_hkv_score_topk(const wa_hkv_topk_args* a, void* stream) {
   WA_CHECK_ARG(a->k >= 1 && a->k <= a->n_pages, "wa_hkv_score_topk: k=%lld outside [1, n_pages]", (long long)a->k);
   TopkParams p{a->index, a->index_stride, a->query, (int)a->n_pages, (int)a->dim, a->scale, a->mask,
                (int)a->k, a->scores, a->sel, a->sel_scores};
-  score_topk_kernel<<<1, 1024, 0, (hipStream_t)stream>>>(p);
+  if (a->scores && a->n_pages > 32) {
+    score_kernel<<<(unsigned)((a->n_pages + 3) / 4), 256, 0, (hipStream_t)stream>>>(p);
+    const int rc = wa_launch_status("score_kernel");
+    if (rc != WA_OK) return rc;
+    score_topk_kernel<true><<<1, 1024, 0, (hipStream_t)stream>>>(p);
+  } else {
+    score_topk_kernel<false><<<1, 1024, 0, (hipStream_t)stream>>>(p);
+  }
   return wa_launch_status("score_topk_kernel");
 }
 

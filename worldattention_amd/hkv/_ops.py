@@ -28,12 +28,23 @@ def factor_table(temporal_freqs: torch.Tensor, new_ids: torch.Tensor, orig_ids: 
     return torch.view_as_real(f.to(device)).contiguous()
 
 
+def derope_in_place(temporal_freqs: torch.Tensor, device: torch.device) -> bool:
+    """Whether the summary kernel can read this temporal table itself: the model's complex128 table (or
+    its leading columns) on the keys' device. Any other table goes through :func:`factor_table`."""
+    t = temporal_freqs
+    return (t.dtype == torch.complex128 and t.device == device and t.dim() == 2 and t.shape[0] >= 1 and t.shape[1] >= 1
+            and t.stride(1) == 1 and t.stride(0) >= t.shape[1] and not t.is_conj() and t.data_ptr() % 16 == 0)
+
+
 def segment_means(x: torch.Tensor, *, heads: int, head_dim: int, seg_tokens: Optional[int] = None,
                   spans: Optional[Sequence[Tuple[int, int]]] = None, factors: Optional[torch.Tensor] = None,
-                  row_tokens: int = 1, normalize: bool = False) -> torch.Tensor:
+                  row_tokens: int = 1, normalize: bool = False, derope=None) -> torch.Tensor:
     """fp32 ``[n_seg, heads * head_dim]`` means over batch and the tokens of each segment of
     ``x`` ``[B, T, heads * head_dim]`` (channels contiguous), optionally de-rotated by ``factors``
-    (``[n_rows, n_temporal, 2]``, row of token t = t // row_tokens) first."""
+    (``[n_rows, n_temporal, 2]``, row of token t = t // row_tokens) first. ``derope`` instead of
+    factors: ``(temporal table, start_row, n_rows)``, a complex128 ``[positions, n_temporal]`` table on
+    ``x``'s device (:func:`derope_in_place`) from which the kernel forms the factors
+    ``table[0] * conj(table[start_row + row])`` itself."""
     dev = _lib.require_gpu(x, factors)
     if x.dim() != 3 or x.shape[-1] != heads * head_dim:
         raise ValueError(f"expected [B, T, {heads}*{head_dim}], got {tuple(x.shape)}")
@@ -59,12 +70,17 @@ def segment_means(x: torch.Tensor, *, heads: int, head_dim: int, seg_tokens: Opt
         n_rows, n_temporal = factors.shape[0], factors.shape[1]
     else:
         n_rows = n_temporal = 0
+    table = (None, 0, 0, 0)
+    if derope is not None:
+        freqs, start_row, n_rows = derope
+        n_temporal = freqs.shape[1]
+        table = (freqs.data_ptr(), freqs.stride(0), freqs.shape[0], int(start_row))
     args = _lib.HkvSummaryArgs(
         x.data_ptr(), x.stride(0), x.stride(1), _lib.dtype_code(x),
         bsz, ntok, heads, head_dim,
         seg, _lib.ptr(span_t), n_seg, max_len,
         _lib.ptr(factors), n_temporal, int(row_tokens), n_rows,
-        int(bool(normalize)), out.data_ptr(), ws.data_ptr())
+        int(bool(normalize)), out.data_ptr(), ws.data_ptr(), *table)
     _lib.call("wa_hkv_page_summary", ctypes.byref(args), _lib.stream_ptr(dev))
     return out
 
@@ -118,12 +134,12 @@ def score_topk(index: torch.Tensor, query: torch.Tensor, k: int, *, scale: float
         mask = mask.to(device=dev, dtype=torch.uint8).contiguous()
     sel = torch.empty((k,), dtype=torch.int32, device=dev)
     sel_scores = torch.empty((k,), dtype=torch.float32, device=dev)
-    scores = torch.empty((n_pages,), dtype=torch.float32, device=dev) if want_scores else None
+    scores = torch.empty((n_pages,), dtype=torch.float32, device=dev)
     args = _lib.HkvTopkArgs(index.data_ptr(), index.stride(0), query.data_ptr(), n_pages, dim,
                             float(scale) if scale and scale > 0 else 0.0, _lib.ptr(mask), int(k),
-                            _lib.ptr(scores), sel.data_ptr(), sel_scores.data_ptr())
+                            scores.data_ptr(), sel.data_ptr(), sel_scores.data_ptr())
     _lib.call("wa_hkv_score_topk", ctypes.byref(args), _lib.stream_ptr(dev))
-    return sel, sel_scores, scores
+    return sel, sel_scores, scores if want_scores else None
 
 
 def _as_blhd(t: torch.Tensor) -> torch.Tensor:

@@ -16,7 +16,7 @@ from typing import List, Optional, Sequence, Tuple
 import torch
 
 from .. import _lib
-from ._ops import factor_table, score_topk, segment_means
+from ._ops import derope_in_place, factor_table, score_topk, segment_means
 from .rope import temporal_complex_dims
 
 __all__ = [
@@ -68,17 +68,20 @@ def page_key_index(keys: torch.Tensor, page_spans: Sequence[Tuple[int, int]], *,
     bsz, ntok, heads, hd = keys.shape
     nt = temporal_complex_dims(hd)
     n_frames = max(-(-ntok // int(frame_seq_length)), 1)
-    frames = int(start_frame) + torch.arange(n_frames)
-    factors = factor_table(temporal_freqs[:, :nt], torch.zeros_like(frames), frames, keys.device)
+    band = temporal_freqs[:, :nt]
+    if derope_in_place(band, keys.device):
+        rope = dict(derope=(band, int(start_frame), n_frames))
+    else:
+        frames = int(start_frame) + torch.arange(n_frames)
+        rope = dict(factors=factor_table(band, torch.zeros_like(frames), frames, keys.device))
     if keys.stride(-1) != 1 or keys.stride(2) != hd or keys.stride(1) != heads * hd:
         keys = keys.contiguous()
     flat = keys.view(bsz, ntok, heads * hd) if keys.is_contiguous() else keys.reshape(bsz, ntok, heads * hd)
     size = _regular_page_tokens(page_spans, ntok)
     if size is not None:
-        return segment_means(flat, heads=heads, head_dim=hd, seg_tokens=size, factors=factors,
-                             row_tokens=int(frame_seq_length))
-    return segment_means(flat, heads=heads, head_dim=hd, spans=list(page_spans), factors=factors,
-                         row_tokens=int(frame_seq_length))
+        return segment_means(flat, heads=heads, head_dim=hd, seg_tokens=size, row_tokens=int(frame_seq_length), **rope)
+    return segment_means(flat, heads=heads, head_dim=hd, spans=list(page_spans), row_tokens=int(frame_seq_length),
+                         **rope)
 
 
 def _scale_of(dim: int, scale: Optional[float]) -> float:
