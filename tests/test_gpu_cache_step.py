@@ -104,6 +104,33 @@ def test_qkv_epilogue_matches_oracle(dtype, w_dtype, d):
         _close(got_means, means[:, :, first:], 1e-5, 1e-6, "block sums / count")
 
 
+@pytest.mark.parametrize("h,d,dtype,n", [(1, 8, torch.bfloat16, 17), (3, 8, torch.float32, 8), (1, 40, torch.bfloat16, 9),
+                                         (13, 40, torch.bfloat16, 23), (40, 128, torch.float32, 7), (9, 1024, torch.float32, 3)])
+def test_qkv_epilogue_row_shapes(h, d, dtype, n):
+    """Token rows at the edges of the row sum (fewer elements than its 32 chains, tails of each length)
+    and of the row tiles (one 16-byte chunk a row or head, rows of 8 to a single one a workgroup,
+    a partial last tile), values and untouched slots exact."""
+    torch.manual_seed(h * d)
+    grid, cap, ws = (1, 1, max(n - 1, 1)), n + 20, 11  # the last token lies past the grid
+    q, k, v = (torch.randn(2, n, h, d).to(dtype) * 2 for _ in range(3))
+    wq, wk = (torch.rand(h * d).to(dtype) + 0.5 for _ in range(2))
+    freqs = OK.rope_freqs(64, d)
+    cache = {"k": torch.full((2, cap, h, d), 5.0, dtype=dtype, device=DEV),
+             "v": torch.full((2, cap, h, d), -5.0, dtype=dtype, device=DEV)}
+    kw = dict(grid_sizes=torch.tensor([list(grid)] * 2), freqs=freqs, start_frame=3, write_start=ws)
+    for norm in (True, False):
+        args = dict(norm_q=wq.to(DEV), norm_k=wk.to(DEV)) if norm else {}
+        got_q = KV.qkv_epilogue(q.to(DEV), k.to(DEV), v.to(DEV), cache, **kw, **args)
+        flat = (2, n, h * d)
+        nq, nk = (OC.rms_norm(t.reshape(flat), w, 1e-6).reshape(t.shape) if norm else t for t, w in ((q, wq), (k, wk)))
+        same = _within_pair_ulp if norm else _equal
+        same(got_q, OC.causal_rope(nq, grid, freqs, 3).to(dtype), "roped q")
+        same(cache["k"][:, ws:ws + n], OC.causal_rope(nk, grid, freqs, 3).to(dtype), "cache k")
+        _equal(cache["v"][:, ws:ws + n], v, "cache v")
+        for t, fill in ((cache["k"], 5), (cache["v"], -5)):
+            assert (t[:, :ws] == fill).all() and (t[:, ws + n:] == fill).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_qkv_epilogue_with_one_grid_per_sample_matches_oracle(dtype):
     """grid_sizes with a grid of its own per sample (``causal_model.py:43`` loops over them): three

@@ -30,7 +30,13 @@ __device__ float tc_cascade(const Load& x, int start, int stride, int n) {
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
   int i = 0;
   while (i + step <= n) {
-    for (int j = 0; j < step; ++j, ++i) acc[0] = wa_add_rn(acc[0], x(start + i * stride));
+    for (int j = 0; j < step; j += 16, i += 16) {  // step >= 16; the loads of 16 elements in flight
+      float v[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) v[u] = x(start + (i + u) * stride);
+#pragma unroll
+      for (int u = 0; u < 16; ++u) acc[0] = wa_add_rn(acc[0], v[u]);
+    }
     for (int j = 1; j < 4; ++j) {
       acc[j] = wa_add_rn(acc[j], acc[j - 1]);
       acc[j - 1] = 0.f;
