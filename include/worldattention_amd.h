@@ -321,6 +321,51 @@ int64_t wa_hsa_fwd_workspace_bytes(int64_t B, int64_t H, int64_t Lq, int64_t Lkv
                                    int64_t n_sparse, int64_t n_linear, int64_t max_visits);
 int wa_hsa_fwd(const wa_hsa_fwd_args* args, void* stream);
 
+/* The HSA inference forward of any head plan in one call (hsa_attention,
+ * wan/modules/hsa/attention.py:153-259): pooling and routing of the sparse heads (wa_block_mean_pool_n,
+ * wa_route), their block-sparse attention (wa_bsa_fwd), the linear branch (wa_compress_kv_n and dense
+ * wa_bsa_fwd over the compressed keys, or wa_elu1_state and wa_elu1_readout) and the gated fusion, from
+ * one workspace; the result equals those calls made one by one. q / k / v: BLHD, fp32 or bf16 (dtype);
+ * the attention kernels' bf16 operands are copied into the workspace where they cannot be read in
+ * place. sparse_heads: both_heads and sparse_only_heads in ascending order; every head of the three
+ * lists writes o. routing: WA_ROUTE_GINI (tau_min, tau_span) or WA_ROUTE_TOPK (head_k, and unit tables
+ * of the two sparse launches with their largest visit counts); split_visits as in wa_bsa_fwd.
+ * held (optional): key block sums (held_sums) or means, [B, H, held_blocks, D] fp32, as wa_route takes
+ * them. kc / vc (optional): compressed keys and values of lc rows; otherwise k_proj / v_proj compress
+ * k and v in segments of segment_len. side_stream and events as in wa_hsa_fwd, used when both branches
+ * run. The workspace is of wa_hsa_fwd_any_workspace_bytes for the same arguments (0: refused). */
+#define WA_LINEAR_LOWRANK 0
+#define WA_LINEAR_ELU1 1
+typedef struct wa_hsa_any_args {
+  const void* q; int64_t q_sb, q_st, q_sh;
+  const void* k; int64_t k_sb, k_st, k_sh;
+  const void* v; int64_t v_sb, v_st, v_sh;
+  int32_t dtype;
+  void* o; int64_t o_sb, o_st, o_sh; int32_t o_dtype;
+  int64_t B, H, Lq, Lkv, D, block_size;
+  float scale;
+  const int32_t* sparse_heads;
+  const int32_t* both_heads; int64_t n_both;
+  const int32_t* sparse_only_heads; int64_t n_sparse_only;
+  const int32_t* linear_only_heads; int64_t n_linear_only;
+  int32_t routing; float tau_min, tau_span; const int32_t* head_k;
+  const int32_t* units_only; int64_t n_units_only, max_visits_only;
+  const int32_t* units_both; int64_t n_units_both, max_visits_both;
+  int64_t split_visits;
+  const float* held; int64_t held_blocks; int32_t held_sums;
+  int32_t linear_mode;
+  const void* kc; int64_t kc_sb, kc_st, kc_sh; int32_t kc_dtype;
+  const void* vc; int64_t vc_sb, vc_st, vc_sh; int32_t vc_dtype;
+  int64_t lc;
+  const void* k_proj; const void* v_proj; int32_t proj_dtype; int64_t proj_rank, proj_len, segment_len;
+  const void* gate_w; const float* gate_b;
+  int32_t gate_pre_bf16, gate_out_bf16, lin_round_bf16;
+  void* workspace;
+  void* side_stream; void* fork_event; void* join_event;
+} wa_hsa_any_args;
+int64_t wa_hsa_fwd_any_workspace_bytes(const wa_hsa_any_args* args);
+int wa_hsa_fwd_any(const wa_hsa_any_args* args, void* stream);
+
 /* The HSA backward of heads that take one branch each, in one call: the gradients of wa_hsa_fwd's
  * output (given its training outputs lse, state, zsum, lin and gate, its routing index / num, and
  * the sparse heads' output o, which the forward wrote rounded to bf16 into its output).

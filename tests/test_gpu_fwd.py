@@ -594,6 +594,70 @@ def test_bsa_long_rows_rank_ranges_match_oracle(case, b, h, nq):
         assert torch.equal(plain, table)
 
 
+_ANY_CALLS = [  # dtype, d, block, routing, linear mode, head modes, keys, coarse, misaligned
+    ("float32", 64, 64, "topk", "elu1", "SL", None, None, False),
+    ("float32", 128, 64, "gini", "lowrank", "BBB", None, None, False),
+    ("bfloat16", 128, 64, "gini", "lowrank", "BBB", "sums", "bfloat16", False),
+    ("bfloat16", 64, 64, "gini", "lowrank", "BSL", "pooled", "float32", False),
+    ("bfloat16", 128, 128, "topk", "elu1", "BSL", None, None, False),
+    ("bfloat16", 64, 128, "topk", "lowrank", "LLS", "sums", None, True),
+    ("float32", 128, 128, "gini", "elu1", "SSB", "pooled", None, False),
+    ("bfloat16", 64, 64, "gini", "elu1", "SSS", None, None, True),
+    ("float32", 64, 128, "topk", "lowrank", "LLL", None, "bfloat16", True),
+    ("bfloat16", 128, 64, "topk", "elu1", "LL", None, None, False),
+]
+
+
+@pytest.mark.parametrize("call", _ANY_CALLS, ids=lambda c: "-".join(str(x) for x in c))
+@pytest.mark.parametrize("b,lq,lkv", [(1, 65, 700), (2, 130, 257)])
+def test_one_call_forward_equals_the_composed_entry_points(call, b, lq, lkv, monkeypatch):
+    """Every form the one-call inference forward takes (types, head modes, routings, held key blocks,
+    coarse caches, rows that need a copy) against the same entry points called one by one from
+    Python: bit for bit, eagerly, on a side stream of the caller's and replayed from a graph."""
+    dtype, d, bs, routing, linear, modes, keys, coarse, shift = call
+    torch.manual_seed(lq + d)
+    dt, h = getattr(torch, dtype), len(modes)
+    pad = 3 if shift else 0
+    q, k, v = (torch.randn(b, n, h, d + pad, device=DEV).to(dt)[..., pad:] for n in (lq, lkv, lkv))
+    seg = 200
+    proj = [(torch.rand(-(-seg // bs), seg, device=DEV) / 40).to(dt) for _ in range(2)]
+    gate = torch.nn.Linear(d, d).to(DEV, dt)
+    kw = dict(k_coarse=None, v_coarse=None, k_proj_mat=proj[0], v_proj_mat=proj[1], gate_lin=gate, block_size=bs,
+              tau_min=0.35, tau_max=1.0, proj_segment_len=seg, routing=routing, topk=[3] * h,
+              head_modes=[{"B": "both", "S": "sparse", "L": "linear"}[m] for m in modes], linear_mode=linear)
+    if coarse:
+        kc, vc = WA._compress_many([(k, proj[0], None), (v, proj[1], None)], segment_len=seg, block_size=bs, layout="blhd")
+        kw.update(k_coarse=kc.to(getattr(torch, coarse)), v_coarse=vc.to(getattr(torch, coarse)))
+    if keys == "pooled":
+        kw["k_pooled"] = WR.pool_blhd(k, lkv, -(-lkv // bs), bs)
+    elif keys == "sums":
+        from worldattention_amd.hsa import kvcache
+        cache = dict(k=k, k_block_sums=kvcache.new_block_sums(k, bs), k_block_sums_block_size=bs)
+        kvcache.refresh_block_sums(cache, lkv)
+        kw["k_block_sums"] = cache["k_block_sums"]
+    with torch.no_grad():
+        monkeypatch.setattr(WA, "ONE_CALL", False)
+        want = WA.hsa_forward(q, k, v, **kw)
+        monkeypatch.setattr(WA, "ONE_CALL", True)
+        got = WA.hsa_forward(q, k, v, **kw)
+        assert torch.isfinite(want.float()).all() and torch.equal(got, want)
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            other = WA.hsa_forward(q, k, v, **kw)
+        torch.cuda.current_stream().wait_stream(side)
+        torch.cuda.synchronize()
+        assert torch.equal(other, want)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            replayed = WA.hsa_forward(q, k, v, **kw)
+        for _ in range(3):
+            graph.replay()
+            WA.hsa_forward(q, k, v, **kw)
+            torch.cuda.synchronize()
+            assert torch.equal(replayed, want)
+
+
 def test_hsa_forward_graph_replays_equal_eager_calls():
     """The cfg 2 call captured in a HIP graph (as bench.py times it): every replay, with eager work
     and synchronizations between replays, equals the eager call bit for bit."""

@@ -21,6 +21,7 @@ WA_OK, WA_ERR_ARG, WA_ERR_UNSUPPORTED, WA_ERR_IO = 0, -1, -2, -3
 WA_F32, WA_BF16 = 0, 1
 WA_ROUTE_GINI, WA_ROUTE_TOPK = 0, 1
 WA_EPI_PLAIN, WA_EPI_FUSE, WA_EPI_GATED = 0, 1, 2
+WA_LINEAR_LOWRANK, WA_LINEAR_ELU1 = 0, 1
 
 
 def _struct(name, fields):
@@ -189,6 +190,35 @@ HsaFwdArgs = _struct("wa_hsa_fwd_args", [
     ("lin_modes", c_void_p),
 ])
 
+HsaAnyArgs = _struct("wa_hsa_any_args", [
+    ("q", c_void_p), ("q_sb", c_int64), ("q_st", c_int64), ("q_sh", c_int64),
+    ("k", c_void_p), ("k_sb", c_int64), ("k_st", c_int64), ("k_sh", c_int64),
+    ("v", c_void_p), ("v_sb", c_int64), ("v_st", c_int64), ("v_sh", c_int64),
+    ("dtype", c_int32),
+    ("o", c_void_p), ("o_sb", c_int64), ("o_st", c_int64), ("o_sh", c_int64), ("o_dtype", c_int32),
+    ("B", c_int64), ("H", c_int64), ("Lq", c_int64), ("Lkv", c_int64), ("D", c_int64), ("block_size", c_int64),
+    ("scale", c_float),
+    ("sparse_heads", c_void_p),
+    ("both_heads", c_void_p), ("n_both", c_int64),
+    ("sparse_only_heads", c_void_p), ("n_sparse_only", c_int64),
+    ("linear_only_heads", c_void_p), ("n_linear_only", c_int64),
+    ("routing", c_int32), ("tau_min", c_float), ("tau_span", c_float), ("head_k", c_void_p),
+    ("units_only", c_void_p), ("n_units_only", c_int64), ("max_visits_only", c_int64),
+    ("units_both", c_void_p), ("n_units_both", c_int64), ("max_visits_both", c_int64),
+    ("split_visits", c_int64),
+    ("held", c_void_p), ("held_blocks", c_int64), ("held_sums", c_int32),
+    ("linear_mode", c_int32),
+    ("kc", c_void_p), ("kc_sb", c_int64), ("kc_st", c_int64), ("kc_sh", c_int64), ("kc_dtype", c_int32),
+    ("vc", c_void_p), ("vc_sb", c_int64), ("vc_st", c_int64), ("vc_sh", c_int64), ("vc_dtype", c_int32),
+    ("lc", c_int64),
+    ("k_proj", c_void_p), ("v_proj", c_void_p), ("proj_dtype", c_int32),
+    ("proj_rank", c_int64), ("proj_len", c_int64), ("segment_len", c_int64),
+    ("gate_w", c_void_p), ("gate_b", c_void_p),
+    ("gate_pre_bf16", c_int32), ("gate_out_bf16", c_int32), ("lin_round_bf16", c_int32),
+    ("workspace", c_void_p),
+    ("side_stream", c_void_p), ("fork_event", c_void_p), ("join_event", c_void_p),
+])
+
 HsaBwdArgs = _struct("wa_hsa_bwd_args", [
     ("q", c_void_p), ("q_sb", c_int64), ("q_st", c_int64), ("q_sh", c_int64),
     ("k", c_void_p), ("k_sb", c_int64), ("k_st", c_int64), ("k_sh", c_int64),
@@ -334,6 +364,8 @@ SIGNATURES = {
     "wa_elu1_readout": (c_int, [POINTER(Elu1ReadoutArgs), c_void_p]),
     "wa_hsa_fwd_workspace_bytes": (c_int64, [c_int64] * 9),
     "wa_hsa_fwd": (c_int, [POINTER(HsaFwdArgs), c_void_p]),
+    "wa_hsa_fwd_any_workspace_bytes": (c_int64, [POINTER(HsaAnyArgs)]),
+    "wa_hsa_fwd_any": (c_int, [POINTER(HsaAnyArgs), c_void_p]),
     "wa_hsa_bwd_workspace_bytes": (c_int64, [c_int64] * 8),
     "wa_hsa_bwd": (c_int, [POINTER(HsaBwdArgs), c_void_p]),
     "wa_bsa_bwd_workspace_bytes": (c_int64, [c_int64] * 6),

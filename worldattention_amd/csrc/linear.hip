@@ -78,7 +78,6 @@ __global__ void __launch_bounds__(kTokenGroups * 2 * D) compress_direct_kernel(C
   f32x16 acc[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) acc[m] = f32x16{};
-#pragma unroll MT == 1 ? 2 : 1
   for (int t0 = 32 * tg; t0 < seg_len; t0 += 32 * kTokenGroups) {
     T xv[2][8];  // tokens t0 + 16 ks + 8 g + e
     if (t0 + 32 <= seg_len) {

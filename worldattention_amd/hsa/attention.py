@@ -29,8 +29,8 @@ import torch.nn as nn
 
 from .. import _lib
 from . import distill
-from .block_sparse import bsa_forward, padded_head_dim, unit_table
-from .routing import BlockRouting, _route, block_counts, pool_for_routing
+from .block_sparse import bsa_forward, default_split, padded_head_dim, unit_table
+from .routing import BlockRouting, _route, block_counts, held_key_blocks, pool_for_routing
 
 __all__ = [
     "HSAAttention",
@@ -80,6 +80,13 @@ def coarse_length(kv_len: int, segment_len: int, proj_rank: int, block_size: int
     return total
 
 
+def _check_segment(seg: int, proj: torch.Tensor) -> None:
+    """The first segment (the longest) must fit the projection."""
+    if seg > proj.shape[1]:
+        raise ValueError(
+            f"segment length {seg} exceeds projection length {proj.shape[1]}; increase proj_segment_len")
+
+
 def _pad_channels(t: Optional[torch.Tensor], d_to: int, value: float = 0.0) -> Optional[torch.Tensor]:
     """``t`` with its last dim padded to ``d_to`` with ``value`` (differentiable)."""
     if t is None or t.shape[-1] == d_to:
@@ -97,11 +104,7 @@ def _compress_job(x: torch.Tensor, proj: torch.Tensor, out: Optional[torch.Tenso
         bsz, length, heads, d = x.shape
     if segment_len <= 0:
         segment_len = length
-    for start in range(0, length, segment_len):
-        seg = min(segment_len, length - start)
-        if seg > proj.shape[1]:
-            raise ValueError(
-                f"segment length {seg} exceeds projection length {proj.shape[1]}; increase proj_segment_len")
+    _check_segment(min(segment_len, length), proj)
     lc = coarse_length(length, segment_len, proj.shape[0], block_size)
     src = x if x.dtype in (torch.float32, torch.bfloat16) else x.float()
     if src.stride(-1) != 1:
@@ -346,6 +349,12 @@ def hsa_forward(q, k, v, *, k_coarse, v_coarse, k_proj_mat, v_proj_mat, gate_lin
         _native_split_forward(q, k, v, plan, _per_head_k(topk, heads), gate, lin_round, block_size, q_len, kv_len,
                               out, save)
         return out if out.dtype == out_dtype else out.to(out_dtype)
+    if save is None and one_call_eligible(q, k, v, k_coarse, v_coarse, k_proj_mat, v_proj_mat, plan, linear_mode):
+        _one_call_forward(q, k, v, plan, out, gate, lin_round, k_coarse=k_coarse, v_coarse=v_coarse,
+                          k_proj_mat=k_proj_mat, v_proj_mat=v_proj_mat, proj_segment_len=proj_segment_len,
+                          block_size=block_size, tau_min=tau_min, tau_max=tau_max, routing=routing, topk=topk,
+                          linear_mode=linear_mode, k_block_sums=k_block_sums, k_pooled=k_pooled, scale=scale)
+        return out if out.dtype == out_dtype else out.to(out_dtype)
     qb = _lib.kernel_ready(q)
     kb = _lib.kernel_ready(k)
     vb = _lib.kernel_ready(v)
@@ -490,6 +499,85 @@ def _native_split_forward(q, k, v, plan, ks, gate, lin_round, block_size, q_len,
     if save is not None:  # top-k routing has no thresholds (the kernel writes zeros)
         save.update(route=BlockRouting(index=index, num=num, mask=None,
                                        thresholds=torch.zeros((heads,), dtype=torch.float32, device=dev)))
+
+
+def one_call_eligible(q, k, v, k_coarse, v_coarse, k_proj_mat, v_proj_mat, plan, linear_mode) -> bool:
+    """Whether ``wa_hsa_fwd_any`` covers this forward: q, k and v of one type, fp32 or bf16, with
+    contiguous channels, and (for the low-rank branch) coarse caches or projections as its kernels take
+    them. Anything else runs the composed entry points from Python, which convert first."""
+    types = (torch.float32, torch.bfloat16)
+    if not ONE_CALL or q.shape[0] == 0 or q.dtype not in types or not q.dtype == k.dtype == v.dtype:
+        return False
+    if any(t.stride(-1) != 1 for t in (q, k, v)):
+        return False
+    if plan.linear and linear_mode == "lowrank":
+        if k_coarse is not None:
+            return all(t.dtype in types and t.stride(-1) == 1 and t.shape[1] > 0 for t in (k_coarse, v_coarse))
+        return (k_proj_mat.dtype in types and k_proj_mat.dtype == v_proj_mat.dtype
+                and k_proj_mat.shape == v_proj_mat.shape and k_proj_mat.is_contiguous() and v_proj_mat.is_contiguous()
+                and k_proj_mat.device == q.device and v_proj_mat.device == q.device and k_proj_mat.dim() == 2)
+    return True
+
+
+def _one_call_forward(q, k, v, plan, out, gate, lin_round, *, k_coarse, v_coarse, k_proj_mat, v_proj_mat,
+                      proj_segment_len, block_size, tau_min, tau_max, routing, topk, linear_mode, k_block_sums,
+                      k_pooled, scale):
+    """:func:`hsa_forward` as one library call (``wa_hsa_fwd_any``) into ``out``: the same entry points
+    with the same arguments on the same two streams as the orchestration below it."""
+    dev = q.device
+    bsz, q_len, heads, d = q.shape
+    kv_len = k.shape[1]
+    _, _, nq, nkv = block_counts(q_len, kv_len, block_size)
+    args = _lib.HsaAnyArgs(*_lib.blhd(q), *_lib.blhd(k), *_lib.blhd(v), _lib.dtype_code(q), *_lib.blhd(out),
+                           _lib.dtype_code(out), bsz, heads, q_len, kv_len, d, block_size, float(scale))
+    for name in ("both", "sparse_only", "linear_only"):
+        if plan.t[name] is not None:
+            setattr(args, name + "_heads", plan.t[name].data_ptr())
+            setattr(args, "n_" + name, plan.t[name].numel())
+    if plan.sparse:
+        args.sparse_heads = plan.t["sparse"].data_ptr()
+        args.split_visits = _lib.bsa_default_split(block_size)
+        if routing == "gini":
+            args.routing, args.tau_min, args.tau_span = _lib.WA_ROUTE_GINI, tau_min, tau_max - tau_min
+            # both sparse launches take one split: the larger one's
+            rows = bsz * max(len(plan.sparse_only), len(plan.both)) * nq
+            args.split_visits = default_split(block_size, rows, True)
+        else:
+            ks = _per_head_k(topk, heads)
+            args.routing, args.tau_span, args.head_k = _lib.WA_ROUTE_TOPK, 1.0, _lib.head_list(ks, dev).data_ptr()
+            for name, hl in (("only", plan.sparse_only), ("both", plan.both)):
+                if hl:
+                    vis = [max(0, min(ks[h], nkv)) for h in hl]
+                    units, n_units = unit_table(bsz, vis, nq, args.split_visits, dev)
+                    setattr(args, "units_" + name, units.data_ptr())
+                    setattr(args, "n_units_" + name, n_units)
+                    setattr(args, "max_visits_" + name, max(max(vis), 1))
+        held = held_key_blocks(q, k, nkv, k_block_sums, k_pooled)
+        if held is not None:
+            args.held, args.held_blocks, args.held_sums = held.data_ptr(), held.shape[2], int(k_block_sums is not None)
+    else:
+        args.routing = _lib.WA_ROUTE_GINI
+    args.linear_mode = _lib.WA_LINEAR_LOWRANK if linear_mode == "lowrank" else _lib.WA_LINEAR_ELU1
+    if plan.linear and linear_mode == "lowrank":
+        if k_coarse is not None:
+            args.kc, args.kc_sb, args.kc_st, args.kc_sh = _lib.blhd(k_coarse)
+            args.vc, args.vc_sb, args.vc_st, args.vc_sh = _lib.blhd(v_coarse)
+            args.kc_dtype, args.vc_dtype, args.lc = _lib.dtype_code(k_coarse), _lib.dtype_code(v_coarse), k_coarse.shape[1]
+        else:
+            first = min(proj_segment_len, kv_len) if proj_segment_len > 0 else kv_len
+            _check_segment(first, k_proj_mat)
+            args.k_proj, args.v_proj, args.proj_dtype = k_proj_mat.data_ptr(), v_proj_mat.data_ptr(), _lib.dtype_code(k_proj_mat)
+            args.proj_rank, args.proj_len, args.segment_len = *k_proj_mat.shape, proj_segment_len
+    args.gate_w, args.gate_b = _lib.ptr(gate.w), _lib.ptr(gate.b)
+    args.gate_pre_bf16, args.gate_out_bf16, args.lin_round_bf16 = int(gate.pre_bf16), int(gate.out_bf16), int(lin_round)
+    main = torch.cuda.current_stream(dev)
+    if plan.sparse and plan.linear:
+        side, fork, join = _fork_join(dev, main)
+        args.side_stream, args.fork_event, args.join_event = side.cuda_stream, fork.cuda_event, join.cuda_event
+    ws = torch.empty((max(_lib.lib().wa_hsa_fwd_any_workspace_bytes(args), 16),), dtype=torch.uint8, device=dev)
+    args.workspace = ws.data_ptr()
+    # the call ends with the caller's stream waiting for the side stream (see _native_split_forward)
+    _lib.call("wa_hsa_fwd_any", args, main.cuda_stream)
 
 
 def _run_linear_heads(plan, linear_mode, q, k, v, qb, k_coarse, v_coarse, k_proj_mat, v_proj_mat, proj_segment_len,

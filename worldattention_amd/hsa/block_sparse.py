@@ -60,6 +60,16 @@ def unit_table(bsz: int, visits_per_slot, nq: int, split: int, device) -> tuple[
     return hit
 
 
+def default_split(block_size: int, rows: int, unknown_lengths: bool) -> int:
+    """Visits per unit of a sparse launch: the library's default, but 64 for many rows of unknown length
+    over 64-key blocks, whose units fill the GPU's 512 unit slots anyway (three units a row at ~180
+    visits). Launch at ~180 of 512 blocks a row, D 128: 888 rows 429 us with 64 against 452 with 48;
+    300 rows 190 against 205; 50 rows 54 against 48."""
+    if unknown_lengths and block_size == 64 and rows >= 256:
+        return 64
+    return _lib.bsa_default_split(block_size)
+
+
 def bsa_forward(q, k, v, *, index, num, block_size, layout="bhld", block_sizes=None, heads=None,
                 out=None, out_dtype=None, want_lse=False, epilogue=_lib.WA_EPI_PLAIN, x=None, gate_w=None,
                 gate_b=None, gate_pre_bf16=False, gate_out_bf16=False, attn_round_bf16=False, lq=None,
@@ -104,15 +114,7 @@ def bsa_forward(q, k, v, *, index, num, block_size, layout="bhld", block_sizes=N
     n_slots = heads.numel() if heads is not None else nheads
     if n_slots == 0:
         return out, lse
-    if not split:
-        split = _lib.bsa_default_split(block_size)
-        # Rows of unknown length over 64-key blocks: units of 64 visits once the rows' units fill the
-        # GPU's 512 unit slots anyway (three units a row at ~180 visits), else 48. Launch at
-        # ~180 of 512 blocks a row, D 128: 888 rows 429 us with 64 against 452 with 48; 300 rows 190
-        # against 205; 50 rows 54 against 48.
-        if visits is None and index is not None and block_size == 64 and bsz * n_slots * nq >= 256:
-            split = 64
-    split = int(split)
+    split = int(split or default_split(block_size, bsz * n_slots * nq, visits is None and index is not None))
     units, n_units, max_visits = None, 0, width
     if visits is not None:
         vis = [max(0, min(int(n), width)) for n in visits]

@@ -148,23 +148,31 @@ def pool_for_routing(q, k, q_len: int, kv_len: int, block_size: int, heads=None,
     Either way only the queries are pooled.
     """
     _, _, nq, nkv = block_counts(q_len, kv_len, block_size)
+    held = held_key_blocks(q, k, nkv, k_block_sums, k_pooled)
+    if held is None:
+        qp, kp = pool_blhd_many([(q, q_len, nq), (k, kv_len, nkv)], block_size, heads=heads)
+        return qp, kp, {}
+    (qp,) = pool_blhd_many([(q, q_len, nq)], block_size, heads=heads)
+    key_args = dict(nkv=nkv, k_pooled_blocks=held.shape[2])
+    if k_block_sums is not None:
+        key_args.update(k_sum_len=kv_len, block_size=block_size, k_sum_bf16=k.dtype == torch.bfloat16)
+    return qp, held, key_args
+
+
+def held_key_blocks(q, k, nkv: int, k_block_sums=None, k_pooled=None):
+    """The caller's checked key block sums or means (see :func:`pool_for_routing`), or None."""
     if k_block_sums is not None and k_pooled is not None:
         raise ValueError("pass k_block_sums or k_pooled, not both")
     held = k_block_sums if k_block_sums is not None else k_pooled
     if held is None:
-        qp, kp = pool_blhd_many([(q, q_len, nq), (k, kv_len, nkv)], block_size, heads=heads)
-        return qp, kp, {}
+        return None
     b, _, h, d = k.shape
     if (held.dtype != torch.float32 or held.dim() != 4 or held.shape[0] != b or held.shape[1] != h
             or held.shape[3] != d or held.shape[2] < nkv or not held.is_contiguous()):
         raise ValueError(f"cached key blocks must be contiguous fp32 [{b}, {h}, >= {nkv}, {d}], got "
                          f"{held.dtype} {tuple(held.shape)}")
     _lib.require_gpu(held, q)
-    (qp,) = pool_blhd_many([(q, q_len, nq)], block_size, heads=heads)
-    key_args = dict(nkv=nkv, k_pooled_blocks=held.shape[2])
-    if k_block_sums is not None:
-        key_args.update(k_sum_len=kv_len, block_size=block_size, k_sum_bf16=k.dtype == torch.bfloat16)
-    return qp, held, key_args
+    return held
 
 
 def _route(probs, qp, kp, *, mode, tau_min=0.0, tau_max=1.0, head_k=None, heads=None,
