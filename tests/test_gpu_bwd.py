@@ -125,6 +125,53 @@ def test_sparse_backward_transposed_lists_by_counting(nq, nkv):
         assert_close(g, r, 2e-2 * scale, 2e-3 * scale, what=name)
 
 
+@pytest.mark.parametrize("d,bs,lkv,sparse,acc,bf16", [
+    (64, 64, 1, False, False, False), (128, 64, 525, False, True, False), (128, 128, 525, False, False, True),
+    (64, 128, 130, True, False, True), (128, 64, 200, True, True, False), (128, 128, 257, True, False, False)])
+def test_key_side_lists_cut_into_runs_match_the_oracle(d, bs, lkv, sparse, acc, bf16):
+    """Few key blocks: every list is cut into runs that a second launch adds up. Dense lists, lists
+    shorter than the number of runs, empty ones, partial last blocks, a heads subset, added-to fp32
+    gradients and bf16 ones (rounded once: 2^-9 of the gradient on top of the fp32 bound)."""
+    from worldattention_amd.hsa._bwd import bsa_backward
+    from worldattention_amd.hsa.block_sparse import bsa_forward
+    torch.manual_seed(lkv + d)
+    b, h, lq = 1, 3, 2500
+    nq, nkv = -(-lq // bs), -(-lkv // bs)
+    q = torch.randn(b, h, lq, d).bfloat16()
+    k, v = (torch.randn(b, h, lkv, d).bfloat16() for _ in range(2))
+    do = torch.randn(b, h, lq, d).bfloat16() * 0.25
+    index = num = None
+    allow = torch.ones(h, lq, lkv, dtype=torch.bool)
+    if sparse:
+        index = torch.stack([torch.randperm(nkv) for _ in range(b * h * nq)]).view(b, h, nq, nkv).int()
+        num = torch.randint(1, nkv + 1, (b, h, nq), dtype=torch.int32)
+        num[0, 0] = (index[0, 0] == nkv - 1).int().argmax(-1).clamp(min=1)  # the last block: (nearly) never
+        index[0, 2, 3:, 0], num[0, 2, 3:] = 0, 1             # blocks other than 0: at most three query blocks
+        blocks = torch.zeros(h, nq, nkv, dtype=torch.bool)
+        for i in range(h):
+            for r in range(nq):
+                blocks[i, r, index[0, i, r, :num[0, i, r]].long()] = True
+        allow = blocks.repeat_interleave(bs, 1)[:, :lq].repeat_interleave(bs, 2)[:, :, :lkv]
+    heads = torch.tensor([2, 0], dtype=torch.int32)
+    dev = lambda t: None if t is None else t.to(DEV)
+    qg, kg, vg = dev(q), dev(k), dev(v)
+    out = torch.zeros(b, h, lq, d, device=DEV)
+    _, lse = bsa_forward(qg, kg, vg, index=dev(index), num=dev(num), block_size=bs, heads=dev(heads), out=out,
+                         want_lse=True)
+    kw = dict(dtype=torch.bfloat16 if bf16 else torch.float32, device=DEV)
+    dk, dv = (torch.full((b, h, lkv, d), 0.5, **kw) for _ in range(2))
+    bsa_backward(qg, kg, vg, out, lse, dev(do), index=dev(index), num=dev(num), block_size=bs, heads=dev(heads),
+                 dk=dk, dv=dv, kv_accumulate=acc)
+    qr, kr, vr = (t[0].double().requires_grad_() for t in (q, k, v))
+    p = (qr @ kr.transpose(1, 2) * d ** -0.5).masked_fill(~allow, float("-inf")).softmax(-1)
+    (p @ vr).backward(do[0].double())
+    for name, g, r in (("dk", dk, kr.grad), ("dv", dv, vr.grad)):
+        for i in range(h):
+            want = r[i] + (0.5 if acc else 0.0) if i in (0, 2) else torch.full_like(r[i], 0.5)
+            scale = max(1.0, r[i].abs().max().item())
+            assert_close(g[0, i], want, 2e-2 * scale, 2e-3 * scale, what=f"{name} head {i}")
+
+
 def test_sparse_backward_many_query_blocks():
     """More than 256 query blocks: the transposed lists come from the scanning kernel instead of the
     counting one."""

@@ -51,6 +51,10 @@ struct BwdParams {
   bf16_t* dob;       // [B, n_heads, Lq, D]
   int32_t* k2q;      // [B, n_heads, Nkv, Nq]: (query block) | (multiplicity << 16)
   int32_t* k2q_num;  // [B, n_heads, Nkv]
+  // dK / dV of launches with few key parts: each list is cut into `parts` runs whose fp32 results
+  // ([parts][dK, dV][B * n_heads][Lkv][D]) one more launch adds up (NULL: the gradients are written)
+  float* part_kv;
+  int parts;
   int4* kv_info;     // [B * n_heads * Nkv] dkdv launch order: per slab, key blocks by descending list
                      // length as {block id, list length, first list entry, 0}
 };
@@ -604,7 +608,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
   // one (else through the slabs in order), so an XCD's workgroups share their slabs' Q and dO
   // tiles; one load gives the block, its list length and its first list entry
   const int gpos = wa_xcd_remap((int)blockIdx.x, (int)gridDim.x);
-  const int pos = gpos / HB, hb = gpos % HB;
+  const int part = gpos % p.parts, hb = gpos / p.parts % HB, pos = gpos / p.parts / HB;
   int id, nl, e0;
   if (p.kv_info) {
     const int4 inf = p.kv_info[pos];
@@ -623,7 +627,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
   const int h = head_of(p, hs);
   if (h < 0 || h >= p.H) return;
   const int kb0 = j * BS + hb * KW;  // first key of this part
-  if (nl == 0) {
+  const int32_t* lst = p.k2q + (((int64_t)b * p.n_heads + hs) * p.Nkv + j) * p.Nq;
+  if (p.parts > 1) {  // this workgroup's run of the list
+    const int l0 = (int)((int64_t)nl * part / p.parts), l1 = (int)((int64_t)nl * (part + 1) / p.parts);
+    lst += l0;
+    nl = l1 - l0;
+    e0 = __builtin_amdgcn_readfirstlane(nl > 0 ? *lst : 0);
+  }
+  if (nl == 0 && !p.part_kv) {
     // no query block listed this key block: its written gradients are zero (accumulated ones
     // keep their values), with no tile streamed
     const int rows = max(0, min(KW, p.Lkv - kb0));
@@ -655,7 +666,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
   const int key = hb * KW + kl;  // ... and within the block
   const bool k_ok = key < real;
   const int64_t srow = ((int64_t)b * p.n_heads + hs) * p.Lq;
-  const int32_t* lst = p.k2q + (((int64_t)b * p.n_heads + hs) * p.Nkv + j) * p.Nq;
   bf16x8 kvf[DC];
   f32x16 acc[DT];   // S-wave: dV^T; dP-wave: dK^T (lane = key, registers = channels)
 #pragma unroll
@@ -764,10 +774,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
   // fragments are waited for before the first step: later, the compiler (which cannot count the
   // ring's inline-assembly loads) would wait for every load in flight.
   static_assert(ST - 1 <= QPB, "the prologue tiles must come from the first list entry");
-  issue(IC<0>{}, 0);
-  if constexpr (ST >= 3) {
-    if (total > 1) issue(IC<1>{}, 1);
-  }
+  if (total > 0) issue(IC<0>{}, 0);
   for (int i = tid; i < min(nl, LM); i += NT) s_lst[i] = lst[i];
   {
     const int kr = j * BS + (k_ok ? key : 0);
@@ -785,16 +792,28 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
   for (int t = 0; t < total; t += ST) {
     step(IC<0>{}, t);
     if (t + 1 < total) step(IC<1>{}, t + 1);
-    if constexpr (ST >= 3) {
-      if (t + 2 < total) step(IC<2>{}, t + 2);
-    }
-    if constexpr (ST >= 4) {
-      if (t + 3 < total) step(IC<3>{}, t + 3);
-    }
   }
   // each lane holds its key's row: channels 32 tt + 8 rq + 4 g .. + 3 of tile tt (keys past the
   // block's end get zeros); dK is scaled here
   const float osc = swave ? 1.f : p.scale;
+  if (p.part_kv) {
+    const int prow = kb0 + kl;
+    if (prow >= p.Lkv) return;
+    const int64_t slab = (int64_t)p.B * p.n_heads;
+    const int64_t at = ((int64_t)part * 2 + (swave ? 1 : 0)) * slab + (int64_t)b * p.n_heads + hs;
+    float* dst = p.part_kv + (at * p.Lkv + prow) * D + 4 * g;
+#pragma unroll
+    for (int tt = 0; tt < DT; ++tt) {
+#pragma unroll
+      for (int rq = 0; rq < 4; ++rq) {
+        f32x4 v4;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v4[i] = k_ok ? acc[tt][rq * 4 + i] * osc : 0.f;
+        *(f32x4*)(dst + 32 * tt + 8 * rq) = v4;
+      }
+    }
+    return;
+  }
   if (p.dkv_vec) {
     // bf16 rows staged in the (drained) ring, row r's 16-byte chunk c at chunk c ^ swz(r): one
     // 8-byte write per (tile, rq), then 16-byte stores of whole rows
@@ -853,6 +872,50 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
     for (int r = 0; r < 16; ++r)
       dst[32 * tt + 8 * (r >> 2) + (r & 3)] = prev[tt][r] + (k_ok ? acc[tt][r] * osc : 0.f);
   }
+}
+
+// Adds the runs' dK and dV (four channels a thread) in run order into the gradients.
+__global__ void __launch_bounds__(256) dkdv_sum_kernel(BwdParams p, int D) {
+  const int64_t slab = (int64_t)p.B * p.n_heads * p.Lkv * (D / 4);
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= 2 * slab) return;
+  const bool is_v = i >= slab;
+  int64_t r = i - (is_v ? slab : 0);
+  const int c = (int)(r % (D / 4)) * 4;
+  r /= D / 4;
+  const int row = (int)(r % p.Lkv), hs = (int)(r / p.Lkv % p.n_heads), b = (int)(r / p.Lkv / p.n_heads);
+  const int h = head_of(p, hs);
+  if (h < 0 || h >= p.H) return;
+  const f32x4* src = (const f32x4*)p.part_kv + i;
+  f32x4 v[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) v[q] = src[min(q, p.parts - 1) * 2 * slab];
+  f32x4 sum = v[0];
+#pragma unroll
+  for (int q = 1; q < 8; ++q)
+    if (q < p.parts) sum += v[q];
+  const int64_t at = is_v ? (int64_t)b * p.dv_sb + (int64_t)h * p.dv_sh + (int64_t)row * p.dv_st + c
+                          : (int64_t)b * p.dk_sb + (int64_t)h * p.dk_sh + (int64_t)row * p.dk_st + c;
+  void* out = is_v ? p.dv : p.dk;
+  if (p.dkv_bf16) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ((bf16_t*)out)[at + e] = (bf16_t)sum[e];
+    return;
+  }
+  const bool add = is_v ? p.dv_acc : p.dk_acc;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) ((float*)out)[at + e] = add ? ((float*)out)[at + e] + sum[e] : sum[e];
+}
+
+// Runs per list: with fewer key parts than the GPU runs at a time (two per CU), long lists are cut so
+// that about 512 workgroups run, each with at least 8 query steps where every query block listed
+// the key block. The dense backward over 525 compressed keys of 12 heads (4680 queries): 148 us as
+// 108 workgroups of 74 steps, 76 + 10 us cut in five (128-key blocks: 120 parts) with the sum.
+int dkdv_parts(int64_t B, int64_t n_heads, int64_t Lq, int64_t Lkv, int64_t block_size) {
+  const int64_t key_parts = B * n_heads * ((Lkv + block_size - 1) / block_size) * (block_size / DKDV_KEYS);
+  if (key_parts <= 0 || key_parts >= 384) return 1;
+  const int64_t steps = (Lq + 63) / 64;
+  return (int)std::max<int64_t>(1, std::min({(int64_t)8, (512 + key_parts - 1) / key_parts, steps / 8}));
 }
 
 // The launches of one backward on stream s; with a second stream sq (and its fork / join events)
@@ -917,14 +980,24 @@ int launch_bwd(const BwdParams& bp, hipStream_t s, hipStream_t sq, hipEvent_t fo
     } else {
       kp.kv_info = nullptr;
     }
-    hipLaunchKernelGGL((bwd_dkdv_kernel<D, BS>), dim3((unsigned)(bp.B * nh * bp.Nkv * (BS / DKDV_KEYS))), dim3(256), 0,
-                       s, kp);
+    hipLaunchKernelGGL((bwd_dkdv_kernel<D, BS>), dim3((unsigned)(bp.B * nh * bp.Nkv * (BS / DKDV_KEYS) * bp.parts)),
+                       dim3(256), 0, s, kp);
     if ((rc = wa_launch_status("bsa_bwd_dkdv"))) return joined(rc);
+    if (bp.part_kv) {
+      const int64_t n = 2 * (int64_t)bp.B * nh * bp.Lkv * (D / 4);
+      hipLaunchKernelGGL(dkdv_sum_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, kp, D);
+      if ((rc = wa_launch_status("bsa_bwd_dkdv_sum"))) return joined(rc);
+    }
   }
   return joined(WA_OK);
 }
 
 int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
+
+int64_t part_bytes(int64_t B, int64_t n_heads, int64_t Lq, int64_t Lkv, int64_t D, int64_t block_size) {
+  const int parts = dkdv_parts(B, n_heads, Lq, Lkv, block_size);
+  return parts > 1 ? align256(parts * 2 * B * n_heads * Lkv * D * 4) : 0;
+}
 
 }  // namespace
 
@@ -932,7 +1005,8 @@ extern "C" int64_t wa_bsa_bwd_workspace_bytes(int64_t B, int64_t n_heads, int64_
                                               int64_t block_size) {
   const int64_t nq = (Lq + block_size - 1) / block_size, nkv = (Lkv + block_size - 1) / block_size;
   return 2 * align256(B * n_heads * Lq * 4) + align256(B * n_heads * Lq * D * 2) +
-         align256(B * n_heads * nkv * nq * 4) + align256(B * n_heads * nkv * 4) + align256(B * n_heads * nkv * 16);
+         align256(B * n_heads * nkv * nq * 4) + align256(B * n_heads * nkv * 4) + align256(B * n_heads * nkv * 16) +
+         part_bytes(B, n_heads, Lq, Lkv, D, block_size);
 }
 
 // wa_bsa_bwd with its dQ pass on a second stream (NULL: one stream), forked from `stream` after the
@@ -1012,6 +1086,9 @@ int wa_bsa_bwd_streams(const wa_bsa_bwd_args* a, void* stream, void* dq_stream, 
   bp.k2q_num = (int32_t*)ws;
   ws += align256(a->B * nh * nkv * 4);
   bp.kv_info = (int4*)ws;
+  ws += align256(a->B * nh * nkv * 16);
+  bp.parts = a->dk && a->dv ? dkdv_parts(a->B, nh, a->Lq, a->Lkv, a->block_size) : 1;
+  bp.part_kv = bp.parts > 1 ? (float*)ws : nullptr;
 
   hipStream_t s = (hipStream_t)stream, sq = (hipStream_t)dq_stream;
   hipEvent_t fe = (hipEvent_t)fork_event, je = (hipEvent_t)join_event;
