@@ -92,6 +92,36 @@ def test_gini_thresholds_equal_torch_fp32_reductions(shape):
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("b,h,nq,nkv,d,heads,bs", [
+    (1, 1, 1, 1, 128, None, 0), (1, 3, 4, 7, 64, [2, 0], 64), (2, 2, 5, 255, 128, None, 48), (1, 2, 9, 256, 64, None, 0),
+    (1, 3, 6, 257, 128, [1], 64), (2, 4, 7, 511, 64, None, 64), (1, 2, 11, 512, 128, None, 128)])
+def test_gini_rows_in_fours_equal_the_one_row_kernel(b, h, nq, nkv, d, heads, bs):
+    """Gini routing from pooled vectors (up to 512 blocks, head dims 64 and 128: four rows a
+    workgroup) against the one-row kernel, which still routes given maps and forms the maps of
+    top-k calls: probabilities, permutations, counts and thresholds bit for bit, at both key widths'
+    edges, a partial last group of rows, a heads subset, cached sums (power-of-two block size or not,
+    partial last block), and equal and underflowed scores."""
+    from worldattention_amd import _lib
+    from worldattention_amd.hsa.routing import _route
+    torch.manual_seed(nkv + d)
+    qp, kp = torch.randn(b, h, nq, d, device=DEV) * 3, torch.randn(b, h, nkv + 2, d, device=DEV)
+    kp[:, :, nkv // 2:nkv] = kp[:, :, :nkv - nkv // 2].clone()   # every score (nearly) twice
+    qp[0, 0, 0] *= 1e3                                           # one block's probability is 1, others 0
+    hl = torch.arange(h) if heads is None else torch.tensor(sorted(heads))
+    kw = dict(heads=None if heads is None else torch.tensor(heads, dtype=torch.int32, device=DEV), nkv=nkv,
+              k_pooled_blocks=nkv + 2)
+    if bs:
+        kw.update(k_sum_len=nkv * bs - (bs // 3 if nkv > 7 else 0), block_size=bs, k_sum_bf16=nkv % 2 == 1)
+    tau = dict(mode=_lib.WA_ROUTE_GINI, tau_min=0.35, tau_max=1.0)
+    got, probs = _route(None, qp, kp, want_probs=True, return_mask=True, **tau, **kw)
+    top, want_probs = _route(None, qp, kp, mode=_lib.WA_ROUTE_TOPK, want_probs=True, **kw)
+    want, _ = _route(torch.nan_to_num(want_probs), None, None, return_mask=True, heads=kw["heads"], **tau)
+    assert torch.equal(probs[:, hl], want_probs[:, hl])
+    assert torch.equal(got.index[:, hl], top.index[:, hl]) and torch.equal(got.index[:, hl], want.index[:, hl])
+    assert torch.equal(got.num, want.num) and torch.equal(got.thresholds, want.thresholds)
+    assert torch.equal(got.mask[:, hl], want.mask[:, hl])
+
+
 @pytest.mark.parametrize("nkv", [16, 37, 256, 512, 1100])
 def test_routing_is_bit_exact_given_identical_maps_with_ties(nkv):
     torch.manual_seed(nkv)

@@ -694,6 +694,171 @@ __global__ void __launch_bounds__(256) route_wave_kernel(RouteParams p) {
   if (lane == 0 && hw == 0) p.num[row] = n;
 }
 
+// Gini routing of rows of at most 512 blocks at head dims 64 and 128: four rows (query blocks
+// i0 .. i0 + 3 of one head) per workgroup of 16 waves, with the values of route_kernel bit for bit
+// (every sum in its order). One row per workgroup read the head's pooled keys from L2 once per row
+// (236 MB at 12 heads of 74 x 512 blocks) and sorted through LDS with a barrier per stage; here a
+// pass over the keys serves four rows, with every load of a thread in flight at once, and the sort
+// runs in registers and lane moves except for its three strides that cross waves. Row r belongs to
+// waves 4r .. 4r + 3 from the softmax on. Bound by the sort's chain of 42 lane-move stages and the
+// one pass over the keys: 38 us with one row per workgroup, 21 us here (12 heads, 74 x 512, D 128).
+constexpr int GINI_ROWS = 4;
+
+template <int DK, int KPT>
+__global__ void __launch_bounds__(256 * GINI_ROWS) route_gini_kernel(RouteParams p) {
+  constexpr int R = GINI_ROWS, NP = 256 * KPT, CPT = DK / 32, U = NP / (32 * R);
+  __shared__ __attribute__((aligned(16))) float q_sh[R][DK];
+  __shared__ float s_sh[R][NP];
+  __shared__ uint64_t xk[2][R][NP];  // keys on their way to another wave, then the Gini terms
+  __shared__ float red_mx[R][4];
+  __shared__ double red_se[R][4];
+  __shared__ float chain[R][32];
+  if (clear_unrouted(p)) return;
+  const int i0 = blockIdx.x * R, hs = blockIdx.y, b = blockIdx.z;
+  const int h = p.heads ? p.heads[hs] : hs;
+  if (h < 0 || h >= p.H) return;  // uniform
+  const int tid = threadIdx.x, lane = tid & 63, rg = tid >> 8, t = tid & 255, wr = t >> 6;
+  const int N = p.Nkv;
+  const int64_t row0 = ((int64_t)b * p.H + h) * p.Nq;
+  const int i = min(i0 + rg, p.Nq - 1);  // past the last row: the last again, not written
+  const bool ok = i0 + rg < p.Nq;
+  const int64_t row = row0 + i;
+
+  // 1. scores: 8 threads per key row, thread tg reads d = 32 c + 4 tg .. + 3 (see route_kernel)
+  {
+    const float* kbase = p.kp + ((int64_t)b * p.H + h) * (int64_t)p.kp_blocks * DK;
+    const int grp = tid >> 3, tg = tid & 7;
+    f32x4 kv[U][CPT];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int c = 0; c < CPT; ++c)
+        kv[u][c] = *(const f32x4*)(kbase + (int64_t)min(32 * R * u + grp, N - 1) * DK + 32 * c + 4 * tg);
+    }
+    if (tid < R * DK) q_sh[tid / DK][tid % DK] = p.qp[(row0 + min(i0 + tid / DK, p.Nq - 1)) * DK + tid % DK];
+#pragma unroll
+    for (int u = 0; u < U; ++u) pooled_key_row(p, kv[u], min(32 * R * u + grp, N - 1));
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      f32x4 qv[CPT];
+#pragma unroll
+      for (int c = 0; c < CPT; ++c) qv[c] = *(const f32x4*)&q_sh[r][32 * c + 4 * tg];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        float s = 0.f;
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s = fmaf(qv[c][e], kv[u][c][e], s);
+        }
+#pragma unroll
+        for (int o = 1; o < 8; o <<= 1) s += __uint_as_float(xor_lanes(__float_as_uint(s), o, lane));
+        const int j = 32 * R * u + grp;
+        if (j < N && tg == 0) s_sh[r][j] = s * p.scale;
+      }
+    }
+  }
+  __syncthreads();
+
+  // 2. softmax over the row: this thread's blocks are t and t + 256
+  float sc[KPT];
+  float mx = -INFINITY;
+#pragma unroll
+  for (int e = 0; e < KPT; ++e) {
+    sc[e] = t + 256 * e < N ? s_sh[rg][t + 256 * e] : -INFINITY;
+    mx = fmaxf(mx, sc[e]);
+  }
+  mx = wa_wave_max(mx);
+  if (lane == 0) red_mx[rg][wr] = mx;
+  __syncthreads();
+  mx = red_mx[rg][0];
+#pragma unroll
+  for (int k = 1; k < 4; ++k) mx = fmaxf(mx, red_mx[rg][k]);
+  double se = 0.0;
+#pragma unroll
+  for (int e = 0; e < KPT; ++e) {
+    if (t + 256 * e < N) {
+      sc[e] = expf(sc[e] - mx);
+      se += (double)sc[e];
+    }
+  }
+  se = wa_wave_sum_d(se);
+  if (lane == 0) red_se[rg][wr] = se;
+  __syncthreads();
+  se = 0.0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) se += red_se[rg][k];
+  const float inv_sum = (float)(1.0 / se);
+
+  // 3. composite keys (see route_kernel) and the bitonic sort, descending; slot pos0 + 64 e + lane
+  uint64_t key[KPT];
+#pragma unroll
+  for (int e = 0; e < KPT; ++e) {
+    const int j = t + 256 * e;
+    key[e] = 0;
+    if (j < N) {
+      const float pj = sc[e] * inv_sum;
+      if (p.probs_out && ok) p.probs_out[row * N + j] = pj;
+      key[e] = ((uint64_t)wa_float_key(pj) << 32) | (uint64_t)(0xFFFFFFFFu - (uint32_t)j);
+    }
+  }
+  const int pos0 = 64 * KPT * wr;
+  int buf = 0;  // alternates: a buffer is written again two barriers after it was read
+#pragma unroll
+  for (int size = 2; size <= NP; size <<= 1) {
+#pragma unroll
+    for (int stride = size >> 1; stride > 0; stride >>= 1) {
+      if (stride >= 64 * KPT) {
+#pragma unroll
+        for (int e = 0; e < KPT; ++e) xk[buf][rg][pos0 + 64 * e + lane] = key[e];
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < KPT; ++e) {
+          const int pos = pos0 + 64 * e + lane;
+          const uint64_t other = xk[buf][rg][pos ^ stride];
+          const bool keep = (key[e] > other) == (((pos & stride) == 0) == ((pos & size) == 0));
+          key[e] = keep ? key[e] : other;
+        }
+        buf ^= 1;
+      } else if (stride >= 64) {  // KPT = 2: this lane's two keys
+        if ((key[0] < key[KPT - 1]) == ((pos0 & size) == 0)) {
+          const uint64_t a = key[0];
+          key[0] = key[KPT - 1];
+          key[KPT - 1] = a;
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < KPT; ++e) {
+          const uint64_t other = shfl_xor_u64(key[e], stride, lane);
+          const int pos = pos0 + 64 * e + lane;
+          const bool keep = (key[e] > other) == (((lane & stride) == 0) == ((pos & size) == 0));
+          key[e] = keep ? key[e] : other;
+        }
+      }
+    }
+  }
+
+  // 4. permutation and Gini terms, summed as in route_kernel (buffer `buf` is free: the last
+  // exchange read the other one)
+  float* tl = (float*)xk[buf][rg];
+#pragma unroll
+  for (int e = 0; e < KPT; ++e) {
+    const int m = pos0 + 64 * e + lane;
+    if (m < N) {
+      const float pm = key_to_float(key[e]);
+      if (ok) {
+        p.index[row * N + m] = (int32_t)(0xFFFFFFFFu - (uint32_t)key[e]);
+        p.ws_sorted[row * N + m] = pm;
+      }
+      tl[m] = wa_mul_rn((float)(N + 1 - 2 * (m + 1)), pm);
+    }
+  }
+  __syncthreads();
+  const float s = tc_inner_sum_wg([&](int m) { return tl[m]; }, 0, N, chain[rg], 256 * rg);
+  if (t == 0 && ok) p.ws_gini[row] = wa_div_rn(s, (float)N);
+}
+
 // Gini second pass: per-head threshold (mean of the head's row Ginis), then the count of sorted
 // slots whose exclusive prefix is below it. The prefix is the reference's: a sequential double
 // running sum rounded to fp32, minus the slot's own weight in fp32 (routing.py:95-113). Two
@@ -1007,7 +1172,17 @@ extern "C" int wa_route(const wa_route_args* a, void* stream) {
     else route_wave_launch<false>(rp, a->D, a->Nkv, wgrid, s);
     return wa_launch_status("route_wave");
   }
-  hipLaunchKernelGGL(route_kernel, grid, dim3(256), (size_t)rp.NP * sizeof(uint64_t), s, rp);
+  // Gini routing from pooled vectors in fours of rows where the sort fits in registers (512 blocks:
+  // two keys a thread) and a thread's key row loads are whole 16-byte chunks (21 us against 38 at
+  // 74 x 512 blocks, 12 heads); given maps, longer rows and other head dims take the one-row kernel.
+  if (a->mode == WA_ROUTE_GINI && !a->probs && a->Nkv <= 512 && (a->D == 64 || a->D == 128)) {
+    const dim3 ggrid((unsigned)((a->Nq + GINI_ROWS - 1) / GINI_ROWS) + 1, (unsigned)nh, (unsigned)a->B);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, ggrid, dim3(256 * GINI_ROWS), 0, s, rp); };
+    if (a->D == 128) a->Nkv <= 256 ? go(route_gini_kernel<128, 1>) : go(route_gini_kernel<128, 2>);
+    else a->Nkv <= 256 ? go(route_gini_kernel<64, 1>) : go(route_gini_kernel<64, 2>);
+  } else {
+    hipLaunchKernelGGL(route_kernel, grid, dim3(256), (size_t)rp.NP * sizeof(uint64_t), s, rp);
+  }
   int rc = wa_launch_status("route");
   if (rc != WA_OK || a->mode != WA_ROUTE_GINI) return rc;
   const int64_t staged = a->B * a->Nq <= GINI_STAGE_MAX ? a->B * a->Nq : 0;
