@@ -442,7 +442,18 @@ typedef struct wa_bsa_bwd_args {
   void* workspace;
   int32_t dkv_dtype;  /* WA_F32 or WA_BF16 */
   int32_t dq_dtype;   /* WA_F32, or WA_BF16 (rounded to nearest even once; requires dq_accumulate off) */
+  /* add_k / add_v (optional, together): the fp32 gradients [B, rows, H, D] (one set of strides, unit
+   * channel stride) of the keys and values compressed from these k / v by the bf16 projections
+   * proj_k / proj_v [add_rank, add_len] (wa_compress_kv over segments of add_segment tokens and
+   * blocks of add_block): E^T g is added to dk / dv in fp32 before they are written, which replaces
+   * wa_compress_kv_bwd's dx. Requires written (not accumulated) dk / dv, no block_sizes, every head's
+   * dk / dv to want the term, and wa_bsa_bwd_key_runs(...) == 1. */
+  const float* add_k; const float* add_v; int64_t add_sb, add_st, add_sh;
+  const void* proj_k; const void* proj_v;
+  int64_t add_rank, add_len, add_segment, add_block;
 } wa_bsa_bwd_args;
+/* Runs that a key block's list is cut into (1 but for launches with few key blocks). */
+int64_t wa_bsa_bwd_key_runs(int64_t B, int64_t n_heads, int64_t Lq, int64_t Lkv, int64_t block_size);
 int64_t wa_bsa_bwd_workspace_bytes(int64_t B, int64_t n_heads, int64_t Lq, int64_t Lkv, int64_t D,
                                    int64_t block_size);
 int wa_bsa_bwd(const wa_bsa_bwd_args* args, void* stream);

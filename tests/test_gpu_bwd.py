@@ -172,6 +172,45 @@ def test_key_side_lists_cut_into_runs_match_the_oracle(d, bs, lkv, sparse, acc, 
             assert_close(g[0, i], want, 2e-2 * scale, 2e-3 * scale, what=f"{name} head {i}")
 
 
+@pytest.mark.parametrize("b,h,d,bs,lkv,seg,rank,bf16", [
+    (1, 2, 128, 64, 700, 156, 3, True), (2, 1, 64, 128, 333, 100, 40, True), (1, 1, 128, 128, 1000, 1000, 128, False),
+    (1, 2, 64, 64, 130, 10, 5, True), (1, 1, 128, 64, 6200, 1560, 25, True)])
+def test_compressed_term_in_the_key_side_pass_equals_its_own_pass(b, h, d, bs, lkv, seg, rank, bf16):
+    """E^T g of compressed keys and values added by the dK/dV pass against wa_compress_kv_bwd's dx
+    (same products in the same order: equal): segments that end within a wave's 32 keys, several
+    segments there, ranks past 32, a partial last block, unlisted key blocks, an infinite gradient."""
+    from worldattention_amd.hsa._autograd import _compress_backward
+    from worldattention_amd.hsa._bwd import bsa_backward
+    from worldattention_amd.hsa.block_sparse import bsa_forward
+    torch.manual_seed(lkv + seg)
+    lq = 300
+    nq, nkv = -(-lq // bs), -(-lkv // bs)
+    q = torch.randn(b, lq, h, d, device=DEV).bfloat16()
+    k, v = (torch.randn(b, lkv, h, d, device=DEV).bfloat16() for _ in range(2))
+    do = torch.randn(b, lq, h, d, device=DEV)
+    index = torch.randint(0, max(nkv - 1, 1), (b, h, nq, nkv), dtype=torch.int32, device=DEV)
+    num = torch.randint(0, min(nkv, 4) + 1, (b, h, nq), dtype=torch.int32, device=DEV)
+    rows = sum(min(rank, -(-min(seg, lkv - s) // bs)) for s in range(0, lkv, seg))
+    gk, gv = (torch.randn(b, rows, h, d, device=DEV) for _ in range(2))
+    gk[0, rows - 1, 0, 3] = float("inf")
+    pk, pv = (torch.randn(rank, seg + 2, device=DEV).bfloat16() for _ in range(2))
+    out = torch.zeros(b, lq, h, d, device=DEV)
+    _, lse = bsa_forward(q, k, v, index=index, num=num, block_size=bs, layout="blhd", out=out, want_lse=True)
+    kw = dict(index=index, num=num, block_size=bs, layout="blhd")
+    dt = torch.bfloat16 if bf16 else torch.float32
+    dk, dv = (torch.full((b, lkv, h, d), 7.0, dtype=dt, device=DEV) for _ in range(2))
+    dq, _, _ = bsa_backward(q, k, v, out, lse, do, dk=dk, dv=dv, compressed=(gk, gv, pk, pv, seg, bs), **kw)
+    dq_want, dk_want, dv_want = bsa_backward(q, k, v, out, lse, do, **kw)
+    dk_want, _ = _compress_backward(gk, k, pk, seg, bs, dx=dk_want, out_dtype=dt)
+    dv_want, _ = _compress_backward(gv, v, pv, seg, bs, dx=dv_want, out_dtype=dt)
+    assert torch.equal(dq, dq_want)
+    assert dk_want.isinf().any() and not dk_want[0, :seg].isinf().any() or lkv <= seg
+    for name, got, want in (("dk", dk, dk_want), ("dv", dv, dv_want)):
+        assert got.dtype == want.dtype
+        torch.testing.assert_close(got, want, rtol=0, atol=0, equal_nan=True, msg=lambda m: f"{name}: {m}")
+    assert _compress_backward(gk, k, pk, seg, bs, want_dx=False)[0] is None
+
+
 def test_sparse_backward_many_query_blocks():
     """More than 256 query blocks: the transposed lists come from the scanning kernel instead of the
     counting one."""

@@ -262,6 +262,9 @@ BsaBwdArgs = _struct("wa_bsa_bwd_args", [
     ("dv", c_void_p), ("dv_sb", c_int64), ("dv_st", c_int64), ("dv_sh", c_int64), ("dv_accumulate", c_int32),
     ("workspace", c_void_p),
     ("dkv_dtype", c_int32), ("dq_dtype", c_int32),
+    ("add_k", c_void_p), ("add_v", c_void_p), ("add_sb", c_int64), ("add_st", c_int64), ("add_sh", c_int64),
+    ("proj_k", c_void_p), ("proj_v", c_void_p),
+    ("add_rank", c_int64), ("add_len", c_int64), ("add_segment", c_int64), ("add_block", c_int64),
 ])
 
 Elu1BwdArgs = _struct("wa_elu1_bwd_args", [
@@ -369,6 +372,7 @@ SIGNATURES = {
     "wa_hsa_bwd_workspace_bytes": (c_int64, [c_int64] * 8),
     "wa_hsa_bwd": (c_int, [POINTER(HsaBwdArgs), c_void_p]),
     "wa_bsa_bwd_workspace_bytes": (c_int64, [c_int64] * 6),
+    "wa_bsa_bwd_key_runs": (c_int64, [c_int64] * 5),
     "wa_bsa_bwd": (c_int, [POINTER(BsaBwdArgs), c_void_p]),
     "wa_elu1_bwd_workspace_bytes": (c_int64, [c_int64] * 4),
     "wa_elu1_bwd": (c_int, [POINTER(Elu1BwdArgs), c_void_p]),

@@ -22,6 +22,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "split3.h"
 #include "tile.h"
 
 namespace {
@@ -55,6 +56,11 @@ struct BwdParams {
   // ([parts][dK, dV][B * n_heads][Lkv][D]) one more launch adds up (NULL: the gradients are written)
   float* part_kv;
   int parts;
+  // A second term of dK and dV formed in the dK/dV pass: E^T g of the compression whose rows got the
+  // gradients add_k / add_v (fp32 [B, rows, H, D]), E = proj_k / proj_v (NULL: none)
+  const float* add_k; const float* add_v; int64_t add_sb, add_st, add_sh;
+  const bf16_t* proj_k; const bf16_t* proj_v;
+  int add_seg, add_block, add_rank, add_full, add_len;  // segment, block, E's rows (full segment: add_full), row length
   int4* kv_info;     // [B * n_heads * Nkv] dkdv launch order: per slab, key blocks by descending list
                      // length as {block id, list length, first list entry, 0}
 };
@@ -582,7 +588,7 @@ __global__ void __launch_bounds__(KV_ORDER_T) kv_order_kernel(BwdParams p) {
 // ---------------------------------------------------------------------------------------------
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
-template <int D, int BS>
+template <int D, int BS, bool ADD>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) bwd_dkdv_kernel(BwdParams p) {
   constexpr int KW = DKDV_KEYS, HB = BS / KW, NKG = KW / 32, NW = 2 * NKG, NT = 64 * NW, DC = D / 16, DT = D / 32;
   constexpr int TILE = 64 * D, ST = DKDV_STAGES, LM = DKDV_LIST_MAX;
@@ -634,7 +640,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
     nl = l1 - l0;
     e0 = __builtin_amdgcn_readfirstlane(nl > 0 ? *lst : 0);
   }
-  if (nl == 0 && !p.part_kv) {
+  if (!ADD && nl == 0 && !p.part_kv) {
     // no query block listed this key block: its written gradients are zero (accumulated ones
     // keep their values), with no tile streamed
     const int rows = max(0, min(KW, p.Lkv - kb0));
@@ -795,7 +801,66 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
   }
   // each lane holds its key's row: channels 32 tt + 8 rq + 4 g .. + 3 of tile tt (keys past the
   // block's end get zeros); dK is scaled here
-  const float osc = swave ? 1.f : p.scale;
+  float osc = swave ? 1.f : p.scale;
+  if constexpr (ADD) {
+    // the compression's term, as compress_bwd_dx_kernel forms it (linear.hip): per segment that the
+    // wave's 32 keys touch, sum_j E[j, key] g[row0 + j, channel] with g split in three bf16 parts,
+    // operands straight from L2 (a head's g is ~270 KB), added by the lanes of that segment
+    const float* gr = (swave ? p.add_v : p.add_k) + (int64_t)b * p.add_sb + (int64_t)h * p.add_sh + l32;
+    const bf16_t* pe = swave ? p.proj_v : p.proj_k;
+#pragma unroll
+    for (int tt = 0; tt < DT; ++tt) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[tt][r] = wa_mul_rn(acc[tt][r], osc);
+    }
+    osc = 1.f;
+    const int last = p.Lkv - 1, t = min(kb0 + kl, last), mine = t / p.add_seg;
+    const int s1 = min(kb0 + kg * 32 + 31, last) / p.add_seg;
+    for (int sg = min(kb0 + kg * 32, last) / p.add_seg; sg <= s1; ++sg) {
+      const int start = sg * p.add_seg, n = min(p.add_seg, p.Lkv - start);
+      const int r = min(p.add_rank, (n + p.add_block - 1) / p.add_block);
+      const float* gs0 = gr + (int64_t)sg * p.add_full * p.add_st;
+      const int te = mine == sg ? t - start : 0;
+      f32x16 sum[DT], none = f32x16{};
+#pragma unroll
+      for (int tt = 0; tt < DT; ++tt) sum[tt] = f32x16{};
+      for (int j0 = 0; j0 < r; j0 += 32) {
+        Plain ep[2];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+          bf16x8 eh;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const int jr = j0 + 16 * ks + 8 * g + e;
+            eh[e] = pe[(int64_t)min(jr, r - 1) * p.add_len + te];
+            if (jr >= r) eh[e] = (bf16_t)0.f;
+          }
+          ep[ks] = {eh, finite8(eh)};
+        }
+#pragma unroll
+        for (int tt = 0; tt < DT; ++tt) {
+#pragma unroll
+          for (int ks = 0; ks < 2; ++ks) {
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const int jr = j0 + 16 * ks + 8 * g + e;
+              v[e] = gs0[(int64_t)min(jr, r - 1) * p.add_st + 32 * tt];
+              if (jr >= r) v[e] = 0.f;
+            }
+            mfma_split(split3(v), ep[ks], sum[tt], none);
+          }
+        }
+      }
+      if (mine == sg) {
+#pragma unroll
+        for (int tt = 0; tt < DT; ++tt) {
+#pragma unroll
+          for (int r2 = 0; r2 < 16; ++r2) acc[tt][r2] += sum[tt][r2];
+        }
+      }
+    }
+  }
   if (p.part_kv) {
     const int prow = kb0 + kl;
     if (prow >= p.Lkv) return;
@@ -980,8 +1045,9 @@ int launch_bwd(const BwdParams& bp, hipStream_t s, hipStream_t sq, hipEvent_t fo
     } else {
       kp.kv_info = nullptr;
     }
-    hipLaunchKernelGGL((bwd_dkdv_kernel<D, BS>), dim3((unsigned)(bp.B * nh * bp.Nkv * (BS / DKDV_KEYS) * bp.parts)),
-                       dim3(256), 0, s, kp);
+    const dim3 kgrid((unsigned)(bp.B * nh * bp.Nkv * (BS / DKDV_KEYS) * bp.parts));
+    if (bp.add_k) hipLaunchKernelGGL((bwd_dkdv_kernel<D, BS, true>), kgrid, dim3(256), 0, s, kp);
+    else hipLaunchKernelGGL((bwd_dkdv_kernel<D, BS, false>), kgrid, dim3(256), 0, s, kp);
     if ((rc = wa_launch_status("bsa_bwd_dkdv"))) return joined(rc);
     if (bp.part_kv) {
       const int64_t n = 2 * (int64_t)bp.B * nh * bp.Lkv * (D / 4);
@@ -1007,6 +1073,10 @@ extern "C" int64_t wa_bsa_bwd_workspace_bytes(int64_t B, int64_t n_heads, int64_
   return 2 * align256(B * n_heads * Lq * 4) + align256(B * n_heads * Lq * D * 2) +
          align256(B * n_heads * nkv * nq * 4) + align256(B * n_heads * nkv * 4) + align256(B * n_heads * nkv * 16) +
          part_bytes(B, n_heads, Lq, Lkv, D, block_size);
+}
+
+extern "C" int64_t wa_bsa_bwd_key_runs(int64_t B, int64_t n_heads, int64_t Lq, int64_t Lkv, int64_t block_size) {
+  return dkdv_parts(B, n_heads, Lq, Lkv, block_size);
 }
 
 // wa_bsa_bwd with its dQ pass on a second stream (NULL: one stream), forked from `stream` after the
@@ -1089,6 +1159,22 @@ int wa_bsa_bwd_streams(const wa_bsa_bwd_args* a, void* stream, void* dq_stream, 
   ws += align256(a->B * nh * nkv * 16);
   bp.parts = a->dk && a->dv ? dkdv_parts(a->B, nh, a->Lq, a->Lkv, a->block_size) : 1;
   bp.part_kv = bp.parts > 1 ? (float*)ws : nullptr;
+  if (a->add_k || a->add_v) {
+    WA_CHECK_ARG(a->add_k && a->add_v && a->proj_k && a->proj_v && a->dk && a->dv && !a->dk_accumulate &&
+                     !a->dv_accumulate && !a->block_sizes,
+                 "wa_bsa_bwd: an added term needs both gradients and projections, written dk / dv and no block sizes");
+    WA_CHECK_ARG(bp.parts == 1, "wa_bsa_bwd: no added term where the key lists are cut into runs");
+    const int64_t n_first = std::min(a->add_segment, a->Lkv);
+    WA_CHECK_ARG(a->add_segment > 0 && a->add_block > 0 && a->add_rank > 0 && n_first <= a->add_len &&
+                     a->add_rank * a->add_len <= INT32_MAX,
+                 "wa_bsa_bwd: bad compression sizes");
+    bp.add_k = a->add_k; bp.add_v = a->add_v;
+    bp.add_sb = a->add_sb; bp.add_st = a->add_st; bp.add_sh = a->add_sh;
+    bp.proj_k = (const bf16_t*)a->proj_k; bp.proj_v = (const bf16_t*)a->proj_v;
+    bp.add_seg = (int)n_first; bp.add_block = (int)std::min<int64_t>(a->add_block, INT32_MAX / 2);
+    bp.add_rank = (int)a->add_rank; bp.add_len = (int)a->add_len;
+    bp.add_full = (int)std::min(a->add_rank, (n_first + a->add_block - 1) / a->add_block);
+  }
 
   hipStream_t s = (hipStream_t)stream, sq = (hipStream_t)dq_stream;
   hipEvent_t fe = (hipEvent_t)fork_event, je = (hipEvent_t)join_event;

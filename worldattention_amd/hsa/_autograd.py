@@ -91,13 +91,14 @@ def elu1_backward(q, k, v, dout, state, zsum, heads_t, dq, dk, dv, *, dq_accumul
 # ----------------------------------------------------------------------------------------------
 # low-rank compression (attention.py:64-110) under autograd
 # ----------------------------------------------------------------------------------------------
-def _compress_backward(grad, x, proj, segment_len, block_size, dx=None, out_dtype=torch.float32):
+def _compress_backward(grad, x, proj, segment_len, block_size, dx=None, out_dtype=torch.float32, want_dx=True):
     """Gradients of ``out_seg = E[:r, :len] @ x_seg`` per segment (``wa_compress_kv_bwd``):
     ``dx_seg = E^T dout_seg`` and ``dE[:r, :len] = sum_{b, h} dout_seg x_seg^T``, fp32, for a
     ``[B, L, H, D]`` x and a ``[B, Lc, H, D]`` gradient. ``dx`` (optional): an fp32 ``[B, L, H, D]``
     tensor with unit last stride that the x gradient is added to; otherwise a new one is returned.
     With ``out_dtype`` bf16 the (accumulated) x gradient comes back as a new bf16 tensor, rounded
-    once, and ``dx`` is only read. Returns ``(dx, dproj)``, dproj fp32 of the projection's shape."""
+    once, and ``dx`` is only read. Returns ``(dx, dproj)``, dproj fp32 of the projection's shape (dx
+    None without ``want_dx``)."""
     dev = _lib.require_gpu(x, proj)
     bsz, length, heads, d = x.shape
     seg = segment_len if segment_len > 0 else length
@@ -107,8 +108,12 @@ def _compress_backward(grad, x, proj, segment_len, block_size, dx=None, out_dtyp
     pj = proj if proj.dtype in (torch.float32, torch.bfloat16) else proj.float()
     pj = pj.contiguous()
     accumulate = dx is not None
-    res = torch.empty((bsz, length, heads, d), dtype=torch.bfloat16, device=dev) if out_dtype == torch.bfloat16 else None
-    if dx is None:
+    res = None
+    if want_dx and out_dtype == torch.bfloat16:
+        res = torch.empty((bsz, length, heads, d), dtype=torch.bfloat16, device=dev)
+    if not want_dx:
+        dx, accumulate = None, False
+    elif dx is None:
         dx = torch.empty((bsz, length, heads, d), dtype=torch.float32, device=dev) if res is None else None
     elif dx.dtype != torch.float32 or tuple(dx.shape) != (bsz, length, heads, d) or dx.stride(-1) != 1:
         raise ValueError(f"dx must be float32 {(bsz, length, heads, d)} with unit last stride")
@@ -293,41 +298,55 @@ class _HSA(torch.autograd.Function):
         fresh_q = split or (lowrank and len(plan.linear) == heads)
         fresh_kv = split or (lowrank and len(plan.sparse) == heads)
         dq = (torch.empty if fresh_q else torch.zeros)((bsz, q_len, heads, d), **f32)
-        # dk / dv are written once in their final type when that is bf16 and no compression backward
-        # adds to them (no fp32 buffer, no cast pass)
+        # dk / dv are written once in their final type when that is bf16 and no separate compression
+        # backward adds to them (no fp32 buffer, no cast pass)
         kd, vd = ctx.dtypes[1], ctx.dtypes[2]
         inline = lowrank and not ctx.has_coarse
-        kv_dt = torch.bfloat16 if fresh_kv and not inline and kd == vd == torch.bfloat16 else torch.float32
+        seg = cfg["proj_segment_len"] if cfg["proj_segment_len"] > 0 else kv_len
+        # Keys compressed in the call: where every head is sparse, the dK/dV pass adds the
+        # compression's term E^T g itself and writes the final type (bf16 projections of one shape,
+        # lists not cut into runs). As a pass of its own it read the fp32 gradients back and wrote
+        # bf16 ones: 2 x 118 us at 12 heads, 32,760 keys, D 128, where the dK/dV pass now takes ~75 us
+        # more; the whole step 2650 -> 2490 us.
+        fuse_dx = (inline and fresh_kv and kd == vd and kd in (torch.bfloat16, torch.float32)
+                   and k_proj_mat.dtype == v_proj_mat.dtype == torch.bfloat16 and k_proj_mat.shape == v_proj_mat.shape
+                   and _lib.lib().wa_bsa_bwd_key_runs(bsz, heads, q_len, kv_len, block_size) == 1)
+        kv_dt = torch.float32
+        if fresh_kv and (fuse_dx or not inline) and kd == vd == torch.bfloat16:
+            kv_dt = torch.bfloat16
         alloc = torch.empty if fresh_kv else torch.zeros
         dk = alloc((bsz, kv_len, heads, d), dtype=kv_dt, device=dev)
         dv = alloc((bsz, kv_len, heads, d), dtype=kv_dt, device=dev)
-        dgw = dgb = dkc = dvc = dEk = dEv = None
+        dgw = dgb = dkc = dvc = dEk = dEv = compressed = None
         if plan.linear:
             dlin = torch.empty((bsz, q_len, heads, d), **f32)
             dgw, dgb = fuse_backward(qb, lin, ex["modes_t"], gate, spec, dout, dlin, dq, lin_round=ex["lin_round"],
                                      dq_accumulate=not fresh_q)
+        if lowrank:
+            lt = plan.t["linear"]
+            lc = kcb.shape[1]
+            fresh_c = len(plan.linear) == heads
+            dkc = (torch.empty if fresh_c else torch.zeros)((bsz, lc, heads, d), **f32)
+            dvc = (torch.empty if fresh_c else torch.zeros)((bsz, lc, heads, d), **f32)
+            bsa_backward(qb, kcb, vcb, lin, lse_l, dlin, index=None, num=None,
+                         block_size=_dense_block(d, block_size), layout="blhd", heads=lt, lq=q_len,
+                         lkv=lc, dq=dq, dk=dkc, dv=dvc, accumulate=True, kv_accumulate=not fresh_c,
+                         scale=cfg.get("scale", 0.0))
+            if fuse_dx:
+                compressed = (dkc, dvc, k_proj_mat.contiguous(), v_proj_mat.contiguous(), seg, block_size)
         if plan.sparse:
             bsa_backward(qb, kb, vb, sparse, lse_s, dout, index=index, num=num, block_size=block_size,
                          layout="blhd", heads=plan.t["sparse"], lq=q_len, lkv=kv_len, dq=dq, dk=dk, dv=dv,
-                         accumulate=not split, kv_accumulate=not fresh_kv, scale=cfg.get("scale", 0.0))
-        if plan.linear:
-            lt = plan.t["linear"]
-            if cfg["linear_mode"] == "elu1":
-                elu1_backward(q, k, v, dlin, state, zsum, lt, dq, dk, dv, dq_accumulate=True,
-                              kv_accumulate=not fresh_kv)
-            else:
-                lc = kcb.shape[1]
-                fresh_c = len(plan.linear) == heads
-                dkc = (torch.empty if fresh_c else torch.zeros)((bsz, lc, heads, d), **f32)
-                dvc = (torch.empty if fresh_c else torch.zeros)((bsz, lc, heads, d), **f32)
-                bsa_backward(qb, kcb, vcb, lin, lse_l, dlin, index=None, num=None,
-                             block_size=_dense_block(d, block_size), layout="blhd", heads=lt, lq=q_len,
-                             lkv=lc, dq=dq, dk=dkc, dv=dvc, accumulate=True, kv_accumulate=not fresh_c,
-                             scale=cfg.get("scale", 0.0))
-                if inline:
-                    seg = cfg["proj_segment_len"]
-                    dk, dEk = _compress_backward(dkc, k, k_proj_mat, seg, block_size, dx=dk, out_dtype=kd)
-                    dv, dEv = _compress_backward(dvc, v, v_proj_mat, seg, block_size, dx=dv, out_dtype=vd)
+                         accumulate=not split, kv_accumulate=not fresh_kv, scale=cfg.get("scale", 0.0),
+                         compressed=compressed)
+        if plan.linear and not lowrank:
+            elu1_backward(q, k, v, dlin, state, zsum, plan.t["linear"], dq, dk, dv, dq_accumulate=True,
+                          kv_accumulate=not fresh_kv)
+        if inline:
+            gk, dEk = _compress_backward(dkc, k, k_proj_mat, seg, block_size, dx=dk, out_dtype=kd, want_dx=not fuse_dx)
+            gv, dEv = _compress_backward(dvc, v, v_proj_mat, seg, block_size, dx=dv, out_dtype=vd, want_dx=not fuse_dx)
+            if not fuse_dx:
+                dk, dv = gk, gv
         qd, kd, vd, kcd, vcd, ekd, evd, gwd, gbd = ctx.dtypes
 
         def cast(t, dt):

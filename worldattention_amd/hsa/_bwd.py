@@ -14,7 +14,7 @@ __all__ = ["bsa_backward"]
 
 def bsa_backward(q, k, v, out, lse, grad_out, *, index, num, block_size, block_sizes=None, layout="bhld",
                  heads=None, lq=None, lkv=None, dq=None, dk=None, dv=None, accumulate=False, scale=0.0,
-                 kv_accumulate=None):
+                 kv_accumulate=None, compressed=None):
     """``(dq, dk, dv)`` of :func:`bsa_forward` in ``layout`` (fp32; given buffers may be bf16).
 
     ``out`` is the forward's attention output (fp32 preferred, it sets ``delta``), ``lse`` its
@@ -22,6 +22,10 @@ def bsa_backward(q, k, v, out, lse, grad_out, *, index, num, block_size, block_s
     Given ``dq`` / ``dk`` / ``dv`` buffers are written, or
     added to with ``accumulate`` (fp32 only; ``kv_accumulate``: for ``dk`` / ``dv``, default as
     ``accumulate``); only the heads in ``heads`` (device int32) are touched.
+    ``compressed``: ``(grad_k, grad_v, k_proj, v_proj, segment_len, block_size)`` of keys and values
+    compressed from these (fp32 contiguous [B, rows, H, D] gradients, bf16 contiguous projections of
+    one shape): their gradients' ``E^T g`` is added to written ``dk`` / ``dv`` before the rounding
+    (every head attended to, and no lists cut into runs: ``wa_bsa_bwd_key_runs``).
     """
     dev = _lib.require_gpu(q, k, v, out, grad_out)
     strides = _lib.bhld if layout == "bhld" else _lib.blhd
@@ -62,5 +66,10 @@ def bsa_backward(q, k, v, out, lse, grad_out, *, index, num, block_size, block_s
         bsz, nheads, lq, lkv, d, block_size, float(scale),
         *strides(dq), int(accumulate), *strides(dk), int(kv_accumulate), *strides(dv), int(kv_accumulate),
         ws.data_ptr(), _lib.dtype_code(dk), _lib.dtype_code(dq))
+    if compressed is not None:
+        gk, gv, pk, pv, segment, block = compressed
+        args.add_k, args.add_sb, args.add_st, args.add_sh = _lib.blhd(gk)
+        args.add_v, args.proj_k, args.proj_v = gv.data_ptr(), pk.data_ptr(), pv.data_ptr()
+        args.add_rank, args.add_len, args.add_segment, args.add_block = *pk.shape, segment, block
     _lib.call("wa_bsa_bwd", args, _lib.stream_ptr(dev))
     return dq, dk, dv
