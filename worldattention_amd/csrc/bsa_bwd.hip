@@ -805,7 +805,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
   if constexpr (ADD) {
     // the compression's term, as compress_bwd_dx_kernel forms it (linear.hip): per segment that the
     // wave's 32 keys touch, sum_j E[j, key] g[row0 + j, channel] with g split in three bf16 parts,
-    // operands straight from L2 (a head's g is ~270 KB), added by the lanes of that segment
+    // operands straight from L2 (a head's g is ~270 KB), added by the lanes of that segment. Bound by
+    // the trip to L2 at a workgroup's end: ~95 us of the launch at 12 heads, 32,760 keys with the
+    // loads tile by tile, ~20 with all of them first
     const float* gr = (swave ? p.add_v : p.add_k) + (int64_t)b * p.add_sb + (int64_t)h * p.add_sh + l32;
     const bf16_t* pe = swave ? p.proj_v : p.proj_k;
 #pragma unroll
@@ -825,31 +827,36 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
 #pragma unroll
       for (int tt = 0; tt < DT; ++tt) sum[tt] = f32x16{};
       for (int j0 = 0; j0 < r; j0 += 32) {
+        // every operand of 32 ranks is loaded before the first product (one trip to L2)
+        float gv[DT][2][8];
+        bf16x8 eh[2];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const int64_t jr = min(j0 + 16 * ks + 8 * g + e, r - 1);
+            eh[ks][e] = pe[jr * p.add_len + te];
+#pragma unroll
+            for (int tt = 0; tt < DT; ++tt) gv[tt][ks][e] = gs0[jr * p.add_st + 32 * tt];
+          }
+        }
+        asm volatile("" ::: "memory");
         Plain ep[2];
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-          bf16x8 eh;
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
-            const int jr = j0 + 16 * ks + 8 * g + e;
-            eh[e] = pe[(int64_t)min(jr, r - 1) * p.add_len + te];
-            if (jr >= r) eh[e] = (bf16_t)0.f;
+            if (j0 + 16 * ks + 8 * g + e < r) continue;
+            eh[ks][e] = (bf16_t)0.f;
+#pragma unroll
+            for (int tt = 0; tt < DT; ++tt) gv[tt][ks][e] = 0.f;
           }
-          ep[ks] = {eh, finite8(eh)};
+          ep[ks] = {eh[ks], finite8(eh[ks])};
         }
 #pragma unroll
         for (int tt = 0; tt < DT; ++tt) {
 #pragma unroll
-          for (int ks = 0; ks < 2; ++ks) {
-            float v[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              const int jr = j0 + 16 * ks + 8 * g + e;
-              v[e] = gs0[(int64_t)min(jr, r - 1) * p.add_st + 32 * tt];
-              if (jr >= r) v[e] = 0.f;
-            }
-            mfma_split(split3(v), ep[ks], sum[tt], none);
-          }
+          for (int ks = 0; ks < 2; ++ks) mfma_split(split3(gv[tt][ks]), ep[ks], sum[tt], none);
         }
       }
       if (mine == sg) {
