@@ -701,18 +701,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
     qs.issue(qd, src0, w);
     ds.issue(qd + TILE, src0, w);
     float* stats = (float*)(qd + 2 * TILE);
-    row_stats_dma(stats, p.lse2 + srow + src0, p.Lq - src0, lane);
-    row_stats_dma(stats + 64, p.delta + srow + src0, p.Lq - src0, lane);
+    if (w == 0) row_stats_dma(stats, p.lse2 + srow + src0, p.Lq - src0, lane);
+    if (w == NW - 1) row_stats_dma(stats + 64, p.delta + srow + src0, p.Lq - src0, lane);
   };
   // step t computes on stage t % ST; the loop is unrolled by ST so that every stage is static
   auto step = [&](auto S, int t) {
     constexpr int SV = decltype(S)::value;
     ring_wait<PER>(min(ST - 2, total - 1 - t));
-    if (t + ST - 1 < total) issue(IC<(SV + ST - 1) % ST>{}, t + ST - 1);  // the stage of step t - 1
     const int e = entry(t / QPB);
     const float mult = (float)(e >> 16);
     const int q0r = (e & 0xFFFF) * BS + 64 * (t % QPB);
-    if (q0r >= p.Lq) return;  // uniform over the workgroup
+    if (q0r >= p.Lq) {
+    if (t + ST - 1 < total) issue(IC<(SV + ST - 1) % ST>{}, t + ST - 1);  // the stage of step t - 1
+      return;
+    }
     const bf16_t* qc = stage_of<SV>(qd0, qd1, qd2, qd3);
     const bf16_t* dc = qc + TILE;
     const float* st_lse2 = (const float*)(qc + 2 * TILE);
@@ -728,6 +730,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
 #pragma unroll
       for (int qt = 0; qt < 2; ++qt) sacc[qt] = wa_mfma32(tile_row8<D>(at, qt * 32 + l32, 2 * c + g), kvf[c], sacc[qt]);
     }
+    if (t + ST - 1 < total) issue(IC<(SV + ST - 1) % ST>{}, t + ST - 1);  // the stage of step t - 1
     // P (scaled by multiplicity) to LDS, or dS from the group's P; queries past Lq stream zero Q,
     // dO and statistics rows, so their dS and dO are 0 and they add nothing; keys past the
     // block's end are dropped by the epilogue
