@@ -594,7 +594,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
   constexpr int TILE = 64 * D, ST = DKDV_STAGES, LM = DKDV_LIST_MAX;
   constexpr int QPB = BS / 64;                     // 64-query steps per query block
   using TS = TileStream<D, NW>;
-  constexpr int PER = 2 * TS::NI + 2;              // Q and dO tiles, lse and delta rows
   // stage s: Q tile at [0, TILE), dO tile at [TILE, 2 TILE), then 64 lse and 64 delta floats
   constexpr int SS = 2 * TILE + 256;
   static_assert(ST == 2 && NW == 4, "two ring stages, four waves");
@@ -693,7 +692,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
     return __builtin_amdgcn_readfirstlane(e);
   };
   auto first_query = [&](int t) { return (entry(t / QPB) & 0xFFFF) * BS + 64 * (t % QPB); };
-  // every wave streams the statistics too (identical values), so all waves count the same loads
+  // the first wave streams the lse row too, the last one the delta row: the waves' counts of loads
+  // in flight differ, so a step waits for all of its own (two stages: nothing else is in flight)
   auto issue = [&](auto S, int t) {
     bf16_t* qd = stage_of<decltype(S)::value>(qd0, qd1, qd2, qd3);
     const int q0r = first_query(t);
@@ -704,15 +704,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
     if (w == 0) row_stats_dma(stats, p.lse2 + srow + src0, p.Lq - src0, lane);
     if (w == NW - 1) row_stats_dma(stats + 64, p.delta + srow + src0, p.Lq - src0, lane);
   };
-  // step t computes on stage t % ST; the loop is unrolled by ST so that every stage is static
+  // step t computes on stage t % ST; the loop is unrolled by ST so that every stage is static. The
+  // next step's tiles are issued behind the first products: ahead of them, and with every wave
+  // streaming both statistics rows, a training step of 12 heads and 32,760 keys took 2,445 us
+  // against 2,402
   auto step = [&](auto S, int t) {
     constexpr int SV = decltype(S)::value;
-    ring_wait<PER>(min(ST - 2, total - 1 - t));
+    ring_wait<0>(0);
     const int e = entry(t / QPB);
     const float mult = (float)(e >> 16);
     const int q0r = (e & 0xFFFF) * BS + 64 * (t % QPB);
-    if (q0r >= p.Lq) {
-    if (t + ST - 1 < total) issue(IC<(SV + ST - 1) % ST>{}, t + ST - 1);  // the stage of step t - 1
+    if (q0r >= p.Lq) {  // uniform over the workgroup
+      if (t + ST - 1 < total) issue(IC<(SV + ST - 1) % ST>{}, t + ST - 1);
       return;
     }
     const bf16_t* qc = stage_of<SV>(qd0, qd1, qd2, qd3);
