@@ -130,3 +130,16 @@ def test_empty_head_lists_are_refused_at_the_c_boundary():
     assert _lib.heads_arg(None) == (None, 0)
     t = torch.tensor([1, 3], dtype=torch.int32)
     assert _lib.heads_arg(t) == (t.data_ptr(), 2)
+
+
+@pytest.mark.parametrize("q_len,kv_len,batch", [(0, 64, 1), (64, 0, 1), (64, 64, 0), (1, 1, 1)])
+def test_empty_calls_keep_the_composed_forward(q_len, kv_len, batch):
+    """The one-call forward refuses empty tensors, so a call without queries, keys or batch entries
+    goes to the composed entry points, which decide about it as they always did."""
+    q = torch.zeros(batch, q_len, 2, 64)
+    k = v = torch.zeros(batch, kv_len, 2, 64)
+    proj = torch.zeros(1, 64)
+    plan = WA.head_plan(2, None, "cpu")
+    for mode in ("lowrank", "elu1"):
+        want = q.numel() > 0 and k.numel() > 0
+        assert WA.one_call_eligible(q, k, v, None, None, proj, proj, plan, mode) is want

@@ -502,11 +502,11 @@ def _native_split_forward(q, k, v, plan, ks, gate, lin_round, block_size, q_len,
 
 
 def one_call_eligible(q, k, v, k_coarse, v_coarse, k_proj_mat, v_proj_mat, plan, linear_mode) -> bool:
-    """Whether ``wa_hsa_fwd_any`` covers this forward: q, k and v of one type, fp32 or bf16, with
+    """Whether ``wa_hsa_fwd_any`` covers this forward: q, k and v of one type, fp32 or bf16, not empty, with
     contiguous channels, and (for the low-rank branch) coarse caches or projections as its kernels take
     them. Anything else runs the composed entry points from Python, which convert first."""
     types = (torch.float32, torch.bfloat16)
-    if not ONE_CALL or q.shape[0] == 0 or q.dtype not in types or not q.dtype == k.dtype == v.dtype:
+    if not ONE_CALL or q.numel() == 0 or k.numel() == 0 or q.dtype not in types or not q.dtype == k.dtype == v.dtype:
         return False
     if any(t.stride(-1) != 1 for t in (q, k, v)):
         return False
