@@ -624,6 +624,32 @@ def test_bsa_long_rows_rank_ranges_match_oracle(case, b, h, nq):
         assert torch.equal(plain, table)
 
 
+@pytest.mark.parametrize("d,bs,split", [(64, 64, 16), (128, 64, 64), (64, 128, 16), (128, 128, 16), (128, 128, 32)])
+@pytest.mark.parametrize("visits", [(1, 16, 33), (48, 63, 64), (5, 65, 80)])
+def test_bsa_unit_tables_equal_the_table_free_launch(d, bs, split, visits):
+    """A unit table whose rows need at most 64 visits runs the kernel instance without rank ranges,
+    longer ones (65, 80) the general one: each gives the bits of the launch without a table (the
+    general instance), which the oracle checks. Rows of both sides of one unit and of 64 visits,
+    partial last blocks."""
+    from worldattention_amd.hsa.block_sparse import bsa_forward
+    torch.manual_seed(d + bs + split)
+    b, h, nq, nkv = 2, len(visits), 3, 81
+    lq, lkv = nq * bs - 7, nkv * bs - 13
+    q, k, v = (torch.randn(b, n, h, d).bfloat16() for n in (lq, lkv, lkv))
+    index = torch.stack([torch.randperm(nkv) for _ in range(b * h * nq)]).view(b, h, nq, nkv).int()
+    num = torch.tensor(visits, dtype=torch.int32).view(1, h, 1).expand(b, h, nq).contiguous()
+    args = dict(index=index.to(DEV), num=num.to(DEV), block_size=bs, layout="blhd", lq=lq, lkv=lkv, split=split,
+                out_dtype=torch.float32, want_lse=True)
+    plain, plain_lse = bsa_forward(q.to(DEV), k.to(DEV), v.to(DEV), **args)
+    table, table_lse = bsa_forward(q.to(DEV), k.to(DEV), v.to(DEV), visits=visits, **args)
+    assert torch.equal(table, plain) and torch.equal(table_lse, plain_lse)
+    qp = O.pad_to_len(q, nq * bs).transpose(1, 2)
+    kp, vp = (O.pad_to_len(t, nkv * bs).transpose(1, 2) for t in (k, v))
+    sizes = O.variable_block_sizes(lkv, nkv * bs, bs)
+    want = O.block_sparse_attention(qp.float(), kp.float(), vp.float(), index, num, sizes, bs).transpose(1, 2)[:, :lq]
+    assert_close(table, want, what=f"unit table {visits}")
+
+
 _ANY_CALLS = [  # dtype, d, block, routing, linear mode, head modes, keys, coarse, misaligned
     ("float32", 64, 64, "topk", "elu1", "SL", None, None, False),
     ("float32", 128, 64, "gini", "lowrank", "BBB", None, None, False),

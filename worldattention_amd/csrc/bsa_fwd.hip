@@ -432,7 +432,11 @@ __device__ __forceinline__ bool pipe_check(const float (&rs)[QT]) {
 // KS = 2 (64-key blocks): each query tile gets two waves, one per 32-key half of every step, which
 // share the K / V tiles and meet through LDS after the loop; a 64-query workgroup is then four
 // waves, so its two workgroups per CU (the LDS ring allows two) give each SIMD two waves.
-template <int D, int BS, int QT, int KS>
+// TABLE: the launch's units come from a table and no row it lists needs more than 64 visits (top-k
+// budgets). Such a unit is a few microseconds long and its prologue a chain of cold instruction
+// fetches: the code of the rank ranges, 1,100 instructions that it only jumps over, and their
+// list loads cost a call of 8 + 4 split heads (4,680 x 32,760, 8-32 of 256 128-key blocks) 0.7 of 121.4 us.
+template <int D, int BS, int QT, int KS, bool TABLE>
 __global__ void __launch_bounds__(2 * BS / QT * KS) __attribute__((amdgpu_waves_per_eu(QT == 1 ? 2 : 1)))
 bsa_unit_kernel(FwdParams p) {
   constexpr int NW = BS / (32 * QT);  // query waves
@@ -447,7 +451,7 @@ bsa_unit_kernel(FwdParams p) {
   __shared__ __attribute__((aligned(1024))) bf16_t vs0[TILE];
   __shared__ __attribute__((aligned(1024))) bf16_t vs1[TILE];
   __shared__ int steptab[NWT][64][2];
-  __shared__ uint32_t s_bits[64];  // listed block ids of a long row
+  __shared__ uint32_t s_bits[TABLE ? 1 : 64];  // listed block ids of a long row
 
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 5, l32 = lane & 31;
@@ -458,7 +462,7 @@ bsa_unit_kernel(FwdParams p) {
   const int hmap = p.heads && lane < min(p.n_heads, 64) ? p.heads[lane] : 0;
   int64_t row;
   int split;
-  if (p.units) {
+  if (TABLE || p.units) {
     const int u = wa_xcd_remap(blockIdx.x, p.n_units);
     row = p.units[2 * u];
     split = p.units[2 * u + 1];
@@ -483,7 +487,7 @@ bsa_unit_kernel(FwdParams p) {
   int j0 = 0, e0 = 0, e1 = 0;
   if (p.index) {
     if (lane < min((int)p.index_width, 64)) j0 = lrow[lane];
-    if (p.index_width > 64) {
+    if (!TABLE && p.index_width > 64) {
       if (tid < p.index_width) e0 = lrow[tid];
       if (tid + NTH < p.index_width) e1 = lrow[tid + NTH];
     }
@@ -526,17 +530,19 @@ bsa_unit_kernel(FwdParams p) {
   // at B 1, H 12, D 128,
   // Lq 4680, Lkv 32760, ~180 of 512 blocks a row, the launch took 617 us with slices, 452 us with
   // rank ranges of at most 48 blocks and 429 us with 64.
-  // Ids listed twice (or more blocks than 2,048, or a list cut off by max_visits) keep the slices.
+  // Ids listed twice (or more blocks than 2,048, or a list cut off by max_visits) keep the slices,
+  // as does a row that lists more than its unit table planned.
   const bool whole = n <= 64;
   int lo = whole ? 0 : s_begin;
   int take = whole ? n : s_end - s_begin;
   int my_j = 0;
-  bool ranked = !p.index && !whole && (int64_t)ns * p.split >= n;  // a dense row lists block i at position i
+  // a dense row lists block i at position i
+  bool ranked = !TABLE && !p.index && !whole && (int64_t)ns * p.split >= n;
   if (ranked) {
     lo = (int)((int64_t)n * split / ns);
     take = (int)((int64_t)n * (split + 1) / ns) - lo;
   }
-  if (p.index && !whole && p.Nkv <= 2048 && (int64_t)ns * p.split >= n) {  // uniform over the workgroup
+  if (!TABLE && p.index && !whole && p.Nkv <= 2048 && (int64_t)ns * p.split >= n) {  // uniform over the workgroup
     if (tid < 64) s_bits[tid] = 0;
     __syncthreads();
     for (int i = tid; i < n; i += NTH) {
@@ -1099,14 +1105,19 @@ int launch(const FwdParams& fp, int64_t rows, bool cleared, bool key_split, hipS
   // visits per row); a short unit (the dense launch over ~9 compressed key blocks) does better
   // with its two waves' pipelined loop (57 against 62 us).
   constexpr int QT = 1;
+  // at most 64 visits a row, the kernel's whole-list form: the leaner instance (see there)
+  const bool table = fp.units && (int64_t)fp.max_splits * fp.split <= 64;
+  auto unit = [&](auto ks) {
+    constexpr int KS = decltype(ks)::value;
+    const dim3 grid(fp.n_units), block(2 * BS / QT * KS);
+    if (table) hipLaunchKernelGGL((bsa_unit_kernel<D, BS, QT, KS, true>), grid, block, 0, stream, fp);
+    else hipLaunchKernelGGL((bsa_unit_kernel<D, BS, QT, KS, false>), grid, block, 0, stream, fp);
+    return wa_launch_status("bsa_fwd_unit");
+  };
   if constexpr (BS == 64) {
-    if (key_split) {
-      hipLaunchKernelGGL((bsa_unit_kernel<D, BS, QT, 2>), dim3(fp.n_units), dim3(4 * BS / QT), 0, stream, fp);
-      return wa_launch_status("bsa_fwd_unit");
-    }
+    if (key_split) return unit(std::integral_constant<int, 2>{});
   }
-  hipLaunchKernelGGL((bsa_unit_kernel<D, BS, QT, 1>), dim3(fp.n_units), dim3(2 * BS / QT), 0, stream, fp);
-  return wa_launch_status("bsa_fwd_unit");
+  return unit(std::integral_constant<int, 1>{});
 }
 
 // Workspace layout: the split partials (fp32 [rows * max_splits][BS][D] outputs, then
