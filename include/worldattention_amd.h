@@ -329,7 +329,9 @@ int wa_hsa_fwd(const wa_hsa_fwd_args* args, void* stream);
  * the attention kernels' bf16 operands are copied into the workspace where they cannot be read in
  * place. sparse_heads: both_heads and sparse_only_heads in ascending order; every head of the three
  * lists writes o. routing: WA_ROUTE_GINI (tau_min, tau_span) or WA_ROUTE_TOPK (head_k, and unit tables
- * of the two sparse launches with their largest visit counts); split_visits as in wa_bsa_fwd.
+ * of the two sparse launches with their largest visit counts); split_visits as in wa_bsa_fwd, of the
+ * sparse-only heads' launch and, unless split_both is set, of the both heads' one (a unit table is cut
+ * by its own launch's).
  * held (optional): key block sums (held_sums) or means, [B, H, held_blocks, D] fp32, as wa_route takes
  * them. kc / vc (optional): compressed keys and values of lc rows; otherwise k_proj / v_proj compress
  * k and v in segments of segment_len. side_stream and events as in wa_hsa_fwd, used when both branches
@@ -362,6 +364,7 @@ typedef struct wa_hsa_any_args {
   int32_t gate_pre_bf16, gate_out_bf16, lin_round_bf16;
   void* workspace;
   void* side_stream; void* fork_event; void* join_event;
+  int64_t split_both;
 } wa_hsa_any_args;
 int64_t wa_hsa_fwd_any_workspace_bytes(const wa_hsa_any_args* args);
 int wa_hsa_fwd_any(const wa_hsa_any_args* args, void* stream);

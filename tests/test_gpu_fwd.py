@@ -714,6 +714,28 @@ def test_one_call_forward_equals_the_composed_entry_points(call, b, lq, lkv, mon
             assert torch.equal(replayed, want)
 
 
+@pytest.mark.parametrize("modes", ["SSSSSB", "SBBBBB"])
+def test_one_call_forward_splits_each_sparse_launch_like_the_composed_path(modes, monkeypatch):
+    """Gini routing over 64-key blocks with 260 rows in one sparse launch and 52 in the other: the
+    rows' ~112 visits make two units of up to 64 visits there and three of up to 48 here, in the
+    one call as in the composed path (bit for bit)."""
+    torch.manual_seed(len(modes))
+    h, d, bs, lq, lkv = len(modes), 64, 64, 52 * 64, 320 * 64
+    q, k, v = (torch.randn(1, n, h, d, device=DEV).bfloat16() for n in (lq, lkv, lkv))
+    proj = torch.rand(20, 1280, device=DEV).bfloat16() / 40
+    kw = dict(k_coarse=None, v_coarse=None, k_proj_mat=proj, v_proj_mat=proj, gate_lin=None, block_size=bs, tau_min=0.35,
+              tau_max=1.0, proj_segment_len=1280, routing="gini", topk=None,
+              head_modes=[{"B": "both", "S": "sparse"}[m] for m in modes], linear_mode="lowrank")
+    with torch.no_grad():
+        monkeypatch.setattr(WA, "ONE_CALL", False)
+        save = {}
+        want = WA.hsa_forward(q, k, v, save=save, **kw)
+        num = save["route"].num.float().mean().item()
+        assert 97 <= num <= 128, num
+        monkeypatch.setattr(WA, "ONE_CALL", True)
+        assert torch.equal(WA.hsa_forward(q, k, v, **kw), want)
+
+
 def test_hsa_forward_graph_replays_equal_eager_calls():
     """The cfg 2 call captured in a HIP graph (as bench.py times it): every replay, with eager work
     and synchronizations between replays, equals the eager call bit for bit."""

@@ -217,6 +217,7 @@ HsaAnyArgs = _struct("wa_hsa_any_args", [
     ("gate_pre_bf16", c_int32), ("gate_out_bf16", c_int32), ("lin_round_bf16", c_int32),
     ("workspace", c_void_p),
     ("side_stream", c_void_p), ("fork_event", c_void_p), ("join_event", c_void_p),
+    ("split_both", c_int64),
 ])
 
 HsaBwdArgs = _struct("wa_hsa_bwd_args", [

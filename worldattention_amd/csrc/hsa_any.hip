@@ -74,7 +74,7 @@ struct View {
 };
 
 struct Plan {
-  int64_t nq, nkv, lc, dense_block, rows_only, rows_both, split;
+  int64_t nq, nkv, lc, dense_block, rows_only, rows_both, split_only, split_both;
   bool linear_side;  // the linear branch runs beside a sparse branch
   // workspace offsets
   int64_t q, k, v, kc, vc, qp, kp, index, num, thresholds, route, arrivals, lin, bsa_only, bsa_both, dense_only,
@@ -104,7 +104,8 @@ Plan make_plan(const wa_hsa_any_args* a) {
   p.nkv = (a->Lkv + bs - 1) / bs;
   p.rows_only = a->B * a->n_sparse_only * p.nq;
   p.rows_both = a->B * a->n_both * p.nq;
-  p.split = a->split_visits;
+  p.split_only = a->split_visits;
+  p.split_both = a->split_both > 0 ? a->split_both : a->split_visits;
   p.linear_side = n_sparse > 0 && n_linear > 0;
   const bool attends = n_sparse > 0 || (n_linear > 0 && lowrank(a));  // some launch reads bf16 q
   int64_t o = 0;
@@ -125,8 +126,8 @@ Plan make_plan(const wa_hsa_any_args* a) {
     p.route = a->routing == WA_ROUTE_GINI ? take(wa_route_workspace_bytes(a->B, a->H, p.nq, p.nkv)) : 0;
     p.arrivals = take((p.rows_only + p.rows_both) * 4);
     const int64_t mv_only = a->units_only ? a->max_visits_only : p.nkv, mv_both = a->units_both ? a->max_visits_both : p.nkv;
-    if (a->n_sparse_only > 0) p.bsa_only = take(wa_bsa_fwd_workspace_bytes(p.rows_only, mv_only, p.split, bs, D));
-    if (a->n_both > 0) p.bsa_both = take(wa_bsa_fwd_workspace_bytes(p.rows_both, mv_both, p.split, bs, D));
+    if (a->n_sparse_only > 0) p.bsa_only = take(wa_bsa_fwd_workspace_bytes(p.rows_only, mv_only, p.split_only, bs, D));
+    if (a->n_both > 0) p.bsa_both = take(wa_bsa_fwd_workspace_bytes(p.rows_both, mv_both, p.split_both, bs, D));
   }
   if (n_linear > 0) {
     if (a->n_both > 0) p.lin = take(a->B * a->Lq * a->H * D * es);
@@ -253,7 +254,7 @@ int run_sparse(const wa_hsa_any_args* a, const Plan& p, char* ws, const View& q,
   f.workspace = ws + (both ? p.bsa_both : p.bsa_only);
   f.units = both ? a->units_both : a->units_only; f.n_units = both ? a->n_units_both : a->n_units_only;
   f.max_visits = f.units ? (both ? a->max_visits_both : a->max_visits_only) : p.nkv;
-  f.split_visits = (int32_t)p.split;
+  f.split_visits = (int32_t)(both ? p.split_both : p.split_only);
   f.arrivals = (int32_t*)(ws + p.arrivals) + (both ? p.rows_only : 0);
   return wa_bsa_fwd(&f, s);
 }
@@ -282,7 +283,8 @@ int check_args(const wa_hsa_any_args* a) {
   WA_CHECK_ARG(!lowrank(a) || a->n_both + a->n_linear_only == 0 ||
                    (a->kc ? a->lc > 0 && a->lc < (1 << 30) : a->k_proj && a->v_proj && a->proj_rank > 0 && a->proj_len > 0),
                "wa_hsa_fwd_any: the low-rank branch needs coarse keys and values or their projections");
-  WA_CHECK_ARG(a->split_visits >= 0 && a->split_visits <= 64, "wa_hsa_fwd_any: bad split");
+  WA_CHECK_ARG(a->split_visits >= 0 && a->split_visits <= 64 && a->split_both >= 0 && a->split_both <= 64,
+               "wa_hsa_fwd_any: bad split");
   WA_CHECK_ARG((a->units_only == nullptr || a->max_visits_only > 0) && (a->units_both == nullptr || a->max_visits_both > 0),
                "wa_hsa_fwd_any: a unit table needs its largest visit count");
   WA_CHECK_ARG(a->held == nullptr || a->held_blocks >= (a->Lkv + a->block_size - 1) / a->block_size,

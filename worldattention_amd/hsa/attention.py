@@ -536,19 +536,18 @@ def _one_call_forward(q, k, v, plan, out, gate, lin_round, *, k_coarse, v_coarse
             setattr(args, "n_" + name, plan.t[name].numel())
     if plan.sparse:
         args.sparse_heads = plan.t["sparse"].data_ptr()
-        args.split_visits = _lib.bsa_default_split(block_size)
+        # each sparse launch's split is its own (the composed path's, launch by launch)
+        args.split_visits, args.split_both = (default_split(block_size, bsz * len(hl) * nq, routing == "gini")
+                                              for hl in (plan.sparse_only, plan.both))
         if routing == "gini":
             args.routing, args.tau_min, args.tau_span = _lib.WA_ROUTE_GINI, tau_min, tau_max - tau_min
-            # both sparse launches take one split: the larger one's
-            rows = bsz * max(len(plan.sparse_only), len(plan.both)) * nq
-            args.split_visits = default_split(block_size, rows, True)
         else:
             ks = _per_head_k(topk, heads)
             args.routing, args.tau_span, args.head_k = _lib.WA_ROUTE_TOPK, 1.0, _lib.head_list(ks, dev).data_ptr()
-            for name, hl in (("only", plan.sparse_only), ("both", plan.both)):
+            for name, hl, split in (("only", plan.sparse_only, args.split_visits), ("both", plan.both, args.split_both)):
                 if hl:
                     vis = [max(0, min(ks[h], nkv)) for h in hl]
-                    units, n_units = unit_table(bsz, vis, nq, args.split_visits, dev)
+                    units, n_units = unit_table(bsz, vis, nq, split, dev)
                     setattr(args, "units_" + name, units.data_ptr())
                     setattr(args, "n_units_" + name, n_units)
                     setattr(args, "max_visits_" + name, max(max(vis), 1))
