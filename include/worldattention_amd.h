@@ -625,7 +625,8 @@ typedef struct wa_hkv_summary_args {
 int64_t wa_hkv_summary_workspace_bytes(int64_t B, int64_t n_seg, int64_t C, int64_t max_seg_tokens);
 int wa_hkv_page_summary(const wa_hkv_summary_args* args, void* stream);
 
-/* Page scoring and selection (with `scores`, more than 32 pages are scored by a launch of their own):
+/* Page scoring and selection (with `scores`, more than 128 pages or WA_HKV_ONE_LAUNCH_VALUES index
+ * values are scored by a launch of their own, which is faster):
  *   scores[p] = (index[p] . query) / scale   (no division when scale <= 0), p < n_pages <= 4096,
  * then the k highest in descending order, the lower page index first among equal scores (NaN
  * ranks highest), into sel (int32) and sel_scores. Pages with mask[p] != 0 (device uint8,
@@ -633,6 +634,7 @@ int wa_hkv_page_summary(const wa_hkv_summary_args* args, void* stream);
  * Replaces score_pages + select_topk_pages (pipeline/hkv/retrieval.py:75-89, 105-126) and the
  * stage-1 cosine ranking select_top_chunks (retrieval.py:92-102, scale = 0). */
 #define WA_HKV_MAX_PAGES 4096
+#define WA_HKV_ONE_LAUNCH_VALUES 98304
 typedef struct wa_hkv_topk_args {
   const float* index; int64_t index_stride;   /* [n_pages][dim] fp32 */
   const float* query;                          /* [dim] fp32 */

@@ -135,7 +135,7 @@ def test_single_segment_means_over_fine_splits(tokens, dim):
 
 @pytest.mark.parametrize("n_pages", [32, 33, 500])
 def test_scores_alone_and_with_the_selection_are_the_same_bits(n_pages):
-    """Up to 32 pages are scored by the selecting workgroup, more by a launch of their own."""
+    """Few pages are scored by the selecting workgroup, more by a launch of their own."""
     torch.manual_seed(n_pages)
     index, query = torch.randn(n_pages, 1000, device=DEV), torch.randn(1000, device=DEV)
     scores = W.score_pages(query, index)
@@ -143,6 +143,20 @@ def test_scores_alone_and_with_the_selection_are_the_same_bits(n_pages):
     assert torch.equal(scores, alone)
     sel, top = W.select_pages(index, query, 5)
     assert torch.equal(top, torch.topk(scores, 5).values) and torch.equal(scores[sel.long()], top)
+
+
+@pytest.mark.parametrize("pages,dim", [(64, 1536), (65, 1536), (128, 200), (129, 200), (2, 49153)])
+def test_selection_on_both_sides_of_the_one_launch_rule(pages, dim):
+    """Pages scored inside the selection launch and by a launch of their own: the same selection and
+    scores, which equal each page scored alone bit for bit; without the scores as well."""
+    torch.manual_seed(pages + dim)
+    index, query = torch.randn(pages, dim, device=DEV), torch.randn(dim, device=DEV)
+    alone = torch.cat([W.score_pages(query, index[i:i + 1]) for i in range(pages)])
+    k = min(5, pages)
+    for want in (True, False):
+        sel, top, scores = _ops.score_topk(index, query, k, scale=math.sqrt(dim), want_scores=want)
+        assert torch.equal(scores, alone) if want else scores is None
+        assert torch.equal(top, torch.topk(alone, k).values) and torch.equal(alone[sel.long()], top)
 
 
 @pytest.mark.parametrize("pages,dim,k", [(120, 1536, 8), (1, 64, 1), (4096, 256, 33), (777, 100, 777)])

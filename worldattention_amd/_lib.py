@@ -312,6 +312,7 @@ HkvSummaryArgs = _struct("wa_hkv_summary_args", [
 ])
 
 HKV_MAX_PAGES = 4096
+HKV_ONE_LAUNCH_PAGES, HKV_ONE_LAUNCH_VALUES = 128, 98304
 
 HkvTopkArgs = _struct("wa_hkv_topk_args", [
     ("index", c_void_p), ("index_stride", c_int64),

@@ -259,9 +259,8 @@ __global__ void __launch_bounds__(256) summary_reduce_kernel(SumParams p, float*
 }
 
 // =============================================================================================
-// Score + top-k: one wave per page forms the scores (in a launch of their own for more than 32 pages,
-// if the caller takes them: one workgroup's 16 waves took 67 us for 120 pages x 1,536 channels,
-// 11 us in two launches), then one workgroup of 1024 threads selects. Keys are (order-preserving score bits, inverted
+// Score + top-k: one wave per page forms the scores (in a launch of their own past 128 pages or
+// WA_HKV_ONE_LAUNCH_VALUES index values, if the caller takes them), then one workgroup of 1024 threads selects. Keys are (order-preserving score bits, inverted
 // page index), sorted descending with a bitonic network in LDS; key 0 marks masked / padding.
 // =============================================================================================
 struct TopkParams {
@@ -551,7 +550,10 @@ extern "C" int wa_hkv_score_topk(const wa_hkv_topk_args* a, void* stream) {
   WA_CHECK_ARG(a->k >= 1 && a->k <= a->n_pages, "wa_hkv_score_topk: k=%lld outside [1, n_pages]", (long long)a->k);
   TopkParams p{a->index, a->index_stride, a->query, (int)a->n_pages, (int)a->dim, a->scale, a->mask,
                (int)a->k, a->scores, a->sel, a->sel_scores};
-  if (a->scores && a->n_pages > 32) {
+  // One workgroup's 16 waves form the scores of 64 pages x 1,536 channels or 120 x 256 in about what
+  // the call costs the host (GPU 12.6 and 13.5 us against 8.4 and 9.5 in two launches, whose call takes
+  // the host 17 us against 12.5); 120 x 1,536: 19 us in one launch, 9.7 in two.
+  if (a->scores && (a->n_pages > 128 || a->n_pages * a->dim > WA_HKV_ONE_LAUNCH_VALUES)) {
     score_kernel<<<(unsigned)((a->n_pages + 3) / 4), 256, 0, (hipStream_t)stream>>>(p);
     const int rc = wa_launch_status("score_kernel");
     if (rc != WA_OK) return rc;

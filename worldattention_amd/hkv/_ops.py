@@ -134,10 +134,12 @@ def score_topk(index: torch.Tensor, query: torch.Tensor, k: int, *, scale: float
         mask = mask.to(device=dev, dtype=torch.uint8).contiguous()
     sel = torch.empty((k,), dtype=torch.int32, device=dev)
     sel_scores = torch.empty((k,), dtype=torch.float32, device=dev)
-    scores = torch.empty((n_pages,), dtype=torch.float32, device=dev)
+    # (few pages are scored and selected in one launch, which needs no scores)
+    scored_first = n_pages > _lib.HKV_ONE_LAUNCH_PAGES or n_pages * dim > _lib.HKV_ONE_LAUNCH_VALUES
+    scores = torch.empty((n_pages,), dtype=torch.float32, device=dev) if want_scores or scored_first else None
     args = _lib.HkvTopkArgs(index.data_ptr(), index.stride(0), query.data_ptr(), n_pages, dim,
                             float(scale) if scale and scale > 0 else 0.0, _lib.ptr(mask), int(k),
-                            scores.data_ptr(), sel.data_ptr(), sel_scores.data_ptr())
+                            _lib.ptr(scores), sel.data_ptr(), sel_scores.data_ptr())
     _lib.call("wa_hkv_score_topk", ctypes.byref(args), _lib.stream_ptr(dev))
     return sel, sel_scores, scores if want_scores else None
 
