@@ -384,6 +384,72 @@ def test_hsa_reference_mode_gradients_match_oracle():
         assert_close(g, r, *tol, what=name)
 
 
+_LOWRANK_TRAINING = [  # dtype, d, head modes, lq, lkv, coarse caches given, runs of a key list > 1
+    ("bfloat16", 128, "BBB", 200, 700, False, False),    # written bf16 dK / dV with the compression's term added
+    ("bfloat16", 128, "BBB", 1100, 330, False, True),    # lists in runs: the term by its own pass, from fp32
+    ("float32", 64, "BB", 1100, 330, False, True),
+    ("float32", 128, "SBB", 200, 700, False, False),     # every head sparse, not every one linear
+    ("bfloat16", 64, "BLB", 200, 330, False, False),     # every head linear, not every one sparse
+    ("bfloat16", 128, "BSL", 300, 700, False, False),    # neither: everything accumulated
+    ("bfloat16", 64, "SL", 1100, 330, False, True),
+    ("bfloat16", 128, "BB", 200, 700, True, False),      # given coarse keys and values
+    ("float32", 64, "SBL", 1100, 330, True, True),
+]
+
+
+@pytest.mark.parametrize("case", _LOWRANK_TRAINING, ids=lambda c: "-".join(str(x) for x in c))
+def test_hsa_lowrank_gradients_match_oracle(case):
+    """Training of the low-rank configuration in every form its backward distinguishes: outputs and
+    gradients of q, k, v, the projections (or the coarse caches) and the gate against fp32 autograd
+    through the oracle. bf16 operands, probabilities, their gradients and results carry up to 2^-9
+    a rounding; five of them are within 1e-2 of a tensor's norm. Memory the backward allocates holds
+    NaN, so that a gradient nobody wrote shows."""
+    from worldattention_amd import _lib
+    dtype, d, modes, lq, lkv, coarse, runs = case
+    torch.manual_seed(lq + lkv + d)
+    dt, h, bs, seg = getattr(torch, dtype), len(modes), 64, 156
+    n_sparse = sum(m != "L" for m in modes)
+    assert (_lib.lib().wa_bsa_bwd_key_runs(1, n_sparse, lq, lkv, bs) > 1) == runs
+    leaves = {n: torch.randn(1, length, h, d).to(dt).float() for n, length in (("q", lq), ("k", lkv), ("v", lkv))}
+    proj = {n: (torch.randn(3, seg) / 16).bfloat16().float() for n in ("pk", "pv")}
+    if coarse:
+        lc = sum(min(3, -(-min(seg, lkv - s) // bs)) for s in range(0, lkv, seg))
+        leaves.update((n, torch.randn(1, lc, h, d).to(dt).float()) for n in ("kc", "vc"))
+    else:
+        leaves.update(proj)
+    leaves.update(w=torch.randn(d, d) * 0.1, bias=torch.randn(d) * 0.1)
+    do = torch.randn(1, lq, h, d).to(dt).float()
+    kw = dict(block_size=bs, routing="gini", linear_mode="lowrank", proj_segment_len=seg,
+              head_modes=[{"B": "both", "S": "sparse", "L": "linear"}[m] for m in modes])
+
+    want = {n: t.clone().requires_grad_() for n, t in leaves.items()}
+    ref = {n: want[n].to(dt) for n in ("q", "k", "v")}
+    extra = {a: want[n].to(dt) for a, n in (("k_coarse", "kc"), ("v_coarse", "vc"))} if coarse else {}
+    out_r = O.hsa_attention(*ref.values(), k_proj_mat=want.get("pk"), v_proj_mat=want.get("pv"), gate_weight=want["w"],
+                            gate_bias=want["bias"], **extra, **kw)
+    out_r.float().backward(do)
+
+    lin = torch.nn.Linear(d, d).to(DEV)
+    with torch.no_grad():
+        lin.weight.copy_(leaves["w"])
+        lin.bias.copy_(leaves["bias"])
+    types = dict(pk=torch.bfloat16, pv=torch.bfloat16)
+    got = {n: t.to(DEV, types.get(n, dt)).requires_grad_() for n, t in leaves.items() if n not in ("w", "bias")}
+    extra = dict(k_coarse=got["kc"], v_coarse=got["vc"]) if coarse else {}
+    pk, pv = (got[n] if n in got else proj[n].to(DEV, torch.bfloat16) for n in ("pk", "pv"))
+    out_g = W.hsa_attention(got["q"], got["k"], got["v"], k_proj_mat=pk, v_proj_mat=pv, gate_lin=lin, **extra, **kw)
+    for _ in range(2):  # every block the caching allocator hands to the backward held NaN
+        junk = [torch.full((n,), float("nan"), device=DEV) for t in got.values() for n in (t.numel(), t.numel() // 2) * 4]
+        del junk
+    out_g.backward(do.to(DEV, out_g.dtype))
+    grads = {n: t.grad for n, t in got.items()} | dict(w=lin.weight.grad, bias=lin.bias.grad)
+    for name, g, r in [("out", out_g, out_r)] + [(n, grads[n], want[n].grad) for n in grads]:
+        g, r = g.detach().double().cpu(), r.detach().double()
+        assert torch.isfinite(g).all(), name
+        rel = ((g - r).norm() / r.norm()).item()
+        assert rel <= 1e-2, f"{name}: relative error {rel:.2e}"
+
+
 @pytest.mark.parametrize("keep_dtype", [True, False], ids=["bf16", "fp32"])
 def test_cfg5_wan_chunk_fwd_bwd_matches_oracle(keep_dtype):
     """cfg 5: Lq=4680, Lkv=32760, H=12, D=128, block 128, top-k 16 on 8 sparse heads + 4 elu1 heads;
