@@ -269,36 +269,29 @@ __global__ void __launch_bounds__(256) k2q_kernel(BwdParams p) {
   p.k2q_num[((int64_t)b * p.n_heads + hs) * p.Nkv + j] = cnt;
 }
 
-// The dq and dkdv passes stream their tiles through a ring of LDS stages: the tile of step t + 1
-// streams in while step t is computed, issued into the stage step t - 1 freed. Every step issues the
-// same number of loads (an empty half-block streams the slab's first rows), so the waits count
-// them. Row lists (with each block's valid row count) are staged in LDS once, so the loop issues no
-// other memory reads while they fit. Both passes run two waves per SIMD (up to 256 registers) as
-// two workgroups per CU, each with a 2-stage ring, its staged list (and for dK/dV the P exchange)
-// in half the CU's LDS: while one workgroup sets up or writes its result, the other computes.
-constexpr int DQ_STAGES = 2, DQ_LIST_MAX = 1024;
-constexpr int DKDV_KEYS = 64, DKDV_STAGES = 2, DKDV_LIST_MAX = 1024;
+// The dq and dkdv passes stream their tiles through a ring of two LDS stages: the tile of step t + 1
+// streams in while step t is computed, issued into the stage step t - 1 freed; with nothing else in
+// flight, a step's top waits for all of this wave's loads. Row lists (with each block's valid row
+// count) are staged in LDS once, so the loop issues no other memory reads while they fit. Both passes
+// run two waves per SIMD (up to 256 registers) as two workgroups per CU, each with its ring, its
+// staged list (and for dK/dV the P exchange) in half the CU's LDS: while one workgroup sets up or
+// writes its result, the other computes.
+constexpr int RING_STAGES = 2, DQ_LIST_MAX = 1024;
+constexpr int DKDV_KEYS = 64, DKDV_LIST_MAX = 1024;
 
 template <int N> using IC = std::integral_constant<int, N>;
 
-// Stage S of a ring kept as its own LDS array (four at most), so that every stage address is static.
+// Stage S of a ring kept as two LDS arrays, so that every stage address is static.
 template <int S, class T>
-__device__ __forceinline__ T* stage_of(T* s0, T* s1, T* s2, T* s3) {
+__device__ __forceinline__ T* stage_of(T* s0, T* s1) {
   if constexpr (S == 0) return s0;
-  else if constexpr (S == 1) return s1;
-  else if constexpr (S == 2) return s2;
-  else return s3;
+  else return s1;
 }
 
-// Top of a step: this wave's loads of the current tile are done (at most `ahead` later tiles of
-// PER loads each still in flight) and so are its LDS reads of the previous step; the barrier
-// extends both to the workgroup, after which the previous step's stage may be refilled.
-template <int PER>
-__device__ __forceinline__ void ring_wait(int ahead) {
-  if (ahead >= 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * PER) : "memory");
-  else if (ahead == 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(PER) : "memory");
-  else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
+// Top of a step: this wave's loads of the current tile are done and so are its LDS reads of the
+// previous step; the barrier extends both to the workgroup, after which the previous step's stage may
+// be refilled.
+__device__ __forceinline__ void ring_wait() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // Lists of at most this many key blocks can be put in block order through a bitmap.
 constexpr int DQ_SORT_BLOCKS = 2048;
@@ -319,9 +312,8 @@ template <int D, int BS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) bwd_dq_kernel(BwdParams p) {
   constexpr int KS = BS == 64 ? 2 : 1, NQW = BS / 32, NW = NQW * KS, DC = D / 16, DT = D / 32;
   constexpr int KT = 2 / KS;                       // 32-key tiles of a step per wave
-  constexpr int TILE = 64 * D, ST = DQ_STAGES, LM = DQ_LIST_MAX;
+  constexpr int TILE = 64 * D, ST = RING_STAGES, LM = DQ_LIST_MAX;
   using TS = TileStream<D, NW>;
-  constexpr int PER = 2 * TS::NI;                  // loads per wave per step: K and V
   constexpr int HPV = BS / 64;                     // 64-key steps per visited block
   static_assert(ST == 2 && NW == 4, "two ring stages, four waves");
   // stage s: K tile at [0, TILE), V tile at [TILE, 2 TILE)
@@ -403,7 +395,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
   vs.init(p.v + (int64_t)b * p.v_sb + (int64_t)h * p.v_sh, p.v_st, p.v_slab, w, lane);
   const int total = n * HPV;
   // step t = (visit t / HPV, half t % HPV): first key row and real key count (<= 0: empty half)
-  // (an empty half streams rows from key 0: never read, keeps the load count uniform)
+  // (an empty half streams rows from key 0, never read)
   auto step_at = [&](int t, int& real) -> int {
     const int s2 = t / HPV, hf = t % HPV;
     const int e = __builtin_amdgcn_readfirstlane(s2 < LM ? s_lst[s2] : packed(block_at(s2)));
@@ -411,7 +403,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
     return real > 0 ? (e & 0xFFFF) * BS + 64 * hf : 0;
   };
   auto issue = [&](auto S, int t) {
-    bf16_t* kv = decltype(S)::value ? kv1 : kv0;
+    bf16_t* kv = stage_of<decltype(S)::value>(kv0, kv1);
     int real;
     const int r0 = step_at(t, real);
     ks.issue(kv, r0, w);
@@ -423,14 +415,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
   // 512 64-key blocks a row, now 550 (128-key blocks: 93 us either way)
   auto step = [&](auto S, int t) {
     constexpr int SV = decltype(S)::value;
-    ring_wait<PER>(min(ST - 2, total - 1 - t));
+    ring_wait();
     int real;
     step_at(t, real);
     if (real <= 0) {  // uniform: an empty half contributes nothing
       if (t + ST - 1 < total) issue(IC<(SV + ST - 1) % ST>{}, t + ST - 1);
       return;
     }
-    const bf16_t* kc = SV ? kv1 : kv0;
+    const bf16_t* kc = stage_of<SV>(kv0, kv1);
     const bf16_t* vc = kc + TILE;
     const int key0 = KS == 2 ? 32 * kh : 0;  // this wave's first key of the step
     // S^T = K Q^T and dP^T = V dO^T (A from LDS, B from registers)
@@ -597,7 +589,7 @@ typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 template <int D, int BS, bool ADD>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) bwd_dkdv_kernel(BwdParams p) {
   constexpr int KW = DKDV_KEYS, HB = BS / KW, NKG = KW / 32, NW = 2 * NKG, NT = 64 * NW, DC = D / 16, DT = D / 32;
-  constexpr int TILE = 64 * D, ST = DKDV_STAGES, LM = DKDV_LIST_MAX;
+  constexpr int TILE = 64 * D, ST = RING_STAGES, LM = DKDV_LIST_MAX;
   constexpr int QPB = BS / 64;                     // 64-query steps per query block
   using TS = TileStream<D, NW>;
   // stage s: Q tile at [0, TILE), dO tile at [TILE, 2 TILE), then 64 lse and 64 delta floats
@@ -605,8 +597,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
   static_assert(ST == 2 && NW == 4, "two ring stages, four waves");
   __shared__ __attribute__((aligned(1024))) bf16_t qd0[SS];
   __shared__ __attribute__((aligned(1024))) bf16_t qd1[SS];
-  bf16_t* const qd2 = qd0;  // (no third or fourth stage)
-  bf16_t* const qd3 = qd1;
   // P of each key group (fp16, accumulator order), register r of 32-query tile qt of lane L at
   // [group][qt][r / 4][L]: every access is 8 bytes per lane, lanes contiguous
   __shared__ __attribute__((aligned(1024))) f16x4 s_p[NKG][2][4][64];
@@ -701,7 +691,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
   // the first wave streams the lse row too, the last one the delta row: the waves' counts of loads
   // in flight differ, so a step waits for all of its own (two stages: nothing else is in flight)
   auto issue = [&](auto S, int t) {
-    bf16_t* qd = stage_of<decltype(S)::value>(qd0, qd1, qd2, qd3);
+    bf16_t* qd = stage_of<decltype(S)::value>(qd0, qd1);
     const int q0r = first_query(t);
     const int src0 = q0r < p.Lq ? q0r : 0;  // a half past Lq streams query 0 (never used)
     qs.issue(qd, src0, w);
@@ -716,7 +706,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
   // against 2,402
   auto step = [&](auto S, int t) {
     constexpr int SV = decltype(S)::value;
-    ring_wait<0>(0);
+    ring_wait();
     const int e = entry(t / QPB);
     const float mult = (float)(e >> 16);
     const int q0r = (e & 0xFFFF) * BS + 64 * (t % QPB);
@@ -724,7 +714,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
       if (t + ST - 1 < total) issue(IC<(SV + ST - 1) % ST>{}, t + ST - 1);
       return;
     }
-    const bf16_t* qc = stage_of<SV>(qd0, qd1, qd2, qd3);
+    const bf16_t* qc = stage_of<SV>(qd0, qd1);
     const bf16_t* dc = qc + TILE;
     const float* st_lse2 = (const float*)(qc + 2 * TILE);
     const float* st_dl = st_lse2 + 64;

@@ -357,19 +357,12 @@ extern "C" int wa_hsa_fwd_any(const wa_hsa_any_args* a, void* stream) {
     rc = wa_compress_kv_n(cj, 2, side);
   }
   if (rc == WA_OK && linear) rc = run_linear(a, p, ws, q, kc, vc, side);
-  // from here the side stream is joined on every path (a capture must end joined)
-  bool joined = !two;
-  auto wait_linear = [&]() -> int {
-    if (joined) return WA_OK;
-    joined = true;
-    if ((e = hipEventRecord(join, side)) != hipSuccess || (e = hipStreamWaitEvent(main, join, 0)) != hipSuccess)
-      return wa_fail((int)e, "wa_hsa_fwd_any: join: %s", hipGetErrorString(e));
-    return WA_OK;
-  };
   if (rc == WA_OK && sparse) rc = run_routing(a, p, ws, main);
   if (rc == WA_OK && a->n_sparse_only > 0) rc = run_sparse(a, p, ws, q, k, v, false, main);
-  const int jc = wait_linear();
-  if (rc == WA_OK) rc = jc;
+  if (two) {  // the side stream is joined on every path (a capture must end joined)
+    if ((e = hipEventRecord(join, side)) != hipSuccess || (e = hipStreamWaitEvent(main, join, 0)) != hipSuccess)
+      return rc != WA_OK ? rc : wa_fail((int)e, "wa_hsa_fwd_any: join: %s", hipGetErrorString(e));
+  }
   if (rc == WA_OK && a->n_both > 0) rc = run_sparse(a, p, ws, q, k, v, true, main);
   return rc;
 }
