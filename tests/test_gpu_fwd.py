@@ -624,6 +624,24 @@ def test_bsa_long_rows_rank_ranges_match_oracle(case, b, h, nq):
         assert torch.equal(plain, table)
 
 
+@pytest.mark.parametrize("d", [64, 128])
+def test_bsa_key_split_launches_repeat_bit_for_bit(d):
+    """Long rows over 64-key blocks at the size of a rollout's chunk (12 heads, 74 rows of ~180 of 512
+    blocks, units of 64 visits): 60 launches on the same inputs give the same bits, output and
+    log-sum-exp (units that share a CU read the same keys at the same time)."""
+    from worldattention_amd.hsa.block_sparse import bsa_forward
+    g = torch.Generator(device=DEV).manual_seed(d)
+    h, bs, nq, nkv = 12, 64, 74, 512
+    q, k, v = (torch.randn(1, n * bs, h, d, generator=g, device=DEV).bfloat16() for n in (nq, nkv, nkv))
+    index = torch.argsort(torch.rand(1, h, nq, nkv, generator=g, device=DEV), dim=-1).int()
+    num = torch.randint(160, 200, (1, h, nq), generator=g, device=DEV).int()
+    args = dict(index=index, num=num, block_size=bs, layout="blhd", split=64, out_dtype=torch.float32, want_lse=True)
+    out, lse = bsa_forward(q, k, v, **args)
+    for _ in range(60):
+        again, again_lse = bsa_forward(q, k, v, **args)
+        assert torch.equal(again, out) and torch.equal(again_lse, lse)
+
+
 @pytest.mark.parametrize("d,bs,split", [(64, 64, 16), (128, 64, 64), (64, 128, 16), (128, 128, 16), (128, 128, 32)])
 @pytest.mark.parametrize("visits", [(1, 16, 33), (48, 63, 64), (5, 65, 80)])
 def test_bsa_unit_tables_equal_the_table_free_launch(d, bs, split, visits):

@@ -261,10 +261,20 @@ __device__ __forceinline__ void write_output(const FwdParams& p, const f32x16 (&
 // Direct-to-LDS 16-byte load through the compiler's builtin: the scheduler sees a memory load (LDS
 // reads move freely around it) and the wait-count pass tracks it per LDS array. Every ring stage is
 // an array of its own and every access names its stage statically, so a read of one stage never
-// waits for loads into another; the kernel still orders loads across waves itself (s_waitcnt
-// vmcnt(0) + s_barrier at the top of each block).
+// waits for loads into another; the kernel still orders loads across waves itself (pipe_sync at the
+// top of each block).
 __device__ __forceinline__ void pipe_dma16(__amdgpu_buffer_rsrc_t rs, bf16_t* lds, int voff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)lds, 16, voff, 0, 0, 0);
+}
+
+// Top of a block: this wave's tile loads (but the AHEAD latest) have landed and its LDS reads have
+// returned, then the same for the workgroup: the stages read last may be refilled. The reads are
+// waited for by name: the products that consume them are free to move below the barrier (the key-split
+// loop's first one does), and a load that hits L1, as one does behind the CU's other workgroup on the
+// same keys, can refill the stage sooner than a read in flight returns.
+template <int AHEAD>
+__device__ __forceinline__ void pipe_sync() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(AHEAD) : "memory");
 }
 
 // Instruction-group order of one slot: after a few leading LDS reads, each product is followed by
@@ -693,7 +703,7 @@ bsa_unit_kernel(FwdParams p) {
       load_tile(0, true, ks0);
       load_tile(1, true, ks1);
       load_tile(0, false, vs0);
-      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * NT::NI) : "memory");
+      pipe_sync<2 * NT::NI>();
       set_neg_m();
       pipe_slot<D, NWT, QT, 1, false, true, false, false>(S, P, oacc, qf, ks0, vs0, k_rd, v_rd, neg_m, sl2, no_load,
                                                          k_off, no_load, v_off, w, rs);
@@ -710,7 +720,7 @@ bsa_unit_kernel(FwdParams p) {
         bf16_t* const knext = PAR ? ks0 : ks1;
         bf16_t* const vprev = PAR ? vs0 : vs1;
         bf16_t* const vcur = PAR ? vs1 : vs0;
-        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+        pipe_sync<0>();
         if (real_prev < 64) pipe_mask<1, QT>(S[1], real_prev, g);
         const PipeLoad ldk{tile_rs(b + 1, true), knext}, ldv{tile_rs(b, false), vcur};
         set_neg_m();
@@ -737,7 +747,7 @@ bsa_unit_kernel(FwdParams p) {
       auto last = [&](auto par) {
         constexpr int PAR = decltype(par)::value;  // (T - 1) % 2: stage of V(T - 1)
         bf16_t* const vprev = PAR ? vs1 : vs0;
-        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+        pipe_sync<0>();
         if (real_prev < 64) pipe_mask<1, QT>(S[1], real_prev, g);
         set_neg_m();
         pipe_slot<D, NWT, QT, 1, true, false, true, false>(S, P, oacc, qf, ks0, vprev, k_rd, v_rd, neg_m, sl2, no_load,
@@ -774,7 +784,7 @@ bsa_unit_kernel(FwdParams p) {
       };
       auto slot = [&](auto par, int b) {
         constexpr int PAR = decltype(par)::value;  // b % 2
-        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+        pipe_sync<0>();
         load_tile(b + 2, true, PAR ? ks1 : ks0);
         load_tile(b, false, PAR ? vs1 : vs0);
         mask_step(par, b);
@@ -787,11 +797,11 @@ bsa_unit_kernel(FwdParams p) {
         for (int qt = 0; qt < QT; ++qt) m_i[qt] = -1e30f;
         load_tile(0, true, ks0);
         load_tile(1, true, ks1);
-        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(NT::NI) : "memory");
+        pipe_sync<NT::NI>();
         pipe_slot<D, NWT, QT, 1, false, true, false, false, KH>(S, P, oacc, qf, ks0, vs0, k_rd, v_rd, neg_m, sl2,
                                                                no_load, k_off, no_load, v_off, w, rs);
         // slot 0: no PV product yet
-        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+        pipe_sync<0>();
         load_tile(2, true, ks0);
         load_tile(0, false, vs0);
         mask_step(std::integral_constant<int, 0>{}, 0);
@@ -805,7 +815,7 @@ bsa_unit_kernel(FwdParams p) {
         }
         if (b < T) slot(std::integral_constant<int, 1>{}, b);
         // the last step's PV product (its V stage is vs[(T - 1) % 2], its P pair (T - 1) % 2)
-        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+        pipe_sync<0>();
         if ((T - 1) & 1)
           pipe_slot<D, NWT, QT, 0, false, false, true, false, KH>(S, P, oacc, qf, ks0, vs1, k_rd, v_rd, neg_m, sl2,
                                                                  no_load, k_off, no_load, v_off, w, rs);
