@@ -304,7 +304,8 @@ constexpr int DQ_SORT_BLOCKS = 2048;
 // with one wave per tile each SIMD had a single wave and nothing to run under its waits. A list
 // without duplicates is walked in block order (whatever the routing order): the rows an XCD runs at
 // a time then sweep a head's keys together and share them in L2. H 12, D 128, Lq 4680, Lkv 32,760,
-// ~180 blocks a row: 698 us with two waves in list order, 575 us here. A list of
+// ~180 blocks a row: 719 us with two waves in list order, 575 with four in block order, 550 with the
+// issue order of the loop. A list of
 // at most 32 blocks keeps its order: the sort's two barriers cost more than it saves (8 heads of 16
 // 128-key blocks: 96 us unsorted, 104-113 us sorted).
 // ---------------------------------------------------------------------------------------------
@@ -808,8 +809,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) b
     // the compression's term, as compress_bwd_dx_kernel forms it (linear.hip): per segment that the
     // wave's 32 keys touch, sum_j E[j, key] g[row0 + j, channel] with g split in three bf16 parts,
     // operands straight from L2 (a head's g is ~270 KB), added by the lanes of that segment. Bound by
-    // the trip to L2 at a workgroup's end: ~95 us of the launch at 12 heads, 32,760 keys with the
-    // loads tile by tile, ~20 with all of them first
+    // the trip to L2 at a workgroup's end: at 12 heads, 32,760 keys the term cost ~95 us with the
+    // loads tile by tile and costs ~55 with all of them first (whole backward 1,378 -> 1,435 us)
     const float* gr = (swave ? p.add_v : p.add_k) + (int64_t)b * p.add_sb + (int64_t)h * p.add_sh + l32;
     const bf16_t* pe = swave ? p.proj_v : p.proj_k;
 #pragma unroll
@@ -981,10 +982,14 @@ __global__ void __launch_bounds__(256) dkdv_sum_kernel(BwdParams p, int D) {
   for (int e = 0; e < 4; ++e) ((float*)out)[at + e] = add ? ((float*)out)[at + e] + sum[e] : sum[e];
 }
 
-// Runs per list: with fewer key parts than the GPU runs at a time (two per CU), long lists are cut so
-// that about 512 workgroups run, each with at least 8 query steps where every query block listed
-// the key block. The dense backward over 525 compressed keys of 12 heads (4680 queries): 148 us as
+// Runs per list: with fewer key parts than the GPU runs at a time (two per CU), lists are cut so that
+// about 512 workgroups run, each with at least 8 query steps where every query block listed the key
+// block. The dense backward over 525 compressed keys of 12 heads (4680 queries): 148 us as
 // 108 workgroups of 74 steps, 76 + 10 us cut in five (128-key blocks: 120 parts) with the sum.
+// The rule sees query lengths, not list lengths (which are on the device): short lists pay for the
+// sum's launch. Whole backward at 2 heads of 74 query and 64 key blocks, 64 / 16 / 4 / 2 blocks a row:
+// 150 / 70 / 50 / 46 us in four runs, 238 / 97 / 52 / 40 in one. Runs by list length, decided on the
+// device with single runs written directly, kept that launch and were no faster for short lists.
 int dkdv_parts(int64_t B, int64_t n_heads, int64_t Lq, int64_t Lkv, int64_t block_size) {
   const int64_t key_parts = B * n_heads * ((Lkv + block_size - 1) / block_size) * (block_size / DKDV_KEYS);
   if (key_parts <= 0 || key_parts >= 384) return 1;

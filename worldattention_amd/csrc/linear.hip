@@ -41,7 +41,8 @@ struct CompressJobs {
 // sums meet in LDS in group order. 16 waves x 16 loads in flight cover a memory round trip; the
 // kernel before it staged x through LDS with 4 waves and one barrier pair per 64 tokens, one
 // element per load: keys and values of H 12, L 32,760, D 128 fp32 at segment 1,560,
-// rank 25 took 379 us (two launches) against 84 us here, and B 2, H 6, L 5,003 336 us against ~20.
+// rank 25 took 379 us (two launches) against 84 us here, and B 2, H 6, L 5,003 335 us against 20 (27-30
+// beside a call's other kernels).
 // =============================================================================================
 constexpr int kTokenGroups = 4;
 

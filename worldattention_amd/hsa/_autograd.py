@@ -306,8 +306,8 @@ class _HSA(torch.autograd.Function):
         # Keys compressed in the call: where every head is sparse, the dK/dV pass adds the
         # compression's term E^T g itself and writes the final type (bf16 projections of one shape,
         # lists not cut into runs). As a pass of its own it read the fp32 gradients back and wrote
-        # bf16 ones: 2 x 118 us at 12 heads, 32,760 keys, D 128, where the dK/dV pass now takes ~30 us
-        # more; the whole step 2650 -> 2440 us.
+        # bf16 ones: 2 x 118 us at 12 heads, 32,760 keys, D 128, where the dK/dV pass now takes ~55 us
+        # more; the whole step 2,650 -> 2,445 us.
         fuse_dx = (inline and fresh_kv and kd == vd and kd in (torch.bfloat16, torch.float32)
                    and k_proj_mat.dtype == v_proj_mat.dtype == torch.bfloat16 and k_proj_mat.shape == v_proj_mat.shape
                    and _lib.lib().wa_bsa_bwd_key_runs(bsz, heads, q_len, kv_len, block_size) == 1)

@@ -63,8 +63,11 @@ def unit_table(bsz: int, visits_per_slot, nq: int, split: int, device) -> tuple[
 def default_split(block_size: int, rows: int, unknown_lengths: bool) -> int:
     """Visits per unit of a sparse launch: the library's default, but 64 for many rows of unknown length
     over 64-key blocks, whose units fill the GPU's 512 unit slots anyway (three units a row at ~180
-    visits). Launch at ~180 of 512 blocks a row, D 128: 888 rows 429 us with 64 against 452 with 48;
-    300 rows 190 against 205; 50 rows 54 against 48."""
+    visits). Launches of 48 / 64 visits a unit, us at D 128 over 512 blocks: 888 rows of ~50 blocks
+    175 / 145, ~90 258 / 244, ~180 452 / 428, ~300 693 / 665; 296 rows 68 / 58, 98 / 95, 161 / 151,
+    246 / 247 (64 is up to 4% slower where it saves no unit, at ~110 to ~128 blocks); 222 rows 60 / 55,
+    86 / 72, 130 / 130, 198 / 190 but ~60 and ~128 60 / 62 and 100 / 108; 50 rows of ~180 48 / 54. Below
+    256 rows neither wins at every length, and with slots to spare more units do."""
     if unknown_lengths and block_size == 64 and rows >= 256:
         return 64
     return _lib.bsa_default_split(block_size)
