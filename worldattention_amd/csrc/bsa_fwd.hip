@@ -445,7 +445,7 @@ __device__ __forceinline__ bool pipe_check(const float (&rs)[QT]) {
 // TABLE: the launch's units come from a table and no row it lists needs more than 64 visits (top-k
 // budgets). Such a unit is a few microseconds long and its prologue a chain of cold instruction
 // fetches: the code of the rank ranges, 1,100 instructions that it only jumps over, and their
-// list loads cost a call of 8 + 4 split heads (4,680 x 32,760, 8-32 of 256 128-key blocks) 0.7 of 121.4 us.
+// list loads cost a call of 8 + 4 split heads (4,680 x 32,760, 8-32 of 256 128-key blocks) 1.0 of 121.4 us.
 template <int D, int BS, int QT, int KS, bool TABLE>
 __global__ void __launch_bounds__(2 * BS / QT * KS) __attribute__((amdgpu_waves_per_eu(QT == 1 ? 2 : 1)))
 bsa_unit_kernel(FwdParams p) {
@@ -490,13 +490,16 @@ bsa_unit_kernel(FwdParams p) {
 
   // The row's first list entries, read before its visit count is known (in bounds of the row's
   // index_width entries): position lane (j0: a row of at most 64 visits) and positions tid and
-  // tid + NTH (e0, e1: a longer row's block-id bitmap).
+  // tid + NTH (e0, e1: a longer row's block-id bitmap). TABLE: position lane of this unit's slice
+  // instead (j1): loaded in the branch that rarely needs it, it made every unit wait for Q there.
   constexpr int NTH = 64 * NWT;
   const int nraw = p.index ? p.num[irow] : p.Nkv;
   const int32_t* lrow = p.index ? p.index + irow * p.index_width : nullptr;
-  int j0 = 0, e0 = 0, e1 = 0;
+  int j0 = 0, j1 = 0, e0 = 0, e1 = 0;
   if (p.index) {
     if (lane < min((int)p.index_width, 64)) j0 = lrow[lane];
+    const int lo1 = split * p.split;
+    if (TABLE && split > 0 && lane < min((int)p.index_width - lo1, 64)) j1 = lrow[lo1 + lane];
     if (!TABLE && p.index_width > 64) {
       if (tid < p.index_width) e0 = lrow[tid];
       if (tid + NTH < p.index_width) e1 = lrow[tid + NTH];
@@ -585,7 +588,7 @@ bsa_unit_kernel(FwdParams p) {
     }
   }
   if (!ranked) {
-    if (lane < take) my_j = p.index ? min(max(lo == 0 ? j0 : lrow[lo + lane], 0), p.Nkv - 1) : lo + lane;
+    if (lane < take) my_j = p.index ? min(max(lo == 0 ? j0 : TABLE ? j1 : lrow[lo + lane], 0), p.Nkv - 1) : lo + lane;
     if (whole || p.index) my_j = wave_sort_ascending(lane < take ? my_j : 0x7fffffff, lane);
   } else if (!p.index && lane < take) {
     my_j = lo + lane;
