@@ -2,9 +2,9 @@
 
 Tolerances: values, and roped queries / keys without the RMSNorm, bit-exact (the rotation uses
 the oracle's fp64 products and roundings). With the RMSNorm, the sum of squares is formed in
-torch's CPU fp32 order but the factor is the correctly rounded 1 / sqrt, while torch's CPU rsqrt
-(MKL) differs from that in the last fp32 bit for ~0.65% of inputs: a normed element may then sit
-one bf16 ulp away, so roped q / k are checked to within one bf16 ulp of the larger element of their
+torch's CPU fp32 order and the factor is 1 / sqrt with both steps correctly rounded, which torch's
+CPU rsqrt gave for every input tried (10^6): one test checks the oracle's bits. The others leave
+room for an rsqrt of another build: roped q / k within one bf16 ulp of the larger element of their
 rotation pair, with at most 0.1% of elements off at all (fp32: four fp32 ulps, at most 2% off).
 Coarse slots within
 1e-2 max-abs / 1e-3 mean-abs (compression: fp32 sums in another order, one bf16 rounding); cache
@@ -129,6 +129,24 @@ def test_qkv_epilogue_row_shapes(h, d, dtype, n):
         _equal(cache["v"][:, ws:ws + n], v, "cache v")
         for t, fill in ((cache["k"], 5), (cache["v"], -5)):
             assert (t[:, :ws] == fill).all() and (t[:, ws + n:] == fill).all()
+
+
+@pytest.mark.parametrize("h,d,dtype,n", [(1, 8, torch.bfloat16, 33), (1, 40, torch.float32, 33), (13, 40, torch.bfloat16, 33),
+                                         (12, 128, torch.bfloat16, 300), (12, 128, torch.float32, 300), (40, 128, torch.bfloat16, 60)])
+def test_qkv_epilogue_with_norm_has_the_oracles_bits(h, d, dtype, n):
+    """RMSNorm and RoPE bit for bit, over enough elements to hold rotated doubles that fp32 rounds
+    onto a bf16 tie: those round to another bf16 where the double is rounded once, 8 in 10^6."""
+    torch.manual_seed(h + d)
+    q, k, v = (torch.randn(1, n, h, d).to(dtype) * 2 for _ in range(3))
+    wq, wk = (torch.rand(h * d).to(dtype) + 0.5 for _ in range(2))
+    freqs = OK.rope_freqs(64, d)
+    cache = {"k": torch.zeros((1, n, h, d), dtype=dtype, device=DEV), "v": torch.zeros((1, n, h, d), dtype=dtype, device=DEV)}
+    grid = (n // 60, 6, 10) if n >= 60 else (1, 3, n // 3)
+    got_q = KV.qkv_epilogue(q.to(DEV), k.to(DEV), v.to(DEV), cache, grid_sizes=torch.tensor([list(grid)]), freqs=freqs,
+                            start_frame=5, write_start=0, norm_q=wq.to(DEV), norm_k=wk.to(DEV))
+    for got, x, w, what in ((got_q, q, wq, "roped q"), (cache["k"], k, wk, "cache k")):
+        normed = OC.rms_norm(x.reshape(1, n, h * d), w, 1e-6).reshape(1, n, h, d)
+        _equal(got, OC.causal_rope(normed, grid, freqs, 5).to(dtype), what)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])

@@ -73,7 +73,7 @@ int kv_copy(const CopyPair& c0, const CopyPair& c1, int dtype, int64_t B, int64_
 // (2c, 2c+1) of each head rotate by the table entry of the band c falls in (temporal: frame
 // start_frame + f, height: row h, width: column w of the token's grid position, found once per row).
 // Bound by reading and writing every row once. 4,680 tokens of 12 x 128 bf16, norm and RoPE: 64 us
-// with 16-row workgroups, 8 threads a row in the sum and four integer divisions per 16 bytes, 37 us
+// with 16-row workgroups, 8 threads a row in the sum and four integer divisions per 16 bytes, 36 us
 // here (86 MB: 17 us at a copy's rate; the rest is the load, sum, rotate chain of a workgroup).
 // ---------------------------------------------------------------------------------------------
 constexpr int kEpiRows = 8;
@@ -114,8 +114,12 @@ __device__ __forceinline__ float epi_to_float(T x) { return (float)x; }
 
 template <typename T>
 __device__ __forceinline__ T epi_from_double(double x) {
-  // the reference's double -> output dtype: to fp32 (nearest), then to the dtype (nearest even)
-  return (T)(float)x;
+#pragma clang fp contract(off)
+  // the reference's double -> output dtype: to fp32 (nearest), then to the dtype (nearest even).
+  // Contraction would fold the two into one rounding of the double: another bf16 for the doubles
+  // that fp32 rounds onto a tie (about 8 in 10^6)
+  const float f = (float)x;
+  return (T)f;
 }
 
 // Row r of the TT rows: RMSNorm factor 1 / sqrt(mean(x^2) + eps) in torch's fp32 order.
